@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cmath>
 #include <type_traits>
+#include <utility>
 
 namespace tl {
 
@@ -1086,60 +1087,113 @@ __global__ void pad_identity_kernel(double* A, int64_t n, int64_t np) {
 // that holds the next pivot block inverts it.  After the last step the lower
 // tiles hold the (symmetric) inverse and are mirrored into the upper ones.
 
+// FP64 matrix-core layouts (v_mfma_f64_16x16x4f64): of a K slice lane l holds
+// A[l%16][l/16] and B[l/16][l%16]; output element i of lane l is
+// C[l/16 + 4i][l%16].  A 16x16 block held in the output layout ("C layout":
+// lane l has rows l/16 + 4i of column l%16) is therefore also a B operand
+// (slice i = element i), and the A operand of its transpose.
+typedef double gj_d4 __attribute__((ext_vector_type(4)));
+
+// value of lane N of the caller's row of 16 lanes
+template <int N>
+__device__ __forceinline__ double gj_row_bcast(double v) {
+  const int2 w = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(
+      double, int2{__builtin_amdgcn_mov_dpp(w.x, 0x150 | N /* row_newbcast */, 0xf, 0xf, true),
+                   __builtin_amdgcn_mov_dpp(w.y, 0x150 | N, 0xf, 0xf, true)});
+}
+
+// value of the lane at the caller's place in row G of 16 lanes
+template <int G>
+__device__ __forceinline__ int gj_group_bcast_b32(int v) {
+  const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);  // halves doubled
+  const int y = (G & 2) ? h[1] : h[0];
+  const auto q = __builtin_amdgcn_permlane16_swap(y, y, false, false);  // rows doubled
+  return (G & 1) ? q[1] : q[0];
+}
+template <int G>
+__device__ __forceinline__ double gj_group_bcast(double v) {
+  const int2 w = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, int2{gj_group_bcast_b32<G>(w.x), gj_group_bcast_b32<G>(w.y)});
+}
+
+// Gauss-Jordan step T of a 32x32 block held as 2 x 2 blocks in the C layout:
+// with p = 1/a_TT, a_ij -= a_iT p a_Tj off row and column T, row T scaled by p,
+// column T by -p, a_TT = p.  All four cases are the one update v - c f after
+// the old row and column are zeroed, c = -1 on row T and f = p on column T.
+template <int T>
+__device__ __forceinline__ void gj_pivot_step(gj_d4 (&v)[2][2], int g, int j) {
+  constexpr int BT = T >> 4, t = T & 15;  // block and place of row and column T
+  constexpr int GT = t & 3, IT = t >> 2;  // row T: element IT of lane group GT
+  double row[2], f[2];
+  gj_d4 c[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    row[b] = gj_group_bcast<GT>(v[BT][b][IT]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) c[b][i] = gj_row_bcast<t>(v[b][BT][i]);
+  }
+  const double p = 1.0 / gj_row_bcast<t>(row[BT]);
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    f[b] = p * row[b];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[b][BT][i] = j == t ? 0.0 : v[b][BT][i];
+  }
+  f[BT] = j == t ? p : f[BT];
+  c[BT][IT] = g == GT ? -1.0 : c[BT][IT];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) v[BT][b][IT] = g == GT ? 0.0 : v[BT][b][IT];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[a][b][i] = __builtin_fma(-c[a][i], f[b], v[a][b][i]);
+}
+
+template <int... T>
+__device__ __forceinline__ void gj_pivot_steps(gj_d4 (&v)[2][2], int g, int j,
+                                               std::integer_sequence<int, T...>) {
+  (gj_pivot_step<T>(v, g, j), ...);
+}
+
 // In-place Gauss-Jordan inverse of the GJB x GJB LDS block by wave 0; every
-// thread of the workgroup calls it.  Lane l keeps row l & 31, columns
-// 16 (l >> 5) .. + 15 in registers; each step publishes the pivot row and
-// column through `pub` (2 x 64 doubles).  One wave's LDS operations execute
-// in order, so the steps need no workgroup barrier.
-__device__ inline void gj_invert_pivot(double (*a)[GJB + 1], double* pub) {
-  static_assert(GJB == 32, "one wave: 32 rows x 2 column halves");
+// thread of the workgroup calls it.  The 32 dependent pivot steps bound it:
+// each moves the pivot row and column by DPP and lane-row swaps (no LDS, no
+// wait) and does sixteen FMAs per lane.  (One row half per lane, rows and
+// columns published through LDS and four selects per entry: 14 us per block.
+// By 16x16 blocks with a Schur complement the steps are shorter, but the
+// inverse of an ill-conditioned block loses digits: residual 1e-4 instead of
+// 1e-8 at condition 8e8.)
+__device__ inline void gj_invert_pivot(double (*a)[GJB + 1]) {
+  static_assert(GJB == 32, "2 x 2 blocks of 16");
   if (threadIdx.x < 64) {
-    const int r = threadIdx.x & 31, h = threadIdx.x >> 5;
-    double v[16];
+    const int j = threadIdx.x & 15, g = threadIdx.x >> 4;
+    gj_d4 v[2][2];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) v[c] = a[r][16 * h + c];
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-    for (int t = 0; t < GJB; ++t) {
-      double* rb = pub + (t & 1) * 64;  // row t
-      double* cb = rb + 32;             // column t
-      if (r == t) {
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-        for (int c = 0; c < 16; ++c) rb[16 * h + c] = v[c];
-      }
-      if (h == (t >> 4)) cb[r] = v[t & 15];
-      __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the step's writes have landed
-      __builtin_amdgcn_wave_barrier();
-      const double att = rb[t], ait = cb[r];
-      double rt[16];
+        for (int i = 0; i < 4; ++i) v[r][c][i] = a[16 * r + g + 4 * i][16 * c + j];
+    gj_pivot_steps(v, g, j, std::make_integer_sequence<int, GJB>{});
 #pragma unroll
-      for (int c = 0; c < 16; ++c) rt[c] = rb[16 * h + c];
-      const double inv = 1.0 / att;  // one reciprocal per step
+    for (int r = 0; r < 2; ++r)
 #pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        const bool jt = h == (t >> 4) && c == (t & 15);
-        const double atj = rt[c] * inv;
-        double nv;
-        if (r == t && jt) nv = inv;
-        else if (r == t) nv = atj;
-        else if (jt) nv = -ait * inv;
-        else nv = v[c] - ait * atj;
-        v[c] = nv;
-      }
-      __builtin_amdgcn_wave_barrier();
-    }
+      for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int c = 0; c < 16; ++c) a[r][16 * h + c] = v[c];
+        for (int i = 0; i < 4; ++i) a[16 * r + g + 4 * i][16 * c + j] = v[r][c][i];
   }
   __syncthreads();
 }
 
 // Step-0 buffers: the row panel R = A[0..GJB)[j] for the workgroup's 64
-// columns; workgroup 0 also inverts the first pivot block.
+// columns; workgroup 0 also inverts the first pivot block (stored transposed).
 __global__ __launch_bounds__(BS) void gj_init_kernel(const double* __restrict__ A, int64_t np,
                                                      double* __restrict__ rowp,
-                                                     double* __restrict__ pinv) {
+                                                     double* __restrict__ pinvt) {
   __shared__ double a[GJB][GJB + 1];
-  __shared__ double pub[128];
   const int64_t c0 = int64_t(blockIdx.x) * 64;
   for (int e = threadIdx.x; e < 64 * GJB; e += BS) {
     const int64_t j = c0 + e % 64;
@@ -1149,8 +1203,8 @@ __global__ __launch_bounds__(BS) void gj_init_kernel(const double* __restrict__ 
   if (blockIdx.x != 0) return;
   for (int e = threadIdx.x; e < GJB * GJB; e += BS) a[e / GJB][e % GJB] = A[(e / GJB) * np + e % GJB];
   __syncthreads();
-  gj_invert_pivot(a, pub);
-  for (int e = threadIdx.x; e < GJB * GJB; e += BS) pinv[e] = a[e / GJB][e % GJB];
+  gj_invert_pivot(a);
+  for (int e = threadIdx.x; e < GJB * GJB; e += BS) pinvt[e] = a[e % GJB][e / GJB];
 }
 
 // lower tile (I, J), I >= J, of linear index b = I (I + 1) / 2 + J
@@ -1162,24 +1216,25 @@ __device__ inline void gj_tile_of(unsigned b, unsigned& I, unsigned& J) {
   J = b - i * (i + 1) / 2;
 }
 
-// Step k on the lower 64x64 tiles.  S = C X on the FP64 matrix cores
-// (v_mfma_f64_16x16x4f64), wave w computing rows 16w..16w+15 as 4 blocks of
-// 16x16, GJB/4 K slices each.  Lane layouts: lane l holds A[l%16][l/16] and
-// B[l/16][l%16] of a K slice; output element i of lane l is C[l/16 + 4i][l%16].
-// The diagonal tile that holds the next pivot block (rows and columns
-// [kb + GJB, kb + 2 GJB)) runs first (hardware block 0) and inverts that
-// block while the other tiles are updated.
-typedef double gj_d4 __attribute__((ext_vector_type(4)));
+// Step k on the lower 64x64 tiles, X = P^-1 R and S = C X on the FP64 matrix
+// cores.  Wave w owns the tile's columns 16w..16w+15: the C layout of its X is
+// the B operand of its S, so a tile needs no LDS, no barrier and one round of
+// loads, all issued before the first product (latency bounds a step: its few
+// hundred workgroups run in one round).  K is 32-aligned, so a 16-column block
+// or a 16-row block lies wholly inside or outside it.  The diagonal tile that
+// holds the next pivot block (rows and columns [kb + GJB, kb + 2 GJB)) runs
+// first (hardware block 0) and inverts that block while the other tiles are
+// updated.  (Panels staged in LDS, X on scalar-operand FMAs: three barriers
+// and a chain of scalar loads, 17-20 us per step with the same pivot
+// inversion.)
 __global__ __launch_bounds__(BS) void gj_step_kernel(double* A, int64_t np, int k, int nbk,
                                                      const double* __restrict__ rowp,
-                                                     const double* __restrict__ pinv,
+                                                     const double* __restrict__ pinvt,
                                                      double* __restrict__ rowp_next,
-                                                     double* __restrict__ pinv_next) {
-  static_assert(BS == 256 && GJB % 4 == 0 && GJB == 32, "four waves, K slices of 4");
-  __shared__ double cp[64][GJB + 1];   // C rows of the tile
-  __shared__ double xp[GJB][64 + 1];   // X columns of the tile
+                                                     double* __restrict__ pinvt_next) {
+  static_assert(BS == 256 && GJB == 32, "four waves, two 16-row blocks per pivot block");
   __shared__ double pb[GJB][GJB + 1];  // the next pivot block (its tile only)
-  __shared__ double pub[128];
+  constexpr int NS = GJB / 4;          // K slices
   const int64_t kb = int64_t(k) * GJB, kn = kb + GJB;
   const bool has_next = k + 1 < nbk;
   const unsigned tn = has_next ? unsigned(kn / 64) : ~0u;    // tile of the next pivot
@@ -1190,94 +1245,75 @@ __global__ __launch_bounds__(BS) void gj_step_kernel(double* A, int64_t np, int 
   const bool own_next = has_next && lb == own;
   unsigned ti, tj;
   gj_tile_of(lb, ti, tj);
-  const int64_t i0 = int64_t(ti) * 64, j0 = int64_t(tj) * 64;
-  double aold[4][4];  // the tile's A values, requested first
-  {
-    const int ww = threadIdx.x >> 6, ll = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l = threadIdx.x & 63, j = l & 15, g = l >> 4;
+  const int64_t i0 = int64_t(ti) * 64, c0 = int64_t(tj) * 64 + 16 * w;  // tile rows, wave columns
+  const bool live = c0 < np;                       // np is a multiple of 32
+  const bool jcol = c0 >= kb && c0 < kn;           // the wave's columns lie in K
+  const bool jnext = has_next && c0 >= kn && c0 < kn + GJB;
+  if (live) {
+    const int64_t jj = c0 + j;
+    // A operands P^-1[16 r + j][4 s + g] (pinvt holds the transpose, so that the
+    // lanes read runs), R[4 s + g][jj], A operands C[i][t] = s(i) R[t][i] and the
+    // old tile values
+    double pv[2][NS], rv[NS], cv[4][NS], aold[4][4];
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int s = 0; s < NS; ++s) {
+      rv[s] = rowp[(4 * s + g) * np + jj];
+#pragma unroll
+      for (int r = 0; r < 2; ++r) pv[r][s] = pinvt[(4 * s + g) * GJB + 16 * r + j];
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t ib = min(i0 + 16 * r, np - 16);  // rows past np are not stored
+#pragma unroll
+      for (int s = 0; s < NS; ++s) cv[r][s] = rowp[(4 * s + g) * np + ib + j];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) aold[r][e] = A[(ib + g + 4 * e) * np + jj];
+    }
+    gj_d4 X[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      X[r] = gj_d4{0.0, 0.0, 0.0, 0.0};
+      if (jcol) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) X[r][e] = pinvt[(jj - kb) * GJB + 16 * r + g + 4 * e];
+      } else {
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+          X[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(pv[r][s], rv[s], X[r], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t ib = i0 + 16 * r;
+      if (ib >= np) continue;
+      gj_d4 S{0.0, 0.0, 0.0, 0.0};
+      const bool swept = ib < kb;
+#pragma unroll
+      for (int s = 0; s < NS; ++s)
+        S = __builtin_amdgcn_mfma_f64_16x16x4f64(swept ? -cv[r][s] : cv[r][s], X[s >> 2][s & 3], S,
+                                                 0, 0, 0);
+      const bool inext = has_next && ib >= kn && ib < kn + GJB;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t i = i0 + 16 * ww + (ll >> 4) + 4 * e, jj = j0 + 16 * b + (ll & 15);
-        aold[b][e] = (i < np && jj < np) ? A[i * np + jj] : 0.0;
+        const int64_t i = ib + g + 4 * e;
+        double v;
+        if (ib >= kb && ib < kn) v = ib == kb ? X[0][e] : X[1][e];  // row panel, P^-1 in K
+        else if (jcol) v = -S[e];                             // column panel
+        else v = aold[r][e] - S[e];                           // trailing update
+        A[i * np + jj] = v;
+        // next row panel: its own tile row direct, the tiles below it transposed
+        if (inext) rowp_next[(i - kn) * np + jj] = v;
+        if (jnext && ti > tn) rowp_next[(jj - kn) * np + i] = v;
+        if (own_next && inext && jnext) pb[i - kn][jj - kn] = v;
       }
-  }
-  // C[r][t] = s(i) R[t][i] for the tile's rows i = i0 + r (0 past np)
-  for (int e = threadIdx.x; e < 64 * GJB; e += BS) {
-    const int t = e / 64, r = e % 64;
-    const int64_t i = i0 + r;
-    const double v = i < np ? rowp[t * np + i] : 0.0;
-    cp[r][t] = i < kb ? -v : v;
-  }
-  // R rows of the tile's columns (0 inside K and past np), staged in xp
-  for (int e = threadIdx.x; e < GJB * 64; e += BS) {
-    const int t = e / 64, c = e % 64;
-    const int64_t jj = j0 + c;
-    xp[t][c] = (jj < np && (jj < kb || jj >= kb + GJB)) ? rowp[t * np + jj] : 0.0;
-  }
-  __syncthreads();
-  // X column j0 + c2, rows rb .. rb + 7 (one wave): P^-1 R[j] outside K,
-  // P^-1 itself inside K, 0 past np.  P^-1 rows are wave-uniform (scalar loads).
-  const int c2 = threadIdx.x & 63;
-  const int rb = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * (GJB / 4);
-  const int64_t j = j0 + c2;
-  const bool jin = j >= kb && j < kb + GJB;
-  const bool active = j < np && !jin;
-  double col[GJB];
-#pragma unroll
-  for (int t = 0; t < GJB; ++t) col[t] = xp[t][c2];
-  __syncthreads();
-#pragma unroll
-  for (int r = rb; r < rb + GJB / 4; ++r) {
-    double sum = 0.0;
-    if (active) {
-#pragma unroll
-      for (int t = 0; t < GJB; ++t) sum += pinv[r * GJB + t] * col[t];
-    } else if (jin) {
-      sum = pinv[r * GJB + (j - kb)];
-    }
-    xp[r][c2] = sum;
-  }
-  __syncthreads();
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
-  gj_d4 acc[4];
-#pragma unroll
-  for (int b = 0; b < 4; ++b) acc[b] = gj_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int sl = 0; sl < GJB / 4; ++sl) {
-    const double av = cp[16 * w + lr][4 * sl + lk];
-#pragma unroll
-    for (int b = 0; b < 4; ++b)
-      acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av, xp[4 * sl + lk][16 * b + lr], acc[b], 0, 0, 0);
-  }
-  // next row panel: rows of the next block in its tile row (direct), its
-  // columns in the tiles below its tile (transposed)
-  const bool below = has_next && ti > tn;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    const int64_t jj = j0 + 16 * b + lr;
-    if (jj >= np) continue;
-    const bool jcol = jj >= kb && jj < kb + GJB;
-    const bool jnext = has_next && jj >= kn && jj < kn + GJB;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int64_t i = i0 + 16 * w + lk + 4 * e;
-      if (i >= np) continue;
-      double v;
-      if (i >= kb && i < kb + GJB) v = xp[i - kb][16 * b + lr];  // row panel, P^-1 inside K
-      else if (jcol) v = -acc[b][e];                              // column panel
-      else v = aold[b][e] - acc[b][e];                            // trailing update
-      A[i * np + jj] = v;
-      const bool inext = has_next && i >= kn && i < kn + GJB;
-      if (inext) rowp_next[(i - kn) * np + jj] = v;
-      if (below && jnext) rowp_next[(jj - kn) * np + i] = v;
-      if (own_next && inext && jnext) pb[i - kn][jj - kn] = v;
     }
   }
   if (!own_next) return;
   __syncthreads();
-  gj_invert_pivot(pb, pub);
-  for (int e = threadIdx.x; e < GJB * GJB; e += BS) pinv_next[e] = pb[e / GJB][e % GJB];
+  gj_invert_pivot(pb);
+  for (int e = threadIdx.x; e < GJB * GJB; e += BS) pinvt_next[e] = pb[e % GJB][e / GJB];
 }
 
 // upper tile (I, J), I < J, of linear index b = J (J - 1) / 2 + I: the
