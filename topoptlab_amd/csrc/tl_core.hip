@@ -971,6 +971,18 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
     P->rec->unsupported = true;  // no multi-instance form of the MFMA operators
     return TL_OK;
   }
+  auto sym = [&]() -> int {
+    if (P->rec) {  // no multi-instance form of the 3D operators
+      P->rec->unsupported = true;
+      return TL_OK;
+    }
+    unsigned nb = 0;
+    TL_TRY(sym_fine_apply(P, a.u, a.y, prec, mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
+                          a.partials, a.done, out64, &nb));
+    if (mode == KU_STORE_DOT || mode == KU_JACOBI_DOT)
+      return launch_fold(P, nb, a.fin, a.dot_out, a.done);
+    return TL_OK;
+  };
   if (prec == TL_PREC_BF16 || prec == TL_PREC_FP16) {
     // V-cycle smoothing and residual on the matrix cores
     TL_ARG(b64 && !fusep && (mode == KU_RESID || mode == KU_JACOBI || mode == KU_JACOBI_DOT),
@@ -993,6 +1005,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
         return launch_fold(P, nb, a.fin, a.dot_out, a.done);
       return TL_OK;
     }
+    if (P->op.sym && (mode == KU_STORE || mode == KU_STORE_DOT || b64)) return sym();
     a.sp = P->op.sp64.ptr; a.KE = P->op.KE64.ptr;
     switch (P->ndpn) {
       case 1: return dispatch_mode<1, double>(P, a, mode, fusep, b64, out64);
@@ -1000,6 +1013,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
       case 3: return dispatch_mode<3, double>(P, a, mode, fusep, b64, out64);
     }
   } else {
+    if (P->op.sym && (mode == KU_STORE || mode == KU_STORE_DOT || b64)) return sym();
     a.sp = P->op.sp32.ptr; a.KE = P->op.KE32.ptr;
     switch (P->ndpn) {
       case 1: return dispatch_mode<1, float>(P, a, mode, fusep, b64, out64);
@@ -1389,6 +1403,7 @@ int tl_create(const tl_grid_desc* d, tl_problem** out) {
   }
   P->fixed_h.assign(d->fixed, d->fixed + d->nfixed);
   detect_ke_pattern(P);
+  P->op.sym = sym_fits(P->g, P->ndpn) && sym_detect(P->ndpn, P->KEh.data(), P->op.symkv);
   P->op.mfma64 = false;  // the vector kernel is faster (tl_set_fp64_operator selects)
   std::vector<float> ke32(nd * nd);
   for (int i = 0; i < nd * nd; ++i) ke32[i] = float(P->KEh[i]);
@@ -1638,9 +1653,10 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     TL_CHECK_LAUNCH();
     TL_TRY(launch_fold(P, c.rb, FIN_RHO, nullptr, c.done));
   }
-  // p = z + beta p ; q = K p ; pq ; alpha.  The fused product (2D, and the
-  // 3D MFMA operator) reads p_k (halo included) while it writes p_{k+1}:
-  // two buffers.  The 3D vector operator takes the update as a separate pass.
+  // p = z + beta p ; q = K p ; pq ; alpha.  The fused product (2D, the tiled
+  // and the MFMA 3D operators) reads p_k (halo included) while it writes
+  // p_{k+1}: two buffers.  The general 3D operator takes the update as a
+  // separate pass.
   double* pin = c.pp[k & 1];
   double* pout = c.pp[(k + 1) & 1];
   P->rec_phase = 2;  // the PCG update after the preconditioner
@@ -1649,7 +1665,7 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     P->rec->unsupported = true;
     return TL_OK;
   }
-  if (P->g.dim == 3 && !(P->op.mfma64 && P->ndpn == 3)) {
+  if (P->g.dim == 3 && !P->op.sym && !(P->op.mfma64 && P->ndpn == 3)) {
     hipLaunchKernelGGL(pupdate_kernel, dim3(c.nb), dim3(BS), 0, s, c.z, pin, pout, &c.st->beta,
                        c.n, c.done);
     TL_CHECK_LAUNCH();

@@ -189,6 +189,8 @@ struct MgState {
   double omega = 0.6;
   std::vector<Level> lv;  // lv[0] is the fine grid (no stencil)
   DevBuf G1;              // 8 x (nd*nd) fp64: child Galerkin matrices
+  bool sym1 = false;      // 3D: level 1 is applied from the densities (tl_sym.hip)
+  double symkv[16] = {};  // group values of its Galerkin matrices
   DevBuf W;               // 8 x 8 fp64: child interpolation weights
   DevBuf cinv;            // dense inverse of the coarsest operator (fp64)
   DevBuf gjw;             // Gauss-Jordan workspace: row panels and pivot inverses of two steps
@@ -203,6 +205,8 @@ struct FineOp {
   bool have_density = false;
   bool fast_ke = false;        // KE matches its unit-cell pattern
   double kv[8] = {};           // group values of the pattern
+  bool sym = false;            // 3D: the tiled reflection-symmetric operator applies (tl_sym.hip)
+  double symkv[16] = {};       // its group values
   // 2D operator workgroup shape per precision [fp64, fp32]: 0 = node line
   // (BS consecutive nodes), TY = 16/32/64: (BS/TY) x TY node tile
   int tile2d[2] = {0, 0};
@@ -309,6 +313,16 @@ int fine_apply_mfma64(tl_problem* P, const double* u, double* y, int mode, const
                       const double* dinv, double omega, const double* pin, double* pout,
                       const double* beta, double* partials, const int* done,
                       unsigned* nblocks_out);
+// tiled 3D operators in the reflection-symmetric form (tl_sym.hip)
+bool sym_detect(int ndpn, const double* KE, double (&kv)[16]);
+bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]);
+bool sym_fits(const Grid& g, int ndpn);
+int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
+                   bool b64, const void* dinv, double omega, const void* pin, void* pout,
+                   const double* beta, double* partials, const int* done, bool out64,
+                   unsigned* nblocks_out);
+int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* b, void* y,
+                     const int* done);
 }  // namespace tl
 
 // First damped-Jacobi sweep from a zero guess, x = omega * dinv * b, in the

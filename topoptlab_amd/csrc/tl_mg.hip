@@ -242,6 +242,7 @@ __global__ void st_finish_kernel(GridD g, int ndpn, const double* __restrict__ s
   const int64_t tot = g.nnodes * nqh;
   for (int64_t t = blockIdx.x * int64_t(BS) + threadIdx.x; t < tot;
        t += int64_t(gridDim.x) * BS) {
+    if (!sth64) break;  // the level is applied from the densities
     const double v = st64[t + int64_t(kc) * ndpn * ndpn * g.nnodes];
     sth64[t] = v;
     st32[t] = float(v);
@@ -1451,6 +1452,14 @@ template <int NDPN, typename T>
 int st_apply(tl_problem* P, int l, int mode, const T* x, const T* b, T* y, const int* done) {
   Level& L = P->mg.lv[l];
   TL_ARG(l >= 1 && l < P->mg.nlevels, "internal: stencil level out of range");
+  if (l == 1 && P->mg.sym1) {  // 3D levels are never recorded for a lockstep batch
+    TL_NONNULL(L.dinv64.ptr); TL_NONNULL(L.dinv32.ptr); TL_NONNULL(L.mask.ptr);
+    TL_NONNULL(x); TL_NONNULL(b); TL_NONNULL(y);
+    ProfEvent e1{};
+    TL_TRY(prof_begin(P, 3 + mode, e1));
+    TL_TRY(sym_coarse_apply(P, std::is_same<T, double>::value, mode, x, b, y, done));
+    return prof_end(P, e1);
+  }
   TL_NONNULL(L.sth64.ptr); TL_NONNULL(L.st32.ptr); TL_NONNULL(L.dinv64.ptr);
   TL_NONNULL(L.dinv32.ptr); TL_NONNULL(L.mask.ptr); TL_NONNULL(x); TL_NONNULL(b); TL_NONNULL(y);
   const T* st = std::is_same<T, double>::value ? static_cast<const T*>(L.sth64.ptr)
@@ -1742,27 +1751,6 @@ extern "C" int tl_setup_mg(tl_problem* P, const tl_mg_opts* o) {
     TL_TRY(level_masks(P, L, masks));
     for (auto& l : M.lv) l.release();
     M.lv.clear();
-    M.lv.resize(L);
-    M.nlevels = L;
-    Grid gl = g;
-    for (int l = 0; l < L; ++l) {
-      Level& lv = M.lv[l];
-      if (l > 0) gl.set(gl.dim, gl.nelx / 2, gl.nely / 2, gl.nelz / 2);
-      lv.g = gl;
-      lv.ndof = gl.nnodes * ndpn;
-      const size_t vb = sizeof(double) * size_t(lv.ndof);
-      TL_TRY(lv.vx.alloc(vb)); TL_TRY(lv.vt.alloc(vb)); TL_TRY(lv.vr.alloc(vb)); TL_TRY(lv.vb.alloc(vb));
-      if (l == 0) continue;
-      TL_TRY(lv.mask.alloc(gl.nnodes));
-      TL_HIP(hipMemcpy(lv.mask.ptr, masks[l].data(), gl.nnodes, hipMemcpyHostToDevice));
-      const size_t nst = size_t(nstencil(gl.dim)) * ndpn * ndpn * gl.nnodes;
-      TL_TRY(lv.st64.alloc(sizeof(double) * nst));
-      const size_t nsh = size_t(center_k(gl.dim) + 1) * ndpn * ndpn * gl.nnodes;
-      TL_TRY(lv.sth64.alloc(sizeof(double) * nsh));
-      TL_TRY(lv.st32.alloc(sizeof(float) * nsh));
-      TL_TRY(lv.dinv64.alloc(sizeof(double) * lv.ndof));
-      TL_TRY(lv.dinv32.alloc(sizeof(float) * lv.ndof));
-    }
     // G1[c] = (W_c x I)^T KE (W_c x I)
     std::vector<double> W;
     child_weights(g.dim, W);
@@ -1790,6 +1778,32 @@ extern "C" int tl_setup_mg(tl_problem* P, const tl_mg_opts* o) {
     }
     TL_TRY(M.G1.alloc(sizeof(double) * G.size()));
     TL_HIP(hipMemcpy(M.G1.ptr, G.data(), sizeof(double) * G.size(), hipMemcpyHostToDevice));
+    Grid g1;
+    g1.set(g.dim, g.nelx / 2, g.nely / 2, g.nelz / 2);
+    M.sym1 = sym_fits(g1, ndpn) && sym_detect_coarse(ndpn, G.data(), M.symkv);
+    M.lv.resize(L);
+    M.nlevels = L;
+    Grid gl = g;
+    for (int l = 0; l < L; ++l) {
+      Level& lv = M.lv[l];
+      if (l > 0) gl.set(gl.dim, gl.nelx / 2, gl.nely / 2, gl.nelz / 2);
+      lv.g = gl;
+      lv.ndof = gl.nnodes * ndpn;
+      const size_t vb = sizeof(double) * size_t(lv.ndof);
+      TL_TRY(lv.vx.alloc(vb)); TL_TRY(lv.vt.alloc(vb)); TL_TRY(lv.vr.alloc(vb)); TL_TRY(lv.vb.alloc(vb));
+      if (l == 0) continue;
+      TL_TRY(lv.mask.alloc(gl.nnodes));
+      TL_HIP(hipMemcpy(lv.mask.ptr, masks[l].data(), gl.nnodes, hipMemcpyHostToDevice));
+      const size_t nst = size_t(nstencil(gl.dim)) * ndpn * ndpn * gl.nnodes;
+      TL_TRY(lv.st64.alloc(sizeof(double) * nst));
+      const size_t nsh = size_t(center_k(gl.dim) + 1) * ndpn * ndpn * gl.nnodes;
+      if (l > 1 || !M.sym1) {
+        TL_TRY(lv.sth64.alloc(sizeof(double) * nsh));
+        TL_TRY(lv.st32.alloc(sizeof(float) * nsh));
+      }
+      TL_TRY(lv.dinv64.alloc(sizeof(double) * lv.ndof));
+      TL_TRY(lv.dinv32.alloc(sizeof(float) * lv.ndof));
+    }
     const Level& Lc = M.lv[L - 1];
     M.cn = Lc.ndof;
     M.cnp = ((M.cn + GJB - 1) / GJB) * GJB;

@@ -1,0 +1,650 @@
+// 3D operators in the reflection-symmetric form of the H8 element matrix: the
+// fine grid's K.u and the first coarse level's Galerkin operator, both
+// matrix-free (the products of topoptlab/topology_optimization.py:429-451 and
+// multigrid.py:142-168).
+//
+// The unit-cell element matrix of an isotropic material commutes with the
+// reflections of the cell.  With H the 8-point Hadamard transform of each
+// displacement component over the element's corners, KE = H^T B H, and B
+// couples only within one parity class: 45 nonzeros instead of 576.  An
+// element then costs about 160 instead of 600 operations: transform the two
+// node planes (each plane's in-plane part is shared by the layers below and
+// above it), 45 multiply-adds, transform back.
+//
+// The Galerkin matrix of a level-1 element is linear in its 8 children's
+// scales, and in the same basis sum_m t_m B_m with t the Hadamard transform of
+// the child scales and B_m constant: 279 nonzeros together.  Applying it from
+// the densities reads about 25 MB at 192x96x96 in FP64 where the stored
+// half-stencil reads 252 MB.
+//
+// A workgroup owns a 16x16 tile of element columns (thread (tx, ty): element
+// column (X0 + tx - 1, Y0 + ty - 1), y fastest) and walks a range of element
+// layers in z; it produces the 15x15 nodes all of whose elements it holds.  A
+// node plane (17x17 nodes) is staged in LDS once, a layer ahead, through
+// registers.  The four columns around a node are summed by a DPP row shift in
+// y and through LDS in x; one barrier per layer covers both the staged plane
+// and that exchange.
+#include "tl_internal.hpp"
+#include "sym_pattern.hpp"
+
+#include <algorithm>
+#include <cmath>
+#include <map>
+#include <mutex>
+#include <tuple>
+
+namespace tl {
+namespace {
+
+constexpr int BS = 256;
+constexpr int TE = 16;       // element columns per tile side
+constexpr int TN = TE - 1;   // nodes produced per tile side
+constexpr int TS = TE + 1;   // nodes staged per tile side
+static_assert(TE * TE == BS, "one element column per thread");
+
+template <typename T>
+struct SymArgs {
+  const T* u;          // input; FUSEP: z
+  const T* pin;        // FUSEP: previous search direction
+  T* pout;             // FUSEP: new search direction
+  const double* beta;  // FUSEP: device scalar
+  const T* sp;         // zero-bordered scales of the fine grid
+  const uint8_t* mask;
+  const void* b;       // KU_RESID / KU_JACOBI*: right-hand side
+  const T* dinv;
+  T omega;
+  void* y;
+  double* partials;
+  const int* done;
+  int nelx, nely, nelz, nx, ny, nz;  // the operator's own grid
+  int fnelx, fnely;                  // CG: the fine grid below it
+  int ncy;                           // tile columns along y
+  unsigned ncol;                     // tile columns
+  T kv[16];                          // group values of the pattern
+};
+
+template <int NDPN, bool CG>
+__host__ __device__ constexpr int sym_tab(int i) {
+  if constexpr (NDPN == 3) return CG ? kTabSymC_elast[i] : kTabSym_elast[i];
+  else return CG ? kTabSymC_poisson[i] : kTabSym_poisson[i];
+}
+
+// parity class of basis function (mode m, component c)
+template <int NDPN>
+__host__ __device__ constexpr int sym_class(int m, int c) {
+  return NDPN == 3 ? m ^ (1 << c) : m;
+}
+// mode of component c in class x
+template <int NDPN>
+__host__ __device__ constexpr int sym_mode(int x, int c) {
+  return NDPN == 3 ? x ^ (1 << c) : x;
+}
+
+__device__ __forceinline__ float sym_fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double sym_fma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
+// value of the next lane in the caller's row of 16 (0 past its end)
+__device__ __forceinline__ float next_lane(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                       0, __builtin_bit_cast(int, v), 0x101 /* row_shl:1 */, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double next_lane(double v) {
+  int2 w = __builtin_bit_cast(int2, v);
+  w.x = __builtin_amdgcn_update_dpp(0, w.x, 0x101, 0xf, 0xf, true);
+  w.y = __builtin_amdgcn_update_dpp(0, w.y, 0x101, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, w);
+}
+
+// 8-point Hadamard transform, index m = mx + 2 my + 4 mz from cz 4 + cx 2 + cy
+template <typename T>
+__device__ __forceinline__ void child_modes(T (&t)[8]) {
+  T s[8];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {  // z
+    s[c] = t[c] + t[4 + c];
+    s[4 + c] = t[c] - t[4 + c];
+  }
+#pragma unroll
+  for (int h = 0; h < 8; h += 4) {  // (cx, cy) -> mx + 2 my
+    const T a = s[h] + s[h + 1], b = s[h] - s[h + 1];          // cx = 0: y sum, difference
+    const T c = s[h + 2] + s[h + 3], d = s[h + 2] - s[h + 3];  // cx = 1
+    t[h] = a + c;
+    t[h + 1] = a - c;
+    t[h + 2] = b + d;
+    t[h + 3] = b - d;
+  }
+}
+
+// Element scales of the thread's column in one layer: the element's own
+// (fine) or its children's modes (CG).
+template <typename T, bool CG>
+struct Scales {
+  T s[CG ? 8 : 1];
+  __device__ __forceinline__ void load(const SymArgs<T>& a, int ix, int iy, int ez) {
+    if constexpr (CG) {
+      // element (ix - 1, iy - 1, ez); zero outside the grid
+      const bool in = ix >= 1 && ix <= a.nelx && iy >= 1 && iy <= a.nely && ez >= 0 && ez < a.nelz;
+      const int cx = min(max(ix, 1), a.nelx), cy = min(max(iy, 1), a.nely),
+                cz = min(max(ez, 0), a.nelz - 1);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int64_t i = (int64_t(2 * cz + (k >> 2) + 1) * (a.fnelx + 2) + 2 * cx - 1 + (k >> 1 & 1)) *
+                              (a.fnely + 2) + 2 * cy - 1 + (k & 1);
+        const T v = a.sp[i];
+        s[k] = in ? v : T(0);
+      }
+    } else {
+      // the border of the padded array holds zeros
+      const int px = min(ix, a.nelx + 1), py = min(iy, a.nely + 1);
+      s[0] = a.sp[(int64_t(ez + 1) * (a.nelx + 2) + px) * (a.nely + 2) + py];
+    }
+  }
+  __device__ __forceinline__ void modes() {
+    if constexpr (CG) child_modes(s);
+  }
+};
+
+// Element contraction of one layer: lower and upper plane's in-plane modes
+// flo, fhi (index mode * NDPN + component, mode = mx + 2 my); adds the lower
+// plane's contribution to tot and returns the upper plane's in up.
+template <int NDPN, typename T, bool CG>
+__device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, CG>& S,
+                                          const T (&flo)[4 * NDPN], const T (&fhi)[4 * NDPN],
+                                          T (&tot)[4 * NDPN], T (&up)[4 * NDPN]) {
+  constexpr int ND = 8 * NDPN;
+  T U[ND];
+#pragma unroll
+  for (int i = 0; i < 4 * NDPN; ++i) {
+    U[i] = flo[i] + fhi[i];
+    U[4 * NDPN + i] = flo[i] - fhi[i];
+  }
+  T ks[16];  // fine: the group values times the element's scale
+  if constexpr (!CG) {
+#pragma unroll
+    for (int g = 0; g < (NDPN == 3 ? kGroupsSym_elast : kGroupsSym_poisson); ++g) ks[g] = S.s[0] * a.kv[g];
+  }
+#pragma unroll
+  for (int i = 0; i < 4 * NDPN; ++i) {
+    T y[2];
+    bool any[2] = {false, false};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int m = 4 * h + i / NDPN, c = i % NDPN, r = m * NDPN + c;
+      y[h] = T(0);
+      if constexpr (!CG) {
+#pragma unroll
+        for (int k = 0; k < NDPN; ++k) {
+          const int col = sym_mode<NDPN>(sym_class<NDPN>(m, c), k) * NDPN + k;
+          const int p = sym_tab<NDPN, false>(r * ND + col);
+          if (p == 0) continue;
+          const T v = ks[(p > 0 ? p : -p) - 1];
+          if (!any[h]) y[h] = p > 0 ? v * U[col] : -v * U[col];
+          else y[h] = sym_fma(p > 0 ? v : -v, U[col], y[h]);
+          any[h] = true;
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          T t = T(0);
+          bool anyq = false;
+#pragma unroll
+          for (int k = 0; k < NDPN; ++k) {
+            const int col = sym_mode<NDPN>(sym_class<NDPN>(m, c) ^ q, k) * NDPN + k;
+            const int p = sym_tab<NDPN, true>((q * ND + r) * ND + col);
+            if (p == 0) continue;
+            const T v = a.kv[(p > 0 ? p : -p) - 1];
+            if (!anyq) t = p > 0 ? v * U[col] : -v * U[col];
+            else t = sym_fma(p > 0 ? v : -v, U[col], t);
+            anyq = true;
+          }
+          if (!anyq) continue;
+          y[h] = any[h] ? sym_fma(S.s[q], t, y[h]) : S.s[q] * t;
+          any[h] = true;
+        }
+      }
+    }
+    if (any[0] && any[1]) {
+      tot[i] += y[0] + y[1];
+      up[i] = y[0] - y[1];
+    } else if (any[0]) {
+      tot[i] += y[0];
+      up[i] = y[0];
+    } else {
+      tot[i] += y[1];
+      up[i] = -y[1];
+    }
+  }
+}
+
+// Staging of one node plane: the thread's entries of the 17x17x NDPN tile,
+// loaded into registers and stored to LDS later.
+template <int NDPN, typename T, bool FUSEP>
+struct Stage {
+  static constexpr int N = TS * TS * NDPN, NR = (N + BS - 1) / BS;
+  uint32_t off[NR];  // entry offsets within a plane (clamped to the grid)
+  T v[NR], w[FUSEP ? NR : 1];
+  __device__ __forceinline__ void init(const SymArgs<T>& a, int x0, int y0) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int e = int(threadIdx.x) + k * BS;
+      const int row = e / (TS * NDPN), rem = e % (TS * NDPN);
+      const int x = min(max(x0 - 1 + row, 0), a.nx - 1), y = min(max(y0 - 1 + rem / NDPN, 0), a.ny - 1);
+      off[k] = uint32_t((x * a.ny + y) * NDPN + rem % NDPN);
+    }
+  }
+  __device__ __forceinline__ void load(const SymArgs<T>& a, int z) {
+    const int64_t base = int64_t(min(max(z, 0), a.nz - 1)) * a.nx * a.ny * NDPN;
+    const T* p = a.u + base;
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (k + 1 < NR || int(threadIdx.x) + k * BS < N) v[k] = p[off[k]];
+    if constexpr (FUSEP) {
+      const T* q = a.pin + base;
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        if (k + 1 < NR || int(threadIdx.x) + k * BS < N) w[k] = q[off[k]];
+    }
+  }
+  __device__ __forceinline__ void store(T* lds, T beta) const {
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (k + 1 < NR || int(threadIdx.x) + k * BS < N) {
+        if constexpr (FUSEP) lds[threadIdx.x + k * BS] = v[k] + beta * w[k];
+        else lds[threadIdx.x + k * BS] = v[k];
+      }
+  }
+};
+
+// In-plane modes of the thread's element from the staged plane, and the value
+// of its own output node (the element's corner (1, 1)).
+template <int NDPN, typename T>
+__device__ __forceinline__ void plane_modes(const T* lds, int tx, int ty, T (&f)[4 * NDPN],
+                                            T (&uc)[NDPN]) {
+  const T* p = lds + (tx * TS + ty) * NDPN;
+#pragma unroll
+  for (int c = 0; c < NDPN; ++c) {
+    const T v00 = p[c], v01 = p[NDPN + c], v10 = p[TS * NDPN + c], v11 = p[(TS + 1) * NDPN + c];
+    const T a = v00 + v01, b = v00 - v01, d = v10 + v11, e = v10 - v11;
+    f[c] = a + d;
+    f[NDPN + c] = a - d;
+    f[2 * NDPN + c] = b + e;
+    f[3 * NDPN + c] = b - e;
+    uc[c] = v11;
+  }
+}
+
+// Node planes z0 .. z1-1 of tile column col.
+template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
+__device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS * TS * NDPN],
+                                            T (*xch)[NDPN * BS], unsigned col, int z0, int z1,
+                                            T beta, double& dot) {
+  const int tid = int(threadIdx.x), tx = tid >> 4, ty = tid & 15;
+  const int x0 = int(col / unsigned(a.ncy)) * TN, y0 = int(col % unsigned(a.ncy)) * TN;
+  const int ix = x0 + tx, iy = y0 + ty;
+  const bool active = tx < TN && ty < TN && ix < a.nx && iy < a.ny;
+  const int64_t node0 = active ? int64_t(ix) * a.ny + iy : 0;
+  const int64_t nplane = int64_t(a.nx) * a.ny;
+  Stage<NDPN, T, FUSEP> st;
+  Scales<T, CG> S, Sn;
+  T flo[4 * NDPN], uc[NDPN], carry[4 * NDPN];
+  st.init(a, x0, y0);
+  st.load(a, z0);
+  S.load(a, ix, iy, z0);
+  __syncthreads();  // the LDS of the previous segment is free
+  st.store(plane[z0 & 1], beta);
+#pragma unroll
+  for (int i = 0; i < 4 * NDPN; ++i) carry[i] = T(0);
+  if (z0 > 0) {  // the layer below gives plane z0's lower part
+    Scales<T, CG> Sb;
+    st.load(a, z0 - 1);
+    Sb.load(a, ix, iy, z0 - 1);
+    st.store(plane[(z0 + 1) & 1], beta);
+    st.load(a, z0 + 1);
+    __syncthreads();
+    T fb[4 * NDPN], unused[4 * NDPN], ub[NDPN];
+    plane_modes<NDPN, T>(plane[(z0 + 1) & 1], tx, ty, fb, ub);
+    plane_modes<NDPN, T>(plane[z0 & 1], tx, ty, flo, uc);
+#pragma unroll
+    for (int i = 0; i < 4 * NDPN; ++i) unused[i] = T(0);
+    Sb.modes();
+    sym_layer<NDPN, T, CG>(a, Sb, fb, flo, unused, carry);
+  } else {
+    st.load(a, z0 + 1);
+    __syncthreads();
+    plane_modes<NDPN, T>(plane[z0 & 1], tx, ty, flo, uc);
+  }
+  if (z0 > 0) __syncthreads();  // plane z0 - 1 has been read
+  st.store(plane[(z0 + 1) & 1], beta);
+  __syncthreads();
+  for (int z = z0; z < z1; ++z) {
+    const bool more = z + 1 < z1;  // uniform
+    if (more) {
+      st.load(a, z + 2);
+      Sn.load(a, ix, iy, z + 1);
+    }
+    // epilogue inputs of the node of plane z
+    const int64_t node = int64_t(z) * nplane + node0;
+    const uint8_t mk = a.mask[node];
+    TB bv[NDPN];
+    T dv[NDPN];
+#pragma unroll
+    for (int c = 0; c < NDPN; ++c) {
+      if constexpr (MODE == KU_RESID || MODE == KU_JACOBI || MODE == KU_JACOBI_DOT)
+        bv[c] = static_cast<const TB*>(a.b)[node * NDPN + c];
+      if constexpr (MODE == KU_JACOBI || MODE == KU_JACOBI_DOT) dv[c] = a.dinv[node * NDPN + c];
+    }
+    T fhi[4 * NDPN], un[NDPN], up[4 * NDPN];
+    plane_modes<NDPN, T>(plane[(z + 1) & 1], tx, ty, fhi, un);
+    S.modes();
+    sym_layer<NDPN, T, CG>(a, S, flo, fhi, carry, up);
+    // carry now holds plane z's in-plane modes from both layers: corner values,
+    // summed over the element columns in y (DPP) and x (LDS)
+    T acc[NDPN];
+    T* xo = xch[z & 1];
+#pragma unroll
+    for (int c = 0; c < NDPN; ++c) {
+      const T p = carry[c] + carry[2 * NDPN + c], q = carry[c] - carry[2 * NDPN + c];
+      const T r = carry[NDPN + c] + carry[3 * NDPN + c], s = carry[NDPN + c] - carry[3 * NDPN + c];
+      xo[c * BS + tid] = (q + s) + next_lane(p + r);
+      acc[c] = (q - s) + next_lane(p - r);
+    }
+    if (more) st.store(plane[z & 1], beta);
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int c = 0; c < NDPN; ++c) {
+        acc[c] += xo[c * BS + tid + TE];
+        const int64_t g = node * NDPN + c;
+        const bool fixed = (mk >> c) & 1;
+        TO* y = static_cast<TO*>(a.y);
+        if constexpr (FUSEP) a.pout[g] = uc[c];
+        if constexpr (MODE == KU_STORE || MODE == KU_STORE_DOT) {
+          const T v = fixed ? T(0) : acc[c];
+          y[g] = TO(v);
+          if constexpr (MODE == KU_STORE_DOT) dot += double(uc[c]) * double(v);
+        } else if constexpr (MODE == KU_RESID) {
+          y[g] = TO(fixed ? T(0) : T(bv[c]) - acc[c]);
+        } else {
+          const T bb = T(bv[c]);
+          const T v = fixed ? T(0) : uc[c] + a.omega * dv[c] * (bb - acc[c]);
+          y[g] = TO(v);
+          if constexpr (MODE == KU_JACOBI_DOT) dot += double(bb) * double(v);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4 * NDPN; ++i) {
+      flo[i] = fhi[i];
+      carry[i] = up[i];
+    }
+#pragma unroll
+    for (int c = 0; c < NDPN; ++c) uc[c] = un[c];
+    S = Sn;
+  }
+}
+
+// The ncol * nz (tile column, node plane) units are split evenly over the
+// workgroups, in column order; each walks one or more column segments, and a
+// segment costs one extra element layer (the one below its first plane).  Two
+// waves per SIMD: 170-184 VGPRs in FP64 (256 for the level-1 form); a bound of
+// three spills (192x96x96, FP64: residual 40.2 instead of 39.9 us, level-1
+// sweep 45.6 instead of 17.2).
+//
+// Measured at 192x96x96 (kernel times, against the general kernels): FP64
+// residual 52.1 -> 39.9 us (146.7 MB; 3.7 TB/s of the 5.1 a copy reaches), last
+// smoothing sweep 53.7 -> 45.7, product with the search-direction update
+// 19.4 + 52.9 -> 52.5; level-1 residual and sweep 59.4 and 54.4 (stored
+// stencil, 252 MB) -> 17.3 and 17.2.
+template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
+__global__ __launch_bounds__(BS, 2) void sym_kernel(SymArgs<T> a) {
+  if (a.done && *a.done) return;
+  __shared__ T plane[2][TS * TS * NDPN];
+  __shared__ T xch[2][NDPN * BS];
+  // workgroups go round-robin over the 8 XCDs: give each a contiguous range
+  const unsigned nb = gridDim.x, hw = blockIdx.x;
+  const unsigned xcd = hw & 7u, q = nb >> 3, r = nb & 7u;
+  const unsigned w = xcd * q + min(xcd, r) + (hw >> 3);
+  const unsigned units = a.ncol * unsigned(a.nz);  // units * (nb + 1) < 2^32 (launcher)
+  unsigned u0 = __builtin_amdgcn_readfirstlane(units * w / nb);
+  const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
+  T beta = T(0);
+  if constexpr (FUSEP) beta = T(*a.beta);
+  double dot = 0.0;
+  while (u0 < u1) {
+    const unsigned col = u0 / unsigned(a.nz);
+    const int z0 = int(u0 - col * unsigned(a.nz));
+    const int z1 = min(a.nz, z0 + int(u1 - u0));
+    sym_segment<NDPN, T, MODE, TB, TO, FUSEP, CG>(a, plane, xch, col, z0, z1, beta, dot);
+    u0 += unsigned(z1 - z0);
+  }
+  if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
+    __shared__ double sh[BS / 64 + 2];
+    double v[1] = {dot};
+    block_sum<1>(v, sh);
+    store_partials<1>(v, a.partials);
+  }
+}
+
+// workgroups the device holds at once (cached per device and kernel)
+int sym_slots(const void* kernel, int64_t& slots) {
+  static std::mutex mu;
+  static std::map<std::pair<int, const void*>, int64_t> cache;
+  int dev = 0;
+  TL_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lk(mu);
+  auto it = cache.find({dev, kernel});
+  if (it == cache.end()) {
+    int ncu = 0, per = 0;
+    TL_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    TL_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, BS, 0));
+    it = cache.emplace(std::make_pair(dev, kernel), int64_t(std::max(ncu, 1)) * std::max(per, 1)).first;
+  }
+  slots = it->second;
+  return TL_OK;
+}
+
+int64_t tile_cols(const Grid& g) {
+  return int64_t((g.nx + TN - 1) / TN) * ((g.ny + TN - 1) / TN);
+}
+
+template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
+int sym_launch(hipStream_t s, const Grid& g, SymArgs<T> a, unsigned* nblocks) {
+  auto* kern = sym_kernel<NDPN, T, MODE, TB, TO, FUSEP, CG>;
+  a.nelx = g.nelx; a.nely = g.nely; a.nelz = g.nelz;
+  a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
+  a.ncy = (g.ny + TN - 1) / TN;
+  a.ncol = unsigned(tile_cols(g));
+  int64_t slots = 0;
+  TL_TRY(sym_slots(reinterpret_cast<const void*>(kern), slots));
+  const int64_t units = int64_t(a.ncol) * g.nz;
+  const int64_t nwg = std::max<int64_t>(1, std::min<int64_t>({slots, units, int64_t(kMaxRedBlocks)}));
+  TL_ARG(units * (nwg + 1) < (int64_t(1) << 32), "internal: grid too large for the tiled operator");
+  if (nblocks) *nblocks = unsigned(nwg);
+  hipLaunchKernelGGL(kern, dim3(unsigned(nwg)), dim3(BS), 0, s, a);
+  TL_CHECK_LAUNCH();
+  return TL_OK;
+}
+
+// 24x24 (8x8) matrix in the Hadamard basis, B = H K H^T / 64
+void to_modes(int ndpn, const double* K, double* B) {
+  const int nd = 8 * ndpn;
+  auto sign = [](int m, int k) {
+    return ((m & 1) * loc_dx(k) + (m >> 1 & 1) * loc_dy(k) + (m >> 2) * loc_dz(k)) & 1 ? -1.0 : 1.0;
+  };
+  std::vector<double> t(size_t(nd) * nd);
+  for (int m = 0; m < 8; ++m)
+    for (int c = 0; c < ndpn; ++c)
+      for (int j = 0; j < nd; ++j) {
+        double s = 0.0;
+        for (int k = 0; k < 8; ++k) s += sign(m, k) * K[size_t(k * ndpn + c) * nd + j];
+        t[size_t(m * ndpn + c) * nd + j] = s;
+      }
+  for (int i = 0; i < nd; ++i)
+    for (int m = 0; m < 8; ++m)
+      for (int c = 0; c < ndpn; ++c) {
+        double s = 0.0;
+        for (int k = 0; k < 8; ++k) s += sign(m, k) * t[size_t(i) * nd + k * ndpn + c];
+        B[size_t(i) * nd + m * ndpn + c] = s / 64.0;
+      }
+}
+
+// Group values of `n` entries against their pattern; false when an entry
+// differs by more than 1e-13 of the largest.
+bool match(const double* v, size_t n, const signed char* tab, const int* first, int ng, double* kv) {
+  double mx = 0.0;
+  for (size_t i = 0; i < n; ++i) mx = std::max(mx, std::fabs(v[i]));
+  for (int g = 0; g < ng; ++g) kv[g] = v[first[g]];
+  for (size_t i = 0; i < n; ++i) {
+    const int p = tab[i];
+    const double want = p == 0 ? 0.0 : (p > 0 ? kv[p - 1] : -kv[-p - 1]);
+    if (!(std::fabs(want - v[i]) <= 1e-13 * mx)) return false;
+  }
+  return true;
+}
+
+}  // namespace
+
+// Whether KE has the reflection-symmetric pattern; fills the group values of
+// the fine operator and of the level-1 Galerkin operator (G: the 8 child
+// matrices, child (cz 2 + cx) 2 + cy).
+bool sym_detect(int ndpn, const double* KE, double (&kv)[16]) {
+  const int nd = 8 * ndpn;
+  std::vector<double> B(size_t(nd) * nd);
+  to_modes(ndpn, KE, B.data());
+  if (ndpn == 3)
+    return match(B.data(), B.size(), kTabSym_elast, kFirstSym_elast, kGroupsSym_elast, kv);
+  if (ndpn == 1)
+    return match(B.data(), B.size(), kTabSym_poisson, kFirstSym_poisson, kGroupsSym_poisson, kv);
+  return false;
+}
+
+bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]) {
+  if (ndpn != 1 && ndpn != 3) return false;
+  const int nd = 8 * ndpn;
+  const size_t n2 = size_t(nd) * nd;
+  std::vector<double> B(8 * n2), K(n2);
+  for (int m = 0; m < 8; ++m) {
+    for (size_t i = 0; i < n2; ++i) {
+      double s = 0.0;
+      for (int c = 0; c < 8; ++c) {
+        const int cy = c & 1, cx = c >> 1 & 1, cz = c >> 2;
+        const bool neg = ((m & 1) * cx + (m >> 1 & 1) * cy + (m >> 2) * cz) & 1;
+        s += neg ? -G[size_t(c) * n2 + i] : G[size_t(c) * n2 + i];
+      }
+      K[i] = s / 8.0;
+    }
+    to_modes(ndpn, K.data(), B.data() + m * n2);
+  }
+  if (ndpn == 3)
+    return match(B.data(), B.size(), kTabSymC_elast, kFirstSymC_elast, kGroupsSymC_elast, kv);
+  return match(B.data(), B.size(), kTabSymC_poisson, kFirstSymC_poisson, kGroupsSymC_poisson, kv);
+}
+
+// The tiled operators take a 3D grid whose launch arithmetic and in-plane
+// offsets fit 32 bits.
+bool sym_fits(const Grid& g, int ndpn) {
+  if (g.dim != 3 || (ndpn != 1 && ndpn != 3)) return false;
+  const int64_t units = tile_cols(g) * g.nz;
+  return units * (kMaxRedBlocks + 1) < (int64_t(1) << 32) &&
+         int64_t(g.nx) * g.ny * ndpn < (int64_t(1) << 31);
+}
+
+template <int NDPN, typename T>
+static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, bool out64, bool fusep,
+                     unsigned* nb) {
+  hipStream_t s = P->stream;
+  const Grid& g = P->g;
+  switch (mode) {
+    case KU_STORE:
+      if (out64) return sym_launch<NDPN, T, KU_STORE, T, double, false, false>(s, g, a, nb);
+      return sym_launch<NDPN, T, KU_STORE, T, T, false, false>(s, g, a, nb);
+    case KU_STORE_DOT:
+      if (fusep) return sym_launch<NDPN, T, KU_STORE_DOT, T, T, true, false>(s, g, a, nb);
+      return sym_launch<NDPN, T, KU_STORE_DOT, T, T, false, false>(s, g, a, nb);
+    case KU_RESID:
+      if (b64) return sym_launch<NDPN, T, KU_RESID, double, T, false, false>(s, g, a, nb);
+      break;
+    case KU_JACOBI:
+      if (b64) return sym_launch<NDPN, T, KU_JACOBI, double, T, false, false>(s, g, a, nb);
+      break;
+    case KU_JACOBI_DOT:
+      if (b64) return sym_launch<NDPN, T, KU_JACOBI_DOT, double, double, false, false>(s, g, a, nb);
+      break;
+  }
+  set_error("internal: unsupported mode of the tiled operator");
+  return TL_EINVAL;
+}
+
+template <int NDPN, typename T>
+static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void* b, bool b64,
+                     const void* dinv, double omega, const void* pin, void* pout,
+                     const double* beta, double* partials, const int* done, bool out64,
+                     unsigned* nb) {
+  SymArgs<T> a{};
+  a.u = static_cast<const T*>(u);
+  a.pin = static_cast<const T*>(pin);
+  a.pout = static_cast<T*>(pout);
+  a.beta = beta;
+  a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
+                        : reinterpret_cast<const T*>(P->op.sp32.ptr);
+  a.mask = P->op.mask.as<uint8_t>();
+  a.b = b;
+  a.dinv = static_cast<const T*>(dinv);
+  a.omega = T(omega);
+  a.y = y;
+  a.partials = partials;
+  a.done = done;
+  for (int g = 0; g < 16; ++g) a.kv[g] = T(P->op.symkv[g]);
+  return fine_mode<NDPN, T>(P, a, mode, b64, out64, pin != nullptr, nb);
+}
+
+int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
+                   bool b64, const void* dinv, double omega, const void* pin, void* pout,
+                   const double* beta, double* partials, const int* done, bool out64,
+                   unsigned* nb) {
+  const bool f64 = prec == TL_PREC_FP64;
+  if (P->ndpn == 3)
+    return f64 ? fine_call<3, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
+                                      done, out64, nb)
+               : fine_call<3, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
+                                     done, out64, nb);
+  return f64 ? fine_call<1, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
+                                    done, out64, nb)
+             : fine_call<1, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
+                                   done, out64, nb);
+}
+
+template <int NDPN, typename T>
+static int coarse_call(tl_problem* P, int mode, const T* x, const T* b, T* y, const int* done) {
+  const Level& L = P->mg.lv[1];
+  SymArgs<T> a{};
+  a.u = x;
+  a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
+                        : reinterpret_cast<const T*>(P->op.sp32.ptr);
+  a.mask = L.mask.as<uint8_t>();
+  a.b = b;
+  a.dinv = reinterpret_cast<const T*>(sizeof(T) == 8 ? L.dinv64.ptr : L.dinv32.ptr);
+  a.omega = T(P->mg.omega);
+  a.y = y;
+  a.done = done;
+  a.fnelx = P->g.nelx;
+  a.fnely = P->g.nely;
+  for (int g = 0; g < 16; ++g) a.kv[g] = T(P->mg.symkv[g]);
+  if (mode == 0) return sym_launch<NDPN, T, KU_RESID, T, T, false, true>(P->stream, L.g, a, nullptr);
+  return sym_launch<NDPN, T, KU_JACOBI, T, T, false, true>(P->stream, L.g, a, nullptr);
+}
+
+int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* b, void* y,
+                     const int* done) {
+  if (P->ndpn == 3)
+    return f64 ? coarse_call<3, double>(P, mode, static_cast<const double*>(x),
+                                        static_cast<const double*>(b), static_cast<double*>(y), done)
+               : coarse_call<3, float>(P, mode, static_cast<const float*>(x),
+                                       static_cast<const float*>(b), static_cast<float*>(y), done);
+  return f64 ? coarse_call<1, double>(P, mode, static_cast<const double*>(x),
+                                      static_cast<const double*>(b), static_cast<double*>(y), done)
+             : coarse_call<1, float>(P, mode, static_cast<const float*>(x),
+                                     static_cast<const float*>(b), static_cast<float*>(y), done);
+}
+
+}  // namespace tl
