@@ -94,3 +94,42 @@ def test_level1_from_densities(gpu, dims, nlevels, ndpn):
         got, _ = op.solve(op.full(torch.as_tensor(b, device=gpu)), maxiter=1, raise_on_fail=False)
         assert rel(got[op._free_t].cpu().numpy(), ref) < tol, prec
     op.close()
+
+
+# convolution layers: result channels and nodes in tiles of 16, source channels
+# in 1, 2, 4, 8 or 16 groups of 4; one channel, partial and several tiles, one
+# node, more node tiles than workgroups
+@pytest.mark.parametrize("stride,shape,cin,cout", [(1, (1, 1, 1), 1, 1), (1, (3, 5, 7), 4, 17),
+                                                   (2, (3, 5, 7), 5, 16), (1, (2, 3, 17), 9, 33),
+                                                   (2, (9, 5, 5), 17, 5), (1, (1, 4, 16), 33, 64),
+                                                   (1, (29, 31, 33), 3, 6)])
+def test_conv_tiles(gpu, stride, shape, cin, cout):
+    """Forward, data gradient (accumulated) and weight gradient against the
+    oracle: fp32 sums of up to 64 x 27 products, 1e-5."""
+    import ctypes as C
+    import torch
+    from oracle import nn
+    from topoptlab_amd._lib import check, lib
+    say("conv tiles", stride, shape, cin, cout)
+    rng = np.random.default_rng(cin + cout)
+    a = rng.standard_normal((cin,) + shape).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 27)) * 0.2).astype(np.float16)
+    b = rng.standard_normal(cout).astype(np.float32)
+    y_ref = nn.conv3d(a.astype(np.float64), w.astype(np.float64), b.astype(np.float64), stride, False)
+    gy = rng.standard_normal(y_ref.shape).astype(np.float32)
+    ga_ref, gw_ref, gb_ref = nn.conv3d_backward(a.astype(np.float64), w.astype(np.float64),
+                                                gy.astype(np.float64), stride, None)
+    t = lambda v: torch.as_tensor(np.ascontiguousarray(v), device=gpu)
+    p = lambda v: C.c_void_p(v.data_ptr())
+    s = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    da, dw, db, dgy = t(a), t(w), t(b), t(gy)
+    y = torch.empty(y_ref.shape, dtype=torch.float32, device=gpu)
+    check(lib().tl_nn_conv3d(cin, cout, *shape, stride, 0, p(da), p(dw), p(db), p(y), s))
+    assert rel(y.cpu().numpy(), y_ref) < 1e-5
+    ga = torch.ones((cin,) + shape, dtype=torch.float32, device=gpu)
+    check(lib().tl_nn_conv3d_bwd_data(cin, cout, *shape, stride, p(dgy), p(dw), p(ga), 1, s))
+    assert rel(ga.cpu().numpy() - 1.0, ga_ref) < 1e-5
+    gw = torch.empty((cout, cin, 27), dtype=torch.float32, device=gpu)
+    gb = torch.empty(cout, dtype=torch.float32, device=gpu)
+    check(lib().tl_nn_conv3d_bwd_weight(cin, cout, *shape, stride, p(da), p(dgy), p(gw), p(gb), s))
+    assert rel(gw.cpu().numpy(), gw_ref) < 1e-5 and rel(gb.cpu().numpy(), gb_ref) < 1e-5

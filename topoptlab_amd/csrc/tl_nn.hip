@@ -10,141 +10,254 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace tl {
 namespace {
 
 constexpr int BS = 256;
-constexpr int CO = 8;  // output channels per thread (forward)
-constexpr int CI = 8;  // input channels per thread (data gradient)
 
 __device__ inline int tap_dz(int t) { return t / 9 - 1; }
 __device__ inline int tap_dx(int t) { return (t / 3) % 3 - 1; }
 __device__ inline int tap_dy(int t) { return t % 3 - 1; }
 
-// y[co][o] = relu?(b[co] + sum_ci sum_t w[co][ci][t] * a[ci][stride*o + off_t])
-__global__ __launch_bounds__(BS) void conv_fwd_kernel(int cin, int cout, int nz, int nx, int ny,
-                                                      int oz, int ox, int oy, int stride, int relu,
-                                                      const float* __restrict__ a,
-                                                      const _Float16* __restrict__ w,
-                                                      const float* __restrict__ b,
-                                                      float* __restrict__ y) {
-  extern __shared__ float wsh[];  // [CO][cin][27] as fp32
-  const int co0 = blockIdx.y * CO;
-  const int nco = min(CO, cout - co0);
-  for (int i = threadIdx.x; i < CO * cin * 27; i += BS) {
-    const int c = i / (cin * 27);
-    wsh[i] = c < nco ? float(w[int64_t(co0) * cin * 27 + i]) : 0.f;
-  }
-  __syncthreads();
-  const int64_t nout = int64_t(oz) * ox * oy;
-  const int64_t o = int64_t(blockIdx.x) * BS + threadIdx.x;
-  if (o >= nout) return;
-  const int iy = int(o % oy), ix = int((o / oy) % ox), iz = int(o / (int64_t(oy) * ox));
-  const int64_t plane = int64_t(nz) * nx * ny;
-  float acc[CO];
+// Forward convolution and its data gradient as an implicit product on the
+// FP32 matrix cores (v_mfma_f32_16x16x4f32: fp32 inputs, fp32 sums):
+//   forward  y[co][o] = relu?(b[co] + sum_t sum_ci w[co][ci][t] a[ci][stride*o + off_t])
+//   BWD      ga[ci][n] (+)= sum_t sum_co w[co][ci][t] gy[co][o], stride*o + off_t = n
+// rows = 16 channels of the result (blockIdx.y), columns = 16 consecutive nodes
+// of the result grid, inner dimension = 4 source channels of one tap.  A lane
+// loads one source value per product, 16 lanes a run of y.  The waves of
+// a workgroup take the taps in turn and their sums are added through LDS;
+// the workgroup's weights are staged once in LDS (fp16, [t][k][16 rows]) for
+// all its node tiles.
+//
+// The grids are small (4,225 nodes for a 48x24x24 design), so the split is
+// over channels and taps as well as nodes.  One thread per node and 8 result
+// channels, looping over all taps and source channels, left most of the chip
+// idle: 186 us (forward) and 148 us (gradient) per layer on average at that
+// size against 25 and 12 now (a design of 192x96x96: forward pass 2.5 -> 0.69
+// ms, forward and backward 26.3 -> 12.8 ms).
+typedef float nn_f4 __attribute__((ext_vector_type(4)));
+// NG: channel groups of 4, at least kc / 4; a power of two, so that every load
+// of a tap is issued before its first product.
+constexpr int CT = 512, CW = CT / 64;  // threads and waves of a workgroup
+template <bool BWD, int NG>
+__global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx, int ry, int sz,
+                                                  int sx, int sy, int stride, int relu,
+                                                  int accumulate, int ntiles,
+                                                  const float* __restrict__ src,
+                                                  const _Float16* __restrict__ w,
+                                                  const float* __restrict__ bias,
+                                                  float* __restrict__ out) {
+  constexpr int TP = 4 * NG * 16 + 2;  // tap pitch: staging writes of 27 taps in 27 banks
+  __shared__ _Float16 wl[27 * TP];     // [27][kp][16]
+  constexpr int kp = 4 * NG;
+  const int m0 = int(blockIdx.y) * 16;
+  // weights in their memory order ([rows][k][t], BWD [k][rows][t]), a batch of
+  // loads in flight
+  constexpr int NW = 27 * kp * 16, NB = 9;
+  for (int i0 = threadIdx.x; i0 < NW; i0 += CT * NB) {
+    _Float16 r[NB];
 #pragma unroll
-  for (int k = 0; k < CO; ++k) acc[k] = 0.f;
-  for (int t = 0; t < 27; ++t) {
-    const int Z = stride * iz + tap_dz(t), X = stride * ix + tap_dx(t), Y = stride * iy + tap_dy(t);
-    if (Z < 0 || Z >= nz || X < 0 || X >= nx || Y < 0 || Y >= ny) continue;
-    const int64_t src = (int64_t(Z) * nx + X) * ny + Y;
-    for (int c = 0; c < cin; ++c) {
-      const float v = a[int64_t(c) * plane + src];
+    for (int b = 0; b < NB; ++b) {
+      const int i = i0 + b * CT;
+      const int k = BWD ? i / (27 * 16) : i / 27 % kp, m = BWD ? i / 27 % 16 : i / (27 * kp);
+      const bool in = i < NW && k < kc && m0 + m < mc;
+      const int64_t at = (BWD ? int64_t(k) * mc + m0 + m : int64_t(m0 + m) * kc + k) * 27 + i % 27;
+      r[b] = w[in ? at : 0];
+      r[b] = in ? r[b] : _Float16(0);
+    }
 #pragma unroll
-      for (int k = 0; k < CO; ++k) acc[k] = fmaf(wsh[(k * cin + c) * 27 + t], v, acc[k]);
+    for (int b = 0; b < NB; ++b) {
+      const int i = i0 + b * CT;
+      const int k = BWD ? i / (27 * 16) : i / 27 % kp, m = BWD ? i / 27 % 16 : i / (27 * kp);
+      if (i < NW) wl[i % 27 * TP + k * 16 + m] = r[b];
     }
   }
-  for (int k = 0; k < nco; ++k) {
-    float v = acc[k] + b[co0 + k];
-    if (relu) v = fmaxf(v, 0.f);
-    y[int64_t(co0 + k) * nout + o] = v;
+  __syncthreads();
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, j = l & 15, g = l >> 4;
+  const int64_t nres = int64_t(rz) * rx * ry, nsrc = int64_t(sz) * sx * sy;
+  // source values of tap t for the lane's node (0 where the tap has none)
+  auto load = [&](int t, int Z, int X, int Y, float (&v)[NG]) {
+    int z, x, y;
+    bool ok;
+    if constexpr (BWD) {
+      const int pz = Z - tap_dz(t), px = X - tap_dx(t), py = Y - tap_dy(t);
+      z = pz / stride; x = px / stride; y = py / stride;
+      ok = pz >= 0 && px >= 0 && py >= 0 && z < sz && x < sx && y < sy &&
+           !(stride == 2 && ((pz | px | py) & 1));
+    } else {
+      z = stride * Z + tap_dz(t); x = stride * X + tap_dx(t); y = stride * Y + tap_dy(t);
+      ok = z >= 0 && z < sz && x >= 0 && x < sx && y >= 0 && y < sy;
+    }
+    const float* p = src + (ok ? (int64_t(z) * sx + x) * sy + y : 0);
+#pragma unroll
+    for (int q = 0; q < NG; ++q) {
+      const int c = 4 * q + g;
+      v[q] = p[int64_t(c < kc ? c : 0) * nsrc];
+      v[q] = ok && c < kc ? v[q] : 0.f;
+    }
+  };
+  auto product = [&](int t, const float (&v)[NG], nn_f4& acc) {
+    const _Float16* wt = wl + t * TP + g * 16 + j;
+#pragma unroll
+    for (int q = 0; q < NG; ++q)
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(float(wt[q * 64]), v[q], acc, 0, 0, 0);
+  };
+  auto node = [&](int64_t o, int& Z, int& X, int& Y) {
+    o = o < nres ? o : nres - 1;
+    Y = int(o % ry); X = int((o / ry) % rx); Z = int(o / (int64_t(ry) * rx));
+  };
+  if constexpr (!BWD) {
+    // a wave per node tile, all taps in order: the sum of every output keeps
+    // the order of a loop over taps and source channels
+    for (int tile = int(blockIdx.x) * CW + wave; tile < ntiles; tile += int(gridDim.x) * CW) {
+      const int64_t o = int64_t(tile) * 16 + j;
+      int Z, X, Y;
+      node(o, Z, X, Y);
+      nn_f4 acc{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 27; t += 3) {
+        float v[3][NG];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) load(t + q, Z, X, Y, v[q]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) product(t + q, v[q], acc);
+      }
+      if (o < nres) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = m0 + 4 * g + i;
+          if (m >= mc) continue;
+          const float v = acc[i] + bias[m];
+          out[int64_t(m) * nres + o] = relu ? fmaxf(v, 0.f) : v;
+        }
+      }
+    }
+  } else {
+    // the waves share a node tile, taps in turn, sums added through LDS
+    __shared__ float red[CW][16][16];
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+      int Z, X, Y;
+      node(int64_t(tile) * 16 + j, Z, X, Y);
+      nn_f4 acc{0.f, 0.f, 0.f, 0.f};
+      for (int t = wave; t < 27; t += CW) {
+        float v[NG];
+        load(t, Z, X, Y, v);
+        product(t, v, acc);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[wave][4 * g + i][j] = acc[i];
+      __syncthreads();
+      const int m = threadIdx.x >> 4, n = threadIdx.x & 15;
+      const int64_t on = int64_t(tile) * 16 + n;
+      if (threadIdx.x < 256 && m0 + m < mc && on < nres) {
+        float v = 0.f;
+#pragma unroll
+        for (int q = 0; q < CW; ++q) v += red[q][m][n];
+        float* dst = out + int64_t(m0 + m) * nres + on;
+        *dst = accumulate ? *dst + v : v;
+      }
+      __syncthreads();
+    }
   }
 }
 
-// ga[ci][n] (+)= sum_co sum_t w[co][ci][t] * gy[co][o] over outputs o with
-// stride*o + off_t = n
-__global__ __launch_bounds__(BS) void conv_bwd_data_kernel(int cin, int cout, int nz, int nx,
-                                                           int ny, int oz, int ox, int oy,
-                                                           int stride, int accumulate,
-                                                           const float* __restrict__ gy,
-                                                           const _Float16* __restrict__ w,
-                                                           float* __restrict__ ga) {
-  extern __shared__ float wsh[];  // [cout][CI][27] as fp32
-  const int ci0 = blockIdx.y * CI;
-  const int nci = min(CI, cin - ci0);
-  for (int i = threadIdx.x; i < cout * CI * 27; i += BS) {
-    const int co = i / (CI * 27), k = (i / 27) % CI, t = i % 27;
-    wsh[i] = k < nci ? float(w[(int64_t(co) * cin + ci0 + k) * 27 + t]) : 0.f;
-  }
-  __syncthreads();
-  const int64_t nin = int64_t(nz) * nx * ny;
-  const int64_t n = int64_t(blockIdx.x) * BS + threadIdx.x;
-  if (n >= nin) return;
-  const int Y = int(n % ny), X = int((n / ny) % nx), Z = int(n / (int64_t(ny) * nx));
-  const int64_t nout = int64_t(oz) * ox * oy;
-  float acc[CI];
-#pragma unroll
-  for (int k = 0; k < CI; ++k) acc[k] = 0.f;
-  for (int t = 0; t < 27; ++t) {
-    const int pz = Z - tap_dz(t), px = X - tap_dx(t), py = Y - tap_dy(t);
-    if (stride == 2 && ((pz | px | py) & 1)) continue;
-    const int iz = pz / stride, ix = px / stride, iy = py / stride;
-    if (pz < 0 || px < 0 || py < 0 || iz >= oz || ix >= ox || iy >= oy) continue;
-    const int64_t src = (int64_t(iz) * ox + ix) * oy + iy;
-    for (int co = 0; co < cout; ++co) {
-      const float g = gy[int64_t(co) * nout + src];
-#pragma unroll
-      for (int k = 0; k < CI; ++k) acc[k] = fmaf(wsh[(co * CI + k) * 27 + t], g, acc[k]);
-    }
-  }
-  const int64_t plane = nin;
-  for (int k = 0; k < nci; ++k) {
-    float* p = ga + int64_t(ci0 + k) * plane + n;
-    *p = accumulate ? *p + acc[k] : acc[k];
-  }
+// Workgroups per 16 result channels: a workgroup stages up to 55 KB of weights
+// before its first tile, so beyond two rounds of the chip (two workgroups of
+// that size per CU) a workgroup takes several tiles.
+constexpr int64_t kConvGroups = 1024;
+
+template <bool BWD>
+int conv_launch(int kc, int mc, int rz, int rx, int ry, int sz, int sx, int sy, int stride,
+                int relu, int accumulate, const float* src, const uint16_t* w16,
+                const float* bias, float* out, void* stream) {
+  const int64_t ntiles = (int64_t(rz) * rx * ry + 15) / 16, mt = (mc + 15) / 16;
+  TL_ARG(ntiles < (int64_t(1) << 31) && mt < 65536, "grid too large for the convolution");
+  const int64_t groups = BWD ? ntiles : (ntiles + CW - 1) / CW;
+  const int64_t gx = std::min<int64_t>(groups, kConvGroups / std::min<int64_t>(mt, 4));
+  auto go = [&](auto ng) {
+    hipLaunchKernelGGL((conv_kernel<BWD, decltype(ng)::value>), dim3(unsigned(gx), unsigned(mt)),
+                       dim3(CT), 0, static_cast<hipStream_t>(stream), kc, mc, rz, rx, ry, sz, sx, sy,
+                       stride, relu, accumulate, int(ntiles), src,
+                       reinterpret_cast<const _Float16*>(w16), bias, out);
+  };
+  if (kc <= 4) go(std::integral_constant<int, 1>{});
+  else if (kc <= 8) go(std::integral_constant<int, 2>{});
+  else if (kc <= 16) go(std::integral_constant<int, 4>{});
+  else if (kc <= 32) go(std::integral_constant<int, 8>{});
+  else go(std::integral_constant<int, 16>{});  // the entry points admit at most 64
+  TL_CHECK_LAUNCH();
+  return TL_OK;
 }
 
-// gw[co][ci][t] = sum_o gy[co][o] * a[ci][stride*o + off_t]; gb[co] = sum_o gy[co][o]
-// One workgroup per (co, ci): fixed-order strided partial sums, then the
-// fixed block tree.
-__global__ __launch_bounds__(BS) void conv_bwd_weight_kernel(int cin, int cout, int nz, int nx,
-                                                             int ny, int oz, int ox, int oy,
-                                                             int stride,
-                                                             const float* __restrict__ a,
-                                                             const float* __restrict__ gy,
-                                                             float* __restrict__ gw,
-                                                             float* __restrict__ gb) {
-  __shared__ double red[28][BS / 64];
-  const int co = blockIdx.x / cin, ci = blockIdx.x % cin;
-  const int64_t nout = int64_t(oz) * ox * oy;
-  const int64_t plane = int64_t(nz) * nx * ny;
-  double acc[28];
+// gw[co][ci][t] = sum_o gy[co][o] * a[ci][stride*o + off_t]; gb[co] = sum_o gy[co][o],
+// products and sums in FP64 on the matrix cores (v_mfma_f64_16x16x4f64, whose
+// operands are exact): rows = 16 output channels, columns = 16 input channels
+// of one tap (blockIdx.x = tap, .y = channel tile), inner dimension = 4 nodes.
+// The 16 waves of a workgroup take runs of 16 nodes in turn (so that the
+// nodes a lane reads in one channel lie in one line), and their sums are
+// added through LDS in a fixed order.  Tap 13 (the centre) also sums gy.
+// One workgroup per channel pair with 28 FP64 sums per thread: 62 us per
+// layer on average for a 48x24x24 design, 23 now.
+typedef double nn_d4 __attribute__((ext_vector_type(4)));
+constexpr int WG_WAVES = 16;
+__global__ __launch_bounds__(64 * WG_WAVES) void conv_bwd_weight_kernel(
+    int cin, int cout, int nz, int nx, int ny, int oz, int ox, int oy, int stride,
+    const float* __restrict__ a, const float* __restrict__ gy, float* __restrict__ gw,
+    float* __restrict__ gb) {
+  __shared__ double red[WG_WAVES][16][17];
+  const int t = int(blockIdx.x), cit = (cin + 15) / 16;
+  const int co0 = int(blockIdx.y) / cit * 16, ci0 = int(blockIdx.y) % cit * 16;
+  const int dz = tap_dz(t), dx = tap_dx(t), dy = tap_dy(t);
+  const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, j = l & 15, g = l >> 4;
+  const int64_t nout = int64_t(oz) * ox * oy, plane = int64_t(nz) * nx * ny;
+  const bool cok = co0 + j < cout, iok = ci0 + j < cin;
+  const float* gp = gy + int64_t(cok ? co0 + j : 0) * nout;
+  const float* ap = a + int64_t(iok ? ci0 + j : 0) * plane;
+  nn_d4 acc{0.0, 0.0, 0.0, 0.0};
+  double gs = 0.0;
+  // lane (j, g): nodes base + 4 g + k of channel row/column j, slice k = 0..3
+  for (int64_t base = int64_t(wave) * 16; base < nout; base += 16 * WG_WAVES) {
+    const int64_t o0 = base + 4 * g;
+    int y = int(o0 % oy), x = int((o0 / oy) % ox), z = int(o0 / (int64_t(oy) * ox));
+    float gv[4], av[4];
 #pragma unroll
-  for (int t = 0; t < 28; ++t) acc[t] = 0.0;
-  for (int64_t o = threadIdx.x; o < nout; o += BS) {
-    const int iy = int(o % oy), ix = int((o / oy) % ox), iz = int(o / (int64_t(oy) * ox));
-    const float g = gy[int64_t(co) * nout + o];
-#pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      const int Z = stride * iz + tap_dz(t), X = stride * ix + tap_dx(t), Y = stride * iy + tap_dy(t);
-      if (Z < 0 || Z >= nz || X < 0 || X >= nx || Y < 0 || Y >= ny) continue;
-      acc[t] += double(g) * double(a[int64_t(ci) * plane + (int64_t(Z) * nx + X) * ny + Y]);
+    for (int k = 0; k < 4; ++k) {
+      const bool in = o0 + k < nout;
+      const int Z = stride * z + dz, X = stride * x + dx, Y = stride * y + dy;
+      const bool ok = in && Z >= 0 && Z < nz && X >= 0 && X < nx && Y >= 0 && Y < ny;
+      const float gq = gp[in ? o0 + k : 0];
+      const float aq = ap[ok ? (int64_t(Z) * nx + X) * ny + Y : 0];
+      gv[k] = in && cok ? gq : 0.f;
+      gs += double(gv[k]);
+      gv[k] = ok ? gv[k] : 0.f;  // both operands: a skipped term stays out whatever it holds
+      av[k] = ok && iok ? aq : 0.f;
+      if (++y == oy) { y = 0; if (++x == ox) { x = 0; ++z; } }
     }
-    acc[27] += double(g);
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-  for (int t = 0; t < 28; ++t) {
-    const double s = wave_sum(acc[t]);
-    if (lane == 0) red[t][wid] = s;
+    for (int k = 0; k < 4; ++k)
+      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(double(gv[k]), double(av[k]), acc, 0, 0, 0);
   }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[wave][g + 4 * i][j] = acc[i];
   __syncthreads();
-  if (threadIdx.x < 28) {
+  if (threadIdx.x < 256) {
+    const int m = threadIdx.x >> 4, n = threadIdx.x & 15;
     double s = 0.0;
-    for (int k = 0; k < BS / 64; ++k) s += red[threadIdx.x][k];
-    if (threadIdx.x < 27) gw[(int64_t(co) * cin + ci) * 27 + threadIdx.x] = float(s);
-    else if (ci == 0) gb[co] = float(s);
+    for (int q = 0; q < WG_WAVES; ++q) s += red[q][m][n];
+    if (co0 + m < cout && ci0 + n < cin)
+      gw[(int64_t(co0 + m) * cin + ci0 + n) * 27 + t] = float(s);
+  }
+  if (t != 13 || ci0 != 0) return;
+  __syncthreads();
+  red[wave][g][j] = gs;
+  __syncthreads();
+  if (threadIdx.x < 16 && co0 + int(threadIdx.x) < cout) {
+    double s = 0.0;
+    for (int q = 0; q < WG_WAVES; ++q)
+      for (int r = 0; r < 4; ++r) s += red[q][r][threadIdx.x];
+    gb[co0 + threadIdx.x] = float(s);
   }
 }
 
@@ -370,13 +483,8 @@ int tl_nn_conv3d(int32_t cin, int32_t cout, int32_t nz, int32_t nx, int32_t ny, 
   TL_ARG(stride == 1 || (stride == 2 && nz % 2 == 1 && nx % 2 == 1 && ny % 2 == 1),
          "stride must be 1, or 2 on odd node counts");
   const int oz = out_dim(nz, stride), ox = out_dim(nx, stride), oy = out_dim(ny, stride);
-  const int64_t nout = int64_t(oz) * ox * oy;
-  const dim3 grid{unsigned((nout + BS - 1) / BS), unsigned((cout + CO - 1) / CO), 1u};
-  hipLaunchKernelGGL(conv_fwd_kernel, grid, dim3(BS), size_t(CO) * cin * 27 * sizeof(float),
-                     static_cast<hipStream_t>(stream), cin, cout, nz, nx, ny, oz, ox, oy, stride,
-                     relu, in, reinterpret_cast<const _Float16*>(w16), bias, out);
-  TL_CHECK_LAUNCH();
-  return TL_OK;
+  return conv_launch<false>(cin, cout, oz, ox, oy, nz, nx, ny, stride, relu, 0, in, w16, bias, out,
+                            stream);
 }
 
 int tl_nn_conv3d_bwd_data(int32_t cin, int32_t cout, int32_t nz, int32_t nx, int32_t ny,
@@ -388,13 +496,8 @@ int tl_nn_conv3d_bwd_data(int32_t cin, int32_t cout, int32_t nz, int32_t nx, int
   TL_ARG(stride == 1 || (stride == 2 && nz % 2 == 1 && nx % 2 == 1 && ny % 2 == 1),
          "stride must be 1, or 2 on odd node counts");
   const int oz = out_dim(nz, stride), ox = out_dim(nx, stride), oy = out_dim(ny, stride);
-  const int64_t nin = int64_t(nz) * nx * ny;
-  const dim3 grid{unsigned((nin + BS - 1) / BS), unsigned((cin + CI - 1) / CI), 1u};
-  hipLaunchKernelGGL(conv_bwd_data_kernel, grid, dim3(BS), size_t(cout) * CI * 27 * sizeof(float),
-                     static_cast<hipStream_t>(stream), cin, cout, nz, nx, ny, oz, ox, oy, stride,
-                     accumulate, gout, reinterpret_cast<const _Float16*>(w16), gin);
-  TL_CHECK_LAUNCH();
-  return TL_OK;
+  return conv_launch<true>(cout, cin, nz, nx, ny, oz, ox, oy, stride, 0, accumulate, gout, w16,
+                           nullptr, gin, stream);
 }
 
 int tl_nn_conv3d_bwd_weight(int32_t cin, int32_t cout, int32_t nz, int32_t nx, int32_t ny,
@@ -405,7 +508,9 @@ int tl_nn_conv3d_bwd_weight(int32_t cin, int32_t cout, int32_t nz, int32_t nx, i
   TL_ARG(stride == 1 || (stride == 2 && nz % 2 == 1 && nx % 2 == 1 && ny % 2 == 1),
          "stride must be 1, or 2 on odd node counts");
   const int oz = out_dim(nz, stride), ox = out_dim(nx, stride), oy = out_dim(ny, stride);
-  hipLaunchKernelGGL(conv_bwd_weight_kernel, dim3(unsigned(cout * cin)), dim3(BS), 0,
+  const int64_t tiles = int64_t((cout + 15) / 16) * ((cin + 15) / 16);
+  TL_ARG(tiles < 65536, "too many channels for the weight gradient");
+  hipLaunchKernelGGL(conv_bwd_weight_kernel, dim3(27, unsigned(tiles)), dim3(64 * WG_WAVES), 0,
                      static_cast<hipStream_t>(stream), cin, cout, nz, nx, ny, oz, ox, oy, stride,
                      in, gout, gw, gb);
   TL_CHECK_LAUNCH();
