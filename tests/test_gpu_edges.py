@@ -133,3 +133,25 @@ def test_conv_tiles(gpu, stride, shape, cin, cout):
     gb = torch.empty(cout, dtype=torch.float32, device=gpu)
     check(lib().tl_nn_conv3d_bwd_weight(cin, cout, *shape, stride, p(da), p(dgy), p(gw), p(gb), s))
     assert rel(gw.cpu().numpy(), gw_ref) < 1e-5 and rel(gb.cpu().numpy(), gb_ref) < 1e-5
+
+
+# one workgroup up to 8,192 elements (256 threads to 2,048, else 1,024), three
+# steps per pass beyond; partial rows, blocks and grids
+@pytest.mark.parametrize("n", [2, 255, 257, 2048, 2049, 8191, 8192, 8193, 131073])
+@pytest.mark.parametrize("l2", [1e9, 1e3, 1.0])  # 40 to 50 steps, 20 to 30, 10
+def test_oc_sizes(gpu, n, l2):
+    """Design bit for bit the oracle's, element flags included."""
+    import torch
+    from topoptlab_amd.optimizer import oc_top88
+    say("oc sizes", n, l2)
+    rng = np.random.default_rng(n)
+    x = 0.05 + 0.9 * rng.random(n)
+    dc = -10.0 ** rng.uniform(-4, 1, n)
+    dv = 0.5 + rng.random(n)
+    fl = rng.choice([0, 0, 0, 1, 2], n)
+    g = 0.01 * n
+    ref, gt = fem.oc_top88(x, 0.3, dc, dv, g, el_flags=fl, l2=l2)
+    t = lambda a: torch.as_tensor(a, device=gpu)
+    got, ggt = oc_top88(t(x), 0.3, t(dc), t(dv), g, el_flags=t(fl), l2=l2)
+    assert np.array_equal(got.cpu().numpy(), ref)
+    assert abs(ggt - gt) <= 1e-12 * np.abs(dv * (ref - x)).sum() + 1e-15

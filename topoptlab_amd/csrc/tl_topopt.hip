@@ -176,60 +176,182 @@ __global__ __launch_bounds__(BS) void fold_sum_kernel(const double* __restrict__
 // OC bisection (optimizer/optimality_criterion.py:61-77), device resident
 // ---------------------------------------------------------------------------
 struct OcState {
-  double l1, l2, g, gt, move;
+  double l1, l2, g, gt, move, lfin;
   int done, steps;
 };
 
-__global__ __launch_bounds__(BS) void oc_step_kernel(const double* __restrict__ x,
-                                                     const double* __restrict__ dc,
-                                                     const double* __restrict__ dv,
-                                                     const int32_t* __restrict__ flags, int64_t n,
-                                                     double* __restrict__ xnew, const OcState* st,
-                                                     double* partials) {
-  if (st->done) return;
-  const double lmid = 0.5 * (st->l2 + st->l1);
-  const double move = st->move;
-  // compensated (two-sum) accumulation so that the sign decision below is
-  // the sign of the exactly rounded total
-  double s = 0.0, comp = 0.0;
-  for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS) {
-    const double xi = x[i];
-    const double cand = xi * sqrt(-dc[i] / dv[i] / lmid);
-    double xn = fmax(0.0, fmax(xi - move, fmin(1.0, fmin(xi + move, cand))));
-    if (flags) {  // passive (1) elements are 0, active (2) elements are 1 (:68-71)
-      const int32_t fl = flags[i];
-      xn = fl == 1 ? 0.0 : (fl == 2 ? 1.0 : xn);
-    }
-    xnew[i] = xn;
-    // explicit rounding ops: a contracted FMA would break the two-sum
-    const double term = __dmul_rn(dv[i], __dsub_rn(xn, xi));
-    const double t = __dadd_rn(s, term);
-    const double bp = __dsub_rn(t, s);
-    comp = __dadd_rn(comp, __dadd_rn(__dsub_rn(s, __dsub_rn(t, bp)), __dsub_rn(term, bp)));
-    s = t;
-  }
-  __shared__ double sh[2 * (BS / 64) + 4];
-  double v[2] = {s, comp};
-  block_sum<2>(v, sh);
-  store_partials<2>(v, partials);
+// (:62-71) the new density for lambda lmid, q = -dc/dv; passive (1) elements
+// are 0, active (2) elements are 1
+__device__ __forceinline__ double oc_density(double x, double q, double lmid, double move,
+                                             int32_t flag) {
+  const double cand = x * sqrt(q / lmid);
+  const double xn = fmax(0.0, fmax(x - move, fmin(1.0, fmin(x + move, cand))));
+  return flag == 1 ? 0.0 : (flag == 2 ? 1.0 : xn);
 }
 
-// one block: gt = g + sum dv*(xnew - x); bisect (optimality_criterion.py:72-77)
-__global__ __launch_bounds__(BS) void oc_fold_kernel(const double* __restrict__ partials,
-                                                     unsigned nb, OcState* st) {
-  if (st->done) return;
-  __shared__ double sh[2 * (BS / 64) + 4];
-  double tot[2];
-  fold_partials<2>(partials, nb, tot, sh);
-  if (threadIdx.x == 0) {
-    const double lmid = 0.5 * (st->l2 + st->l1);
-    const double gt = st->g + (tot[0] + tot[1]);
-    st->gt = gt;
-    if (gt > 0) st->l1 = lmid;
-    else st->l2 = lmid;
-    st->steps += 1;
-    if (!((st->l2 - st->l1) / (st->l1 + st->l2) > 1e-3)) st->done = 1;
+// Compensated (two-sum) accumulation of dv*(xn - x), so that the sign decision
+// of a step is the sign of the exactly rounded total.  Explicit rounding ops:
+// a contracted FMA would break the two-sum.
+__device__ __forceinline__ void oc_add(double xn, double x, double dv, double& s, double& comp) {
+  const double term = __dmul_rn(dv, __dsub_rn(xn, x));
+  const double t = __dadd_rn(s, term);
+  const double bp = __dsub_rn(t, s);
+  comp = __dadd_rn(comp, __dadd_rn(__dsub_rn(s, __dsub_rn(t, bp)), __dsub_rn(term, bp)));
+  s = t;
+}
+
+// (:72-77) one bisection step for the midpoint's gt
+__device__ __forceinline__ void oc_decide(OcState& st, double lmid, double gt) {
+  st.gt = gt;
+  st.lfin = lmid;
+  if (gt > 0) st.l1 = lmid;
+  else st.l2 = lmid;
+  st.steps += 1;
+  if (!((st.l2 - st.l1) / (st.l1 + st.l2) > 1e-3)) st.done = 1;
+}
+
+// Designs of up to kOcSmall elements: the whole bisection in one workgroup,
+// eight elements per thread in registers.  A step is one evaluation and one
+// block sum (about 2 us) where two launches per step cost 5.3 us of kernel
+// time and their gaps; from 8,192 elements on the single workgroup's
+// evaluations cost as much.
+constexpr int64_t kOcSmall = 8192;
+constexpr int kOcElems = 8;
+__global__ __launch_bounds__(1024) void oc_small_kernel(const double* __restrict__ x,
+                                                        const double* __restrict__ dc,
+                                                        const double* __restrict__ dv,
+                                                        const int32_t* __restrict__ flags, int n,
+                                                        double* __restrict__ xnew, OcState st0,
+                                                        OcState* out) {
+  __shared__ double sh[2 * 16 + 4];
+  OcState st = st0;  // the same in every thread
+  const int bs = blockDim.x;
+  double xi[kOcElems], q[kOcElems], d[kOcElems];
+  int32_t fl[kOcElems];
+#pragma unroll
+  for (int e = 0; e < kOcElems; ++e) {
+    const int i = int(threadIdx.x) + e * bs;
+    xi[e] = q[e] = d[e] = 0.0;
+    fl[e] = 0;
+    if (i < n) {
+      xi[e] = x[i];
+      d[e] = dv[i];
+      q[e] = -dc[i] / d[e];
+      if (flags) fl[e] = flags[i];
+    }
   }
+  const int ne = (n + bs - 1) / bs;
+  while (!st.done && st.steps < 400) {
+    const double lmid = 0.5 * (st.l2 + st.l1);
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int e = 0; e < kOcElems; ++e)
+      if (e < ne && int(threadIdx.x) + e * bs < n)
+        oc_add(oc_density(xi[e], q[e], lmid, st.move, fl[e]), xi[e], d[e], v[0], v[1]);
+    block_sum<2>(v, sh);
+    oc_decide(st, lmid, st.g + (v[0] + v[1]));
+  }
+  if (st.steps > 0) {
+#pragma unroll
+    for (int e = 0; e < kOcElems; ++e) {
+      const int i = int(threadIdx.x) + e * bs;
+      if (i < n) xnew[i] = oc_density(xi[e], q[e], st.lfin, st.move, fl[e]);
+    }
+  }
+  if (threadIdx.x == 0) *out = st;
+}
+
+// Larger designs: three bisection steps per pass.  The 1 + 2 + 4 midpoints that
+// the three steps can reach are evaluated together (seven independent sums
+// per element hide each other's square roots and divisions), the fold then
+// takes the three decisions in order.  Midpoint k's children are 2k + 1 (gt <=
+// 0) and 2k + 2 (gt > 0).  Sixteen passes instead of 48 steps for an usual
+// bisection: 32 instead of 96 launches.
+constexpr int kOcMids = 7;
+constexpr int kOcThreads = 512;
+__device__ __forceinline__ void oc_midpoints(double l1, double l2, double (&m)[kOcMids]) {
+  double lo[kOcMids], hi[kOcMids];
+  lo[0] = l1;
+  hi[0] = l2;
+#pragma unroll
+  for (int k = 0; k < kOcMids; ++k) {
+    m[k] = 0.5 * (hi[k] + lo[k]);
+    if (2 * k + 2 < kOcMids) {
+      lo[2 * k + 1] = lo[k];
+      hi[2 * k + 1] = m[k];
+      lo[2 * k + 2] = m[k];
+      hi[2 * k + 2] = hi[k];
+    }
+  }
+}
+
+__global__ __launch_bounds__(kOcThreads) void oc_pass_kernel(const double* __restrict__ x,
+                                                             const double* __restrict__ dc,
+                                                             const double* __restrict__ dv,
+                                                             const int32_t* __restrict__ flags,
+                                                             int64_t n, const OcState* st,
+                                                             double* partials, unsigned stride) {
+  if (st->done) return;
+  double m[kOcMids];
+  oc_midpoints(st->l1, st->l2, m);
+  const double move = st->move;
+  double v[2 * kOcMids];
+#pragma unroll
+  for (int k = 0; k < 2 * kOcMids; ++k) v[k] = 0.0;
+  for (int64_t i = blockIdx.x * int64_t(kOcThreads) + threadIdx.x; i < n;
+       i += int64_t(gridDim.x) * kOcThreads) {
+    const double xi = x[i], d = dv[i], q = -dc[i] / d;
+    const int32_t fl = flags ? flags[i] : 0;
+#pragma unroll
+    for (int k = 0; k < kOcMids; ++k)
+      oc_add(oc_density(xi, q, m[k], move, fl), xi, d, v[2 * k], v[2 * k + 1]);
+  }
+  __shared__ double sh[2 * kOcMids * (kOcThreads / 64)];
+  block_sum<2 * kOcMids>(v, sh);
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int k = 0; k < 2 * kOcMids; ++k) partials[k * stride + blockIdx.x] = v[k];
+  }
+}
+
+// one block, a wave per midpoint: its gt, then the decisions
+__global__ __launch_bounds__(512) void oc_fold_kernel(const double* __restrict__ partials,
+                                                      unsigned nb, unsigned stride, OcState* stp) {
+  if (stp->done) return;
+  __shared__ double tot[8];
+  const int k = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (k < kOcMids) {
+    double a = 0.0, c = 0.0;
+    for (unsigned b = lane; b < nb; b += 64) {
+      a += partials[(2 * k) * stride + b];
+      c += partials[(2 * k + 1) * stride + b];
+    }
+    a = wave_sum(a);
+    c = wave_sum(c);
+    if (lane == 0) tot[k] = a + c;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    OcState st = *stp;
+    for (int j = 0, at = 0; j < 3 && !st.done; ++j) {
+      const double gt = st.g + tot[at];
+      oc_decide(st, 0.5 * (st.l2 + st.l1), gt);
+      at = 2 * at + (gt > 0 ? 2 : 1);
+    }
+    *stp = st;
+  }
+}
+
+// the design of the last step's midpoint
+__global__ __launch_bounds__(BS) void oc_apply_kernel(const double* __restrict__ x,
+                                                      const double* __restrict__ dc,
+                                                      const double* __restrict__ dv,
+                                                      const int32_t* __restrict__ flags, int64_t n,
+                                                      double* __restrict__ xnew, const OcState* st) {
+  if (st->steps == 0) return;
+  const double lmid = st->lfin, move = st->move;
+  for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS)
+    xnew[i] = oc_density(x[i], -dc[i] / dv[i], lmid, move, flags ? flags[i] : 0);
 }
 
 __global__ __launch_bounds__(BS) void mean_maxdiff_kernel(const double* __restrict__ a,
@@ -299,28 +421,40 @@ Scratch& scratch_for_device() {
 }
 
 // The bisection of optimality_criterion.py:61-77 on `stream`, with the
-// block partials (two values, kMaxRedBlocks stride, at most kOcBlocks
-// blocks) and the state in caller-provided device memory.
-constexpr unsigned kOcBlocks = 1024;
+// block partials (kOcBlocks doubles per sum) and the state in caller-provided
+// device memory.
+constexpr unsigned kOcBlocks = 256;
 
 int oc_bisect(int64_t n, const double* x, const double* dc, const double* dv,
               const int32_t* el_flags, double g, double move, double l1, double l2,
               double* xnew, double* gt, hipStream_t s, double* partials, OcState* st) {
-  OcState h{l1, l2, g, g, move, 0, 0};
+  OcState h{l1, l2, g, g, move, 0.0, 0, 0};
   h.done = ((l2 - l1) / (l1 + l2) > 1e-3) ? 0 : 1;
-  TL_HIP(hipMemcpyAsync(st, &h, sizeof(OcState), hipMemcpyHostToDevice, s));
-  const unsigned nb = unsigned(std::min<int64_t>(nblk(n), kOcBlocks));
-  for (int launched = 0; launched < 400;) {
-    for (int k = 0; k < 16; ++k) {
-      hipLaunchKernelGGL(oc_step_kernel, dim3(nb), dim3(BS), 0, s, x, dc, dv, el_flags, n, xnew,
-                         st, partials);
-      hipLaunchKernelGGL(oc_fold_kernel, dim3(1), dim3(BS), 0, s, partials, nb, st);
-    }
+  if (n <= kOcSmall) {
+    hipLaunchKernelGGL(oc_small_kernel, dim3(1), dim3(n <= 2048 ? 256 : 1024), 0, s, x, dc, dv,
+                       el_flags, int(n), xnew, h, st);
     TL_CHECK_LAUNCH();
-    launched += 16;
     TL_HIP(hipMemcpyAsync(&h, st, sizeof(OcState), hipMemcpyDeviceToHost, s));
     TL_HIP(hipStreamSynchronize(s));
-    if (h.done) break;
+  } else {
+    TL_HIP(hipMemcpyAsync(st, &h, sizeof(OcState), hipMemcpyHostToDevice, s));
+    const unsigned nb =
+        unsigned(std::min<int64_t>((n + kOcThreads - 1) / kOcThreads, kOcBlocks));
+    // 48 steps before the first look at the state, then 12 at a time
+    for (int pass = 0, batch = 16; pass * 3 < 400; batch = 4) {
+      for (int k = 0; k < batch; ++k, ++pass) {
+        hipLaunchKernelGGL(oc_pass_kernel, dim3(nb), dim3(kOcThreads), 0, s, x, dc, dv, el_flags, n,
+                           st, partials, kOcBlocks);
+        hipLaunchKernelGGL(oc_fold_kernel, dim3(1), dim3(512), 0, s, partials, nb, kOcBlocks, st);
+      }
+      // (a design of an unfinished bisection is overwritten by the next one)
+      hipLaunchKernelGGL(oc_apply_kernel, dim3(std::min<unsigned>(nblk(n), 4096u)), dim3(BS), 0, s,
+                         x, dc, dv, el_flags, n, xnew, st);
+      TL_CHECK_LAUNCH();
+      TL_HIP(hipMemcpyAsync(&h, st, sizeof(OcState), hipMemcpyDeviceToHost, s));
+      TL_HIP(hipStreamSynchronize(s));
+      if (h.done) break;
+    }
   }
   TL_ARG(h.done, "OC bisection did not terminate within 400 steps");
   *gt = h.gt;
@@ -328,15 +462,16 @@ int oc_bisect(int64_t n, const double* x, const double* dc, const double* dv,
 }
 
 // Scratch of tl_oc_update_noalloc, statically allocated on every device the
-// library runs on: the block partials of oc_step_kernel (two values per
-// block at stride kMaxRedBlocks, at most kOcBlocks blocks) followed by the
-// bisection state.  41,216 bytes per device, held until the process ends.
-constexpr size_t kNoAllocPartialDoubles = size_t(kMaxRedBlocks) + kOcBlocks;
+// library runs on: the block partials of oc_pass_kernel (2 kOcMids sums of at
+// most kOcBlocks blocks) followed by the bisection state.  41,216 bytes per
+// device, held until the process ends.
+constexpr size_t kNoAllocPartialDoubles = 5120;
 constexpr size_t kNoAllocStateOffset = sizeof(double) * kNoAllocPartialDoubles;
 constexpr size_t kNoAllocScratchBytes = kNoAllocStateOffset + 256;
 static_assert(sizeof(OcState) <= 256, "bisection state must fit its scratch slot");
 static_assert(kNoAllocStateOffset % 256 == 0, "state slot must stay 256-byte aligned");
-static_assert(kOcBlocks <= kMaxRedBlocks, "oc_bisect's grid must fit the partial stride");
+static_assert(2 * kOcMids * kOcBlocks <= kNoAllocPartialDoubles, "the partials must fit");
+static_assert(2 * kOcMids * kOcBlocks <= 2 * kMaxRedBlocks, "the partials must fit the shared scratch");
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
