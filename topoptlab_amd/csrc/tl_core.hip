@@ -114,7 +114,8 @@ struct KuArgs {
   const void* u;        // input (T); with FUSEP: z
   const void* pin;      // FUSEP: previous p (T)
   void* pout;           // FUSEP: new p (T)
-  const double* beta;   // FUSEP: device scalar
+  const double* beta;   // FUSEP: device scalar, or the partials of rho
+  FoldIn rho;
   const void* sp;       // padded scale (T)
   const void* KE;       // element matrix (T), nd x nd row-major
   const uint8_t* mask;  // per node
@@ -184,8 +185,8 @@ __device__ inline void ku_epilogue(const KuArgs& a, int64_t node, const T (&uc)[
 }
 
 template <typename T>
-__device__ inline T stage_val(const KuArgs& a, int64_t g, bool fusep) {
-  if (fusep) return ldval<T>(a.u, g) + T(*a.beta) * ldval<T>(a.pin, g);
+__device__ inline T stage_val(const KuArgs& a, int64_t g, bool fusep, T beta) {
+  if (fusep) return ldval<T>(a.u, g) + beta * ldval<T>(a.pin, g);
   return ldval<T>(a.u, g);
 }
 
@@ -249,7 +250,8 @@ __device__ inline void node_sum(const KuArgs& a, const T (&U)[3][9][NDPN],
 }
 
 template <int NDPN, typename T>
-__device__ inline void stage_plane(const KuArgs& a, T* lds, int pz, int64_t j0, bool fusep) {
+__device__ inline void stage_plane(const KuArgs& a, T* lds, int pz, int64_t j0, bool fusep,
+                                   T beta) {
   const int L = BS + 2 * a.ny + 2;
   const int64_t base = j0 - a.ny - 1;
   const bool zin = pz >= 0 && pz < a.nz;
@@ -257,7 +259,7 @@ __device__ inline void stage_plane(const KuArgs& a, T* lds, int pz, int64_t j0, 
     const int64_t jj = base + t / NDPN;
     T v = T(0);
     if (zin && jj >= 0 && jj < a.plane)
-      v = stage_val<T>(a, (int64_t(pz) * a.plane + jj) * NDPN + (t % NDPN), fusep);
+      v = stage_val<T>(a, (int64_t(pz) * a.plane + jj) * NDPN + (t % NDPN), fusep, beta);
     lds[t] = v;
   }
 }
@@ -597,7 +599,10 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
   const int ix = int(uint32_t(jc) / uint32_t(a.ny)), iy = int(jc) - ix * a.ny;
   T U[3][9][NDPN];
   T S[3][4];
-  stage_plane<NDPN, T>(a, lds, 0, j0, FUSEP);
+  __shared__ double sh[BS / 64 + 2];
+  T beta = T(0);
+  if constexpr (FUSEP) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
+  stage_plane<NDPN, T>(a, lds, 0, j0, FUSEP, beta);
   // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
   {
     const T* sp = static_cast<const T*>(a.sp);
@@ -623,7 +628,6 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
     ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
-    __shared__ double sh[BS / 64 + 2];
     double v[1] = {dot};
     block_sum<1>(v, sh);
     store_partials_at<1>(v, a.partials, bid);
@@ -659,12 +663,15 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
   const int lx = threadIdx.x / TY, ly = threadIdx.x % TY;
   const int ix = x0 + lx, iy = y0 + ly;
   const bool active = ix < a.nx && iy < a.ny;
+  __shared__ double sh[BS / 64 + 2];
+  T beta = T(0);
+  if constexpr (FUSEP) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
   for (int t = threadIdx.x; t < HN * NDPN; t += BS) {
     const int h = t / NDPN, c = t % NDPN;
     const int hx = x0 - 1 + h / HY, hy = y0 - 1 + h % HY;
     T v = T(0);
     if (hx >= 0 && hx < a.nx && hy >= 0 && hy < a.ny)
-      v = stage_val<T>(a, (int64_t(hx) * a.ny + hy) * NDPN + c, FUSEP);
+      v = stage_val<T>(a, (int64_t(hx) * a.ny + hy) * NDPN + c, FUSEP, beta);
     lds[t] = v;
   }
   T U[3][9][NDPN];
@@ -702,7 +709,6 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
     ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
-    __shared__ double sh[BS / 64 + 2];
     double v[1] = {dot};
     block_sum<1>(v, sh);
     store_partials_at<1>(v, a.partials, bid);
@@ -911,6 +917,13 @@ static int dispatch_mode(const tl_problem* P, const KuArgs& a, int mode, bool fu
 static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, bool fusep, bool b64,
                                bool out64);
 
+// Block partials of a reduction: rho, p.q and r.r have slots of their own,
+// because a consumer may still fold one while the next is written.
+static double* fin_partials(tl_problem* P, int fin) {
+  double* p = P->partials.as<double>();
+  return fin == FIN_PQ ? p + kMaxRedBlocks : (fin == FIN_RR ? p + 2 * kMaxRedBlocks : p);
+}
+
 // Generic entry used by the solver and the V-cycle.  prec selects T; b is
 // fp64 when b64; the output type is T except for KU_JACOBI_DOT (fp64) and
 // KU_STORE with prec fp32 and out64 (fp64 output).
@@ -922,11 +935,12 @@ int fine_apply_ex(tl_problem* P, const void* u, void* y, int prec, int mode, con
   a.u = u; a.y = y; a.b = b; a.dinv = dinv; a.omega = omega;
   a.pin = zfuse_pin; a.pout = pout; a.beta = beta;
   a.mask = P->op.mask.as<uint8_t>();
-  a.partials = P->partials.as<double>();
+  a.partials = fin_partials(P, fin);
   a.dot_out = dot_out;
   a.st = P->state.as<PcgState>();
   a.fin = fin;
   a.done = done;
+  if (zfuse_pin && P->rho_nb) a.rho = {fin_partials(P, FIN_RHO), P->rho_nb, a.st};
   for (int g = 0; g < 8; ++g) {
     a.kv64[g] = P->op.kv[g];
     a.kv32[g] = float(P->op.kv[g]);
@@ -978,7 +992,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
     }
     unsigned nb = 0;
     TL_TRY(sym_fine_apply(P, a.u, a.y, prec, mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
-                          a.partials, a.done, out64, &nb));
+                          a.rho, a.partials, a.done, out64, &nb));
     if (mode == KU_STORE_DOT || mode == KU_JACOBI_DOT)
       return launch_fold(P, nb, a.fin, a.dot_out, a.done);
     return TL_OK;
@@ -1195,12 +1209,14 @@ struct UpdateArgs {
   TS omega;
   const int* done;
   unsigned nb;  // blocks of the system's grid-stride loop
+  FoldIn pq;    // partials of p.q, or none: alpha is in the state
 };
 
 template <typename TS>
 __device__ __forceinline__ void update_body(const UpdateArgs<TS>& a, unsigned bid) {
   if (*a.done) return;
-  const double alpha = a.st->alpha;
+  __shared__ double sh[BS / 64 + 4];
+  const double alpha = fold_in_alpha(a.pq, a.st, sh);
   double s = 0.0;
   for (int64_t i = bid * int64_t(BS) + threadIdx.x; i < a.n; i += int64_t(a.nb) * BS) {
     const double xv = __builtin_nontemporal_load(&a.x[i]) + alpha * __builtin_nontemporal_load(&a.p[i]);
@@ -1211,7 +1227,6 @@ __device__ __forceinline__ void update_body(const UpdateArgs<TS>& a, unsigned bi
     if (a.xs) a.xs[i] = zero_guess_sweep<TS, double>(a.omega, a.dinv[i], rv);
   }
   double v[1] = {s};
-  __shared__ double sh[BS / 64 + 4];
   block_sum<1>(v, sh);
   store_partials_at<1>(v, a.partials, bid);
 }
@@ -1305,14 +1320,21 @@ static unsigned grid_for(int64_t n) {
 }
 
 static int launch_fold(tl_problem* P, unsigned nb, int fin, double* out, const int* done) {
+  if (fin == FIN_RHO || fin == FIN_PQ) {
+    // left to the consumer; the FP64 MFMA product reads beta from the state
+    const bool in = nb <= kFoldInBlocks && !(fin == FIN_RHO && P->op.mfma64);
+    (fin == FIN_RHO ? P->rho_nb : P->pq_nb) = in ? nb : 0u;
+    if (in) return TL_OK;
+  }
+  const double* partials = fin_partials(P, fin);
   if (P->rec) {
     P->rec->add(P->rec_phase, P->rec_level, &fold_multi_launch,
-                FoldArgs{P->partials.as<double>(), nb, fin, P->state.as<PcgState>(), out, done},
+                FoldArgs{partials, nb, fin, P->state.as<PcgState>(), out, done},
                 1u, 0);
     return TL_OK;
   }
-  hipLaunchKernelGGL(fold_kernel, dim3(1), dim3(BS), 0, P->stream, P->partials.as<double>(), nb,
-                     fin, P->state.as<PcgState>(), out, done);
+  hipLaunchKernelGGL(fold_kernel, dim3(1), dim3(BS), 0, P->stream, partials, nb, fin,
+                      P->state.as<PcgState>(), out, done);
   TL_CHECK_LAUNCH();
   return TL_OK;
 }
@@ -1623,10 +1645,11 @@ int pcg_init(tl_problem* P, const PcgCtx& c, const double* f, const double* x0, 
 __global__ __launch_bounds__(BS) void pupdate_kernel(const double* __restrict__ z,
                                                      const double* __restrict__ pin,
                                                      double* __restrict__ pout,
-                                                     const double* __restrict__ beta, int64_t n,
-                                                     const int* done) {
+                                                     const double* __restrict__ beta, FoldIn rho,
+                                                     int64_t n, const int* done) {
   if (*done) return;
-  const double b = *beta;
+  __shared__ double sh[BS / 64 + 2];
+  const double b = fold_in_beta(rho, beta, blockIdx.x == 0 && threadIdx.x == 0, sh);
   for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS)
     __builtin_nontemporal_store(__builtin_nontemporal_load(&z[i]) + b * __builtin_nontemporal_load(&pin[i]),
                                 &pout[i]);
@@ -1666,8 +1689,10 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     return TL_OK;
   }
   if (P->g.dim == 3 && !P->op.sym && !(P->op.mfma64 && P->ndpn == 3)) {
+    FoldIn rho;
+    if (P->rho_nb) rho = {fin_partials(P, FIN_RHO), P->rho_nb, c.st};
     hipLaunchKernelGGL(pupdate_kernel, dim3(c.nb), dim3(BS), 0, s, c.z, pin, pout, &c.st->beta,
-                       c.n, c.done);
+                       rho, c.n, c.done);
     TL_CHECK_LAUNCH();
     TL_TRY(fine_apply_ex(P, pout, c.q, TL_PREC_FP64, KU_STORE_DOT, nullptr, false, nullptr, 0.0,
                          nullptr, nullptr, nullptr, nullptr, FIN_PQ, c.done, false));
@@ -1676,6 +1701,9 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
                          pin, pout, &c.st->beta, nullptr, FIN_PQ, c.done, false));
   }
   // x += alpha p ; r -= alpha q ; rr ; done
+  FoldIn pq;
+  if (P->pq_nb) pq = {fin_partials(P, FIN_PQ), P->pq_nb, c.st};
+  double* rrp = fin_partials(P, FIN_RR);
   auto upd = [&](auto ua) -> int {
     using TS = std::remove_pointer_t<decltype(ua.xs)>;
     if (P->rec) {
@@ -1687,16 +1715,16 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     return TL_OK;
   };
   if (fx0 && P->mg.prec == TL_PREC_FP64)
-    TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, c.partials, c.st,
+    TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                   P->mg.lv[0].vx.as<double>(), P->op.dinv64.as<double>(),
-                                  P->mg.omega, c.done, c.rb}));
+                                  P->mg.omega, c.done, c.rb, pq}));
   else if (fx0)
-    TL_TRY(upd(UpdateArgs<float>{x, c.r, pout, c.q, c.n, c.partials, c.st,
+    TL_TRY(upd(UpdateArgs<float>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                  P->mg.lv[0].vx.as<float>(), P->op.dinv32.as<float>(),
-                                 float(P->mg.omega), c.done, c.rb}));
+                                 float(P->mg.omega), c.done, c.rb, pq}));
   else
-    TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, c.partials, c.st, nullptr, nullptr,
-                                  0.0, c.done, c.rb}));
+    TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, rrp, c.st, nullptr, nullptr,
+                                  0.0, c.done, c.rb, pq}));
   return launch_fold(P, c.rb, FIN_RR, nullptr, c.done);
 }
 

@@ -170,6 +170,37 @@ struct PcgState {
   int it, maxiter, done, pad;
 };
 
+// A PCG scalar whose block partials the consuming kernel folds itself (every
+// workgroup in the same fixed order as fold_kernel) instead of a one-block
+// kernel in between: a launch of 3.5-4.8 us less per scalar.  Beyond
+// kFoldInBlocks partials the reads of all workgroups together cost more than
+// the launch.  partials == nullptr: the scalar is in the state.
+constexpr unsigned kFoldInBlocks = 1024;
+struct FoldIn {
+  const double* partials = nullptr;
+  unsigned nb = 0;
+  PcgState* st = nullptr;
+};
+
+// beta = rho / rho_prev (0 in the first iteration); `writer` (one thread of the
+// grid) stores rho for the kernels after it.  sh: blockDim/64 + 2 doubles.
+__device__ __forceinline__ double fold_in_beta(const FoldIn& f, const double* beta, bool writer,
+                                               double* sh) {
+  if (!f.partials) return *beta;
+  double tot[1];
+  fold_partials<1>(f.partials, f.nb, tot, sh);
+  if (writer) f.st->rho = tot[0];
+  return f.st->it == 0 ? 0.0 : tot[0] / f.st->rho_prev;
+}
+
+// alpha = rho / p.q
+__device__ __forceinline__ double fold_in_alpha(const FoldIn& f, const PcgState* st, double* sh) {
+  if (!f.partials) return st->alpha;
+  double tot[1];
+  fold_partials<1>(f.partials, f.nb, tot, sh);
+  return st->rho / tot[0];
+}
+
 struct Level {
   void release();
   Grid g;
@@ -285,6 +316,8 @@ struct tl_problem {
   hipGraphExec_t chunk_exec = nullptr;
   int64_t chunk_key[5] = {-1, -1, -1, -1, -1};
   tl::DevBuf partials, state;
+  // rho and p.q partials left for their consumer to fold (0: in the state)
+  unsigned rho_nb = 0, pq_nb = 0;
   // launch timing of the fine operator (tl_profile)
   bool prof_on = false;
   std::vector<tl::ProfEvent> prof_used, prof_free;
@@ -319,8 +352,8 @@ bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]);
 bool sym_fits(const Grid& g, int ndpn);
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
-                   const double* beta, double* partials, const int* done, bool out64,
-                   unsigned* nblocks_out);
+                   const double* beta, const FoldIn& rho, double* partials, const int* done,
+                   bool out64, unsigned* nblocks_out);
 int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* b, void* y,
                      const int* done);
 }  // namespace tl

@@ -47,7 +47,8 @@ struct SymArgs {
   const T* u;          // input; FUSEP: z
   const T* pin;        // FUSEP: previous search direction
   T* pout;             // FUSEP: new search direction
-  const double* beta;  // FUSEP: device scalar
+  const double* beta;  // FUSEP: device scalar, or the partials of rho
+  FoldIn rho;
   const T* sp;         // zero-bordered scales of the fine grid
   const uint8_t* mask;
   const void* b;       // KU_RESID / KU_JACOBI*: right-hand side
@@ -407,8 +408,10 @@ __global__ __launch_bounds__(BS, 2) void sym_kernel(SymArgs<T> a) {
   const unsigned units = a.ncol * unsigned(a.nz);  // units * (nb + 1) < 2^32 (launcher)
   unsigned u0 = __builtin_amdgcn_readfirstlane(units * w / nb);
   const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
+  __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
-  if constexpr (FUSEP) beta = T(*a.beta);
+  if constexpr (FUSEP)
+    beta = T(fold_in_beta(a.rho, a.beta, blockIdx.x == 0 && threadIdx.x == 0, sh));
   double dot = 0.0;
   while (u0 < u1) {
     const unsigned col = u0 / unsigned(a.nz);
@@ -418,7 +421,6 @@ __global__ __launch_bounds__(BS, 2) void sym_kernel(SymArgs<T> a) {
     u0 += unsigned(z1 - z0);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
-    __shared__ double sh[BS / 64 + 2];
     double v[1] = {dot};
     block_sum<1>(v, sh);
     store_partials<1>(v, a.partials);
@@ -578,13 +580,14 @@ static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, boo
 template <int NDPN, typename T>
 static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void* b, bool b64,
                      const void* dinv, double omega, const void* pin, void* pout,
-                     const double* beta, double* partials, const int* done, bool out64,
-                     unsigned* nb) {
+                     const double* beta, const FoldIn& rho, double* partials, const int* done,
+                     bool out64, unsigned* nb) {
   SymArgs<T> a{};
   a.u = static_cast<const T*>(u);
   a.pin = static_cast<const T*>(pin);
   a.pout = static_cast<T*>(pout);
   a.beta = beta;
+  a.rho = rho;
   a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
                         : reinterpret_cast<const T*>(P->op.sp32.ptr);
   a.mask = P->op.mask.as<uint8_t>();
@@ -600,18 +603,18 @@ static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void
 
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
-                   const double* beta, double* partials, const int* done, bool out64,
-                   unsigned* nb) {
+                   const double* beta, const FoldIn& rho, double* partials, const int* done,
+                   bool out64, unsigned* nb) {
   const bool f64 = prec == TL_PREC_FP64;
   if (P->ndpn == 3)
-    return f64 ? fine_call<3, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
-                                      done, out64, nb)
-               : fine_call<3, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
-                                     done, out64, nb);
-  return f64 ? fine_call<1, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
-                                    done, out64, nb)
-             : fine_call<1, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, partials,
-                                   done, out64, nb);
+    return f64 ? fine_call<3, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
+                                      partials, done, out64, nb)
+               : fine_call<3, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
+                                     partials, done, out64, nb);
+  return f64 ? fine_call<1, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
+                                    partials, done, out64, nb)
+             : fine_call<1, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
+                                   partials, done, out64, nb);
 }
 
 template <int NDPN, typename T>
