@@ -1627,7 +1627,7 @@ int pcg_init(tl_problem* P, const PcgCtx& c, const double* f, const double* x0, 
   TL_TRY(launch_fold(P, c.rb, FIN_RR0, nullptr, nullptr));
   TL_HIP(hipMemsetAsync(c.pp[0], 0, sizeof(double) * n, s));
   TL_HIP(hipMemsetAsync(c.pp[1], 0, sizeof(double) * n, s));
-  if (pcg_fuses_x0(P, o->precond)) {
+  if (pcg_fuses_x0(P, o->precond) && !mg_seeds_x0(P)) {
     const MgState& M = P->mg;
     if (M.prec == TL_PREC_FP64)
       hipLaunchKernelGGL(zero_sweep_kernel<double>, dim3(c.nb), dim3(BS), 0, s, c.r,
@@ -1714,11 +1714,12 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     TL_CHECK_LAUNCH();
     return TL_OK;
   };
-  if (fx0 && P->mg.prec == TL_PREC_FP64)
+  const bool xs = fx0 && !mg_seeds_x0(P);  // the update also writes the first sweep
+  if (xs && P->mg.prec == TL_PREC_FP64)
     TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                   P->mg.lv[0].vx.as<double>(), P->op.dinv64.as<double>(),
                                   P->mg.omega, c.done, c.rb, pq}));
-  else if (fx0)
+  else if (xs)
     TL_TRY(upd(UpdateArgs<float>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                  P->mg.lv[0].vx.as<float>(), P->op.dinv32.as<float>(),
                                  float(P->mg.omega), c.done, c.rb, pq}));

@@ -334,6 +334,10 @@ int fine_diag(tl_problem* P);
 // launch timing (tl_profile): no-ops while profiling is off
 int prof_begin(tl_problem* P, int kind, ProfEvent& ev);
 int prof_end(tl_problem* P, ProfEvent& ev);
+// Whether the V-cycle forms its fine level's first (zero-guess) sweep, and the
+// iterate after the coarse correction, inside its two tiled operator calls:
+// no fine iterate is stored.  3D V(1,1) cycles in FP64 or FP32.
+bool mg_seeds_x0(const tl_problem* P);
 // x0_ready: the fine level's first (zero-guess) smoothing sweep is already
 // in lv[0].vx (written by the PCG's residual update, see pcg_fuses_x0)
 int mg_vcycle(tl_problem* P, const double* r, double* z, const int* done, bool x0_ready);
@@ -354,8 +358,8 @@ int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, co
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
                    const double* beta, const FoldIn& rho, double* partials, const int* done,
                    bool out64, unsigned* nblocks_out);
-int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* b, void* y,
-                     const int* done);
+int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* xc,
+                     const void* b, void* y, const int* done);
 }  // namespace tl
 
 // First damped-Jacobi sweep from a zero guess, x = omega * dinv * b, in the

@@ -31,7 +31,8 @@
 #include <cmath>
 #include <map>
 #include <mutex>
-#include <tuple>
+#include <type_traits>
+#include <utility>
 
 namespace tl {
 namespace {
@@ -42,13 +43,28 @@ constexpr int TN = TE - 1;   // nodes produced per tile side
 constexpr int TS = TE + 1;   // nodes staged per tile side
 static_assert(TE * TE == BS, "one element column per thread");
 
+// What a staged node value is (the operator's input x):
+enum {
+  SRC_U = 0,          // u
+  SRC_P = 1,          // z + beta p, the new search direction (written out for the own nodes)
+  SRC_SEED = 2,       // omega D^-1 b, the first sweep from a zero guess
+  SRC_CORR = 3,       // u + (P xc) on the free DOFs: the iterate after the coarse correction
+  SRC_SEED_CORR = 4,  // omega D^-1 b + (P xc)
+};
+constexpr bool src_seed(int s) { return s == SRC_SEED || s == SRC_SEED_CORR; }
+constexpr bool src_corr(int s) { return s == SRC_CORR || s == SRC_SEED_CORR; }
+constexpr int TC = 10;  // coarse nodes per tile side that 17 staged nodes interpolate from
+constexpr int CR = 4;   // coarse tiles kept in LDS
+
 template <typename T>
 struct SymArgs {
-  const T* u;          // input; FUSEP: z
-  const T* pin;        // FUSEP: previous search direction
-  T* pout;             // FUSEP: new search direction
-  const double* beta;  // FUSEP: device scalar, or the partials of rho
+  const T* u;          // input; SRC_P: z
+  const T* pin;        // SRC_P: previous search direction
+  T* pout;             // SRC_P: new search direction
+  const double* beta;  // SRC_P: device scalar, or the partials of rho
   FoldIn rho;
+  const T* xc;         // SRC_*CORR: the coarse level's correction
+  int cnx, cny, cnz;   // and its node counts
   const T* sp;         // zero-bordered scales of the fine grid
   const uint8_t* mask;
   const void* b;       // KU_RESID / KU_JACOBI*: right-hand side
@@ -218,12 +234,25 @@ __device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, C
 }
 
 // Staging of one node plane: the thread's entries of the 17x17x NDPN tile,
-// loaded into registers and stored to LDS later.
-template <int NDPN, typename T, bool FUSEP>
+// loaded into registers and stored to LDS later.  With a coarse correction the
+// stored value adds the in-plane interpolation of the coarse tile of its plane
+// (`ring`, plane z at z % CR, already interpolated in z): in a direction with
+// an even coordinate both neighbours are the coinciding coarse node, so one
+// average serves every case.
+template <int NDPN, typename T, typename TB, int SRC>
 struct Stage {
   static constexpr int N = TS * TS * NDPN, NR = (N + BS - 1) / BS;
+  static constexpr bool kTwo = SRC == SRC_P || src_seed(SRC), kCorr = src_corr(SRC);
+  using V = std::conditional_t<src_seed(SRC), TB, T>;
   uint32_t off[NR];  // entry offsets within a plane (clamped to the grid)
-  T v[NR], w[FUSEP ? NR : 1];
+  int co[kCorr ? NR : 1];      // coarse tile entry, + 1024 if y is odd, + 2048 if x is odd
+  struct Vals {  // a plane's values in flight
+    V v[NR];
+    T w[kTwo ? NR : 1];
+    uint8_t mk[kCorr ? NR : 1];  // masks of the entries' nodes
+    int z;                       // the plane asked for (past the grid: the last one is held)
+  };
+  __device__ __forceinline__ bool has(int k) const { return k + 1 < NR || int(threadIdx.x) + k * BS < N; }
   __device__ __forceinline__ void init(const SymArgs<T>& a, int x0, int y0) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
@@ -231,29 +260,107 @@ struct Stage {
       const int row = e / (TS * NDPN), rem = e % (TS * NDPN);
       const int x = min(max(x0 - 1 + row, 0), a.nx - 1), y = min(max(y0 - 1 + rem / NDPN, 0), a.ny - 1);
       off[k] = uint32_t((x * a.ny + y) * NDPN + rem % NDPN);
+      if constexpr (kCorr)
+        co[k] = (((x >> 1) - coarse_base(x0)) * TC + (y >> 1) - coarse_base(y0)) * NDPN + rem % NDPN +
+                (y & 1) * 1024 + (x & 1) * 2048;
     }
   }
-  __device__ __forceinline__ void load(const SymArgs<T>& a, int z) {
+  __device__ __forceinline__ static int coarse_base(int x0) { return max(x0 - 1, 0) >> 1; }
+  __device__ __forceinline__ void load(const SymArgs<T>& a, int z, Vals& q) const {
+    q.z = z;
     const int64_t base = int64_t(min(max(z, 0), a.nz - 1)) * a.nx * a.ny * NDPN;
-    const T* p = a.u + base;
+    const V* p = (src_seed(SRC) ? static_cast<const V*>(a.b) : reinterpret_cast<const V*>(a.u)) + base;
 #pragma unroll
     for (int k = 0; k < NR; ++k)
-      if (k + 1 < NR || int(threadIdx.x) + k * BS < N) v[k] = p[off[k]];
-    if constexpr (FUSEP) {
-      const T* q = a.pin + base;
+      if (has(k)) q.v[k] = p[off[k]];
+    if constexpr (kTwo) {
+      const T* p2 = (src_seed(SRC) ? a.dinv : a.pin) + base;
 #pragma unroll
       for (int k = 0; k < NR; ++k)
-        if (k + 1 < NR || int(threadIdx.x) + k * BS < N) w[k] = q[off[k]];
+        if (has(k)) q.w[k] = p2[off[k]];
+    }
+    if constexpr (kCorr) {
+      const uint8_t* m = a.mask + int64_t(min(max(z, 0), a.nz - 1)) * a.nx * a.ny;
+#pragma unroll
+      for (int k = 0; k < NR; ++k)
+        if (has(k)) q.mk[k] = m[off[k] / NDPN];
     }
   }
-  __device__ __forceinline__ void store(T* lds, T beta) const {
+  __device__ __forceinline__ T value(const SymArgs<T>& a, int k, const Vals& q, T beta) const {
+    if constexpr (SRC == SRC_P) return T(q.v[k]) + beta * q.w[k];
+    else if constexpr (src_seed(SRC)) return zero_guess_sweep<T, TB>(a.omega, q.w[k], q.v[k]);
+    else return q.v[k];
+  }
+  __device__ __forceinline__ void store(const SymArgs<T>& a, T* lds, const T* ring, T beta,
+                                        const Vals& q) const {
 #pragma unroll
     for (int k = 0; k < NR; ++k)
-      if (k + 1 < NR || int(threadIdx.x) + k * BS < N) {
-        if constexpr (FUSEP) lds[threadIdx.x + k * BS] = v[k] + beta * w[k];
-        else lds[threadIdx.x + k * BS] = v[k];
+      if (has(k)) {
+        T r = value(a, k, q, beta);
+        if constexpr (kCorr) {
+          const int e = co[k] & 1023, dy = (co[k] & 1024) ? NDPN : 0, dx = (co[k] & 2048) ? TC * NDPN : 0;
+          const T* c = ring + (q.z % CR) * (TC * TC * NDPN) + e;
+          const T s = T(0.25) * ((c[0] + c[dy]) + (c[dx] + c[dx + dy]));
+          if (!((q.mk[k] >> (off[k] % NDPN)) & 1)) r += s;
+        }
+        lds[threadIdx.x + k * BS] = r;
       }
   }
+};
+
+// The thread's entries of the coarse 10x10 tiles (clamped to the grid).  Fine
+// plane z interpolates from coarse planes z/2 and (z+1)/2; `next` holds the
+// latter of the plane prepared last.
+template <int NDPN, typename T>
+struct CoarseStage {
+  static constexpr int N = TC * TC * NDPN, NR = (N + BS - 1) / BS;
+  uint32_t off[NR];
+  T cur[NR], next[NR];
+  __device__ __forceinline__ bool has(int k) const { return int(threadIdx.x) + k * BS < N; }
+  __device__ __forceinline__ void load(const SymArgs<T>& a, int c, T (&v)[NR]) const {
+    const T* p = a.xc + int64_t(min(c, a.cnz - 1)) * a.cnx * a.cny * NDPN;
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (has(k)) v[k] = p[off[k]];
+  }
+  // Tiles of planes z0 - 1 (if any) to z0 + 2.
+  __device__ __forceinline__ void begin(const SymArgs<T>& a, int x0, int y0, int z0, T* ring) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) {
+      const int e = int(threadIdx.x) + k * BS;
+      const int x = min((max(x0 - 1, 0) >> 1) + e / (TC * NDPN), a.cnx - 1);
+      const int y = min((max(y0 - 1, 0) >> 1) + e % (TC * NDPN) / NDPN, a.cny - 1);
+      off[k] = uint32_t((x * a.cny + y) * NDPN + e % NDPN);
+    }
+    const int z = max(z0 - 1, 0);
+    T v[NR];
+    load(a, z >> 1, cur);
+    load(a, (z + 1) >> 1, next);
+    load(a, (z + 2) >> 1, v);
+    put(ring, z, cur, next);
+    put(ring, z + 1, next, v);
+    load(a, (z + 3) >> 1, cur);
+    put(ring, z + 2, v, cur);
+    if (z0 > 0) {
+      load(a, (z + 4) >> 1, next);
+      put(ring, z + 3, cur, next);
+    } else {
+#pragma unroll
+      for (int k = 0; k < NR; ++k) next[k] = cur[k];
+    }
+  }
+  __device__ __forceinline__ void put(T* ring, int z, const T (&lo)[NR], const T (&hi)[NR]) const {
+#pragma unroll
+    for (int k = 0; k < NR; ++k)
+      if (has(k)) ring[(z % CR) * N + threadIdx.x + k * BS] = T(0.5) * (lo[k] + hi[k]);
+  }
+  // Start of the step that prepares plane z, and its end.
+  __device__ __forceinline__ void advance(const SymArgs<T>& a, int z) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) cur[k] = next[k];
+    if (z & 1) load(a, (z + 1) >> 1, next);
+  }
+  __device__ __forceinline__ void finish(T* ring, int z) const { put(ring, z, cur, next); }
 };
 
 // In-plane modes of the thread's element from the staged plane, and the value
@@ -275,32 +382,41 @@ __device__ __forceinline__ void plane_modes(const T* lds, int tx, int ty, T (&f)
 }
 
 // Node planes z0 .. z1-1 of tile column col.
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
 __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS * TS * NDPN],
-                                            T (*xch)[NDPN * BS], unsigned col, int z0, int z1,
-                                            T beta, double& dot) {
+                                            T (*xch)[NDPN * BS], T* ring, unsigned col, int z0,
+                                            int z1, T beta, double& dot) {
+  constexpr bool CORR = src_corr(SRC);
   const int tid = int(threadIdx.x), tx = tid >> 4, ty = tid & 15;
   const int x0 = int(col / unsigned(a.ncy)) * TN, y0 = int(col % unsigned(a.ncy)) * TN;
   const int ix = x0 + tx, iy = y0 + ty;
   const bool active = tx < TN && ty < TN && ix < a.nx && iy < a.ny;
   const int64_t node0 = active ? int64_t(ix) * a.ny + iy : 0;
   const int64_t nplane = int64_t(a.nx) * a.ny;
-  Stage<NDPN, T, FUSEP> st;
+  Stage<NDPN, T, TB, SRC> st;
+  CoarseStage<NDPN, T> cs;
   Scales<T, CG> S, Sn;
   T flo[4 * NDPN], uc[NDPN], carry[4 * NDPN];
+  // (planes z0 - 1, z0 and z0 + 1 requested together: product and residual 3 us
+  // slower at 192x96x96)
+  typename Stage<NDPN, T, TB, SRC>::Vals in;
   st.init(a, x0, y0);
-  st.load(a, z0);
+  st.load(a, z0, in);
   S.load(a, ix, iy, z0);
   __syncthreads();  // the LDS of the previous segment is free
-  st.store(plane[z0 & 1], beta);
+  if constexpr (CORR) {
+    cs.begin(a, x0, y0, z0, ring);
+    __syncthreads();
+  }
+  st.store(a, plane[z0 & 1], ring, beta, in);
 #pragma unroll
   for (int i = 0; i < 4 * NDPN; ++i) carry[i] = T(0);
   if (z0 > 0) {  // the layer below gives plane z0's lower part
     Scales<T, CG> Sb;
-    st.load(a, z0 - 1);
+    st.load(a, z0 - 1, in);
     Sb.load(a, ix, iy, z0 - 1);
-    st.store(plane[(z0 + 1) & 1], beta);
-    st.load(a, z0 + 1);
+    st.store(a, plane[(z0 + 1) & 1], ring, beta, in);
+    st.load(a, z0 + 1, in);
     __syncthreads();
     T fb[4 * NDPN], unused[4 * NDPN], ub[NDPN];
     plane_modes<NDPN, T>(plane[(z0 + 1) & 1], tx, ty, fb, ub);
@@ -310,18 +426,19 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
     Sb.modes();
     sym_layer<NDPN, T, CG>(a, Sb, fb, flo, unused, carry);
   } else {
-    st.load(a, z0 + 1);
+    st.load(a, z0 + 1, in);
     __syncthreads();
     plane_modes<NDPN, T>(plane[z0 & 1], tx, ty, flo, uc);
   }
   if (z0 > 0) __syncthreads();  // plane z0 - 1 has been read
-  st.store(plane[(z0 + 1) & 1], beta);
+  st.store(a, plane[(z0 + 1) & 1], ring, beta, in);
   __syncthreads();
   for (int z = z0; z < z1; ++z) {
     const bool more = z + 1 < z1;  // uniform
     if (more) {
-      st.load(a, z + 2);
+      st.load(a, z + 2, in);
       Sn.load(a, ix, iy, z + 1);
+      if constexpr (CORR) cs.advance(a, z + 3);  // plane z + 3 is staged in the next step
     }
     // epilogue inputs of the node of plane z
     const int64_t node = int64_t(z) * nplane + node0;
@@ -349,7 +466,10 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
       xo[c * BS + tid] = (q + s) + next_lane(p + r);
       acc[c] = (q - s) + next_lane(p - r);
     }
-    if (more) st.store(plane[z & 1], beta);
+    if (more) {
+      st.store(a, plane[z & 1], ring, beta, in);
+      if constexpr (CORR) cs.finish(ring, z + 3);
+    }
     __syncthreads();
     if (active) {
 #pragma unroll
@@ -358,7 +478,7 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
         const int64_t g = node * NDPN + c;
         const bool fixed = (mk >> c) & 1;
         TO* y = static_cast<TO*>(a.y);
-        if constexpr (FUSEP) a.pout[g] = uc[c];
+        if constexpr (SRC == SRC_P) a.pout[g] = uc[c];
         if constexpr (MODE == KU_STORE || MODE == KU_STORE_DOT) {
           const T v = fixed ? T(0) : acc[c];
           y[g] = TO(v);
@@ -384,6 +504,11 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
   }
 }
 
+template <int NDPN, typename T, int SRC, bool CG>
+constexpr int sym_waves() {
+  return NDPN == 3 && sizeof(T) == 8 && CG && src_corr(SRC) ? 1 : 2;
+}
+
 // The ncol * nz (tile column, node plane) units are split evenly over the
 // workgroups, in column order; each walks one or more column segments, and a
 // segment costs one extra element layer (the one below its first plane).  Two
@@ -394,13 +519,19 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
 // Measured at 192x96x96 (kernel times, against the general kernels): FP64
 // residual 52.1 -> 39.9 us (146.7 MB; 3.7 TB/s of the 5.1 a copy reaches), last
 // smoothing sweep 53.7 -> 45.7, product with the search-direction update
-// 19.4 + 52.9 -> 52.5; level-1 residual and sweep 59.4 and 54.4 (stored
-// stencil, 252 MB) -> 17.3 and 17.2.
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
-__global__ __launch_bounds__(BS, 2) void sym_kernel(SymArgs<T> a) {
+// 19.4 + 52.9 -> 54; level-1 residual and sweep 59.4 and 54.4 (stored
+// stencil, 252 MB) -> 17.3 and 17.2.  Inside V(1,1) cycles: residual from the
+// seed 45, last sweep from the seed and the coarse correction 57.5 (45.7 and a
+// prolongation of 33 before), level-1 sweep with the correction 24 (17.2 + 7),
+// and 9 us less in the PCG update, which no longer writes the seed.
+// Measured and not kept: two layers per loop turn without the register moves
+// (the sweep spills, the rest is unchanged: the moves are not what bounds it).
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
+__global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kernel(SymArgs<T> a) {
   if (a.done && *a.done) return;
   __shared__ T plane[2][TS * TS * NDPN];
   __shared__ T xch[2][NDPN * BS];
+  __shared__ T ring[src_corr(SRC) ? CR * TC * TC * NDPN : 1];
   // workgroups go round-robin over the 8 XCDs: give each a contiguous range
   const unsigned nb = gridDim.x, hw = blockIdx.x;
   const unsigned xcd = hw & 7u, q = nb >> 3, r = nb & 7u;
@@ -410,14 +541,14 @@ __global__ __launch_bounds__(BS, 2) void sym_kernel(SymArgs<T> a) {
   const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
   __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
-  if constexpr (FUSEP)
+  if constexpr (SRC == SRC_P)
     beta = T(fold_in_beta(a.rho, a.beta, blockIdx.x == 0 && threadIdx.x == 0, sh));
   double dot = 0.0;
   while (u0 < u1) {
     const unsigned col = u0 / unsigned(a.nz);
     const int z0 = int(u0 - col * unsigned(a.nz));
     const int z1 = min(a.nz, z0 + int(u1 - u0));
-    sym_segment<NDPN, T, MODE, TB, TO, FUSEP, CG>(a, plane, xch, col, z0, z1, beta, dot);
+    sym_segment<NDPN, T, MODE, TB, TO, SRC, CG>(a, plane, xch, ring, col, z0, z1, beta, dot);
     u0 += unsigned(z1 - z0);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
@@ -449,9 +580,9 @@ int64_t tile_cols(const Grid& g) {
   return int64_t((g.nx + TN - 1) / TN) * ((g.ny + TN - 1) / TN);
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool CG>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
 int sym_launch(hipStream_t s, const Grid& g, SymArgs<T> a, unsigned* nblocks) {
-  auto* kern = sym_kernel<NDPN, T, MODE, TB, TO, FUSEP, CG>;
+  auto* kern = sym_kernel<NDPN, T, MODE, TB, TO, SRC, CG>;
   a.nelx = g.nelx; a.nely = g.nely; a.nelz = g.nelz;
   a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
   a.ncy = (g.ny + TN - 1) / TN;
@@ -552,25 +683,28 @@ bool sym_fits(const Grid& g, int ndpn) {
 }
 
 template <int NDPN, typename T>
-static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, bool out64, bool fusep,
+static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, bool out64, int src,
                      unsigned* nb) {
   hipStream_t s = P->stream;
   const Grid& g = P->g;
   switch (mode) {
     case KU_STORE:
-      if (out64) return sym_launch<NDPN, T, KU_STORE, T, double, false, false>(s, g, a, nb);
-      return sym_launch<NDPN, T, KU_STORE, T, T, false, false>(s, g, a, nb);
+      if (out64) return sym_launch<NDPN, T, KU_STORE, T, double, SRC_U, false>(s, g, a, nb);
+      return sym_launch<NDPN, T, KU_STORE, T, T, SRC_U, false>(s, g, a, nb);
     case KU_STORE_DOT:
-      if (fusep) return sym_launch<NDPN, T, KU_STORE_DOT, T, T, true, false>(s, g, a, nb);
-      return sym_launch<NDPN, T, KU_STORE_DOT, T, T, false, false>(s, g, a, nb);
+      if (src == SRC_P) return sym_launch<NDPN, T, KU_STORE_DOT, T, T, SRC_P, false>(s, g, a, nb);
+      return sym_launch<NDPN, T, KU_STORE_DOT, T, T, SRC_U, false>(s, g, a, nb);
     case KU_RESID:
-      if (b64) return sym_launch<NDPN, T, KU_RESID, double, T, false, false>(s, g, a, nb);
+      if (src == SRC_SEED) return sym_launch<NDPN, T, KU_RESID, double, T, SRC_SEED, false>(s, g, a, nb);
+      if (b64) return sym_launch<NDPN, T, KU_RESID, double, T, SRC_U, false>(s, g, a, nb);
       break;
     case KU_JACOBI:
-      if (b64) return sym_launch<NDPN, T, KU_JACOBI, double, T, false, false>(s, g, a, nb);
+      if (b64) return sym_launch<NDPN, T, KU_JACOBI, double, T, SRC_U, false>(s, g, a, nb);
       break;
     case KU_JACOBI_DOT:
-      if (b64) return sym_launch<NDPN, T, KU_JACOBI_DOT, double, double, false, false>(s, g, a, nb);
+      if (src == SRC_SEED_CORR)
+        return sym_launch<NDPN, T, KU_JACOBI_DOT, double, double, SRC_SEED_CORR, false>(s, g, a, nb);
+      if (b64) return sym_launch<NDPN, T, KU_JACOBI_DOT, double, double, SRC_U, false>(s, g, a, nb);
       break;
   }
   set_error("internal: unsupported mode of the tiled operator");
@@ -598,7 +732,18 @@ static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void
   a.partials = partials;
   a.done = done;
   for (int g = 0; g < 16; ++g) a.kv[g] = T(P->op.symkv[g]);
-  return fine_mode<NDPN, T>(P, a, mode, b64, out64, pin != nullptr, nb);
+  int src = pin ? SRC_P : SRC_U;
+  if (!u) {  // the V-cycle's first sweep on the fly, with the coarse correction in the last one
+    src = mode == KU_RESID ? SRC_SEED : SRC_SEED_CORR;
+    a.dinv = reinterpret_cast<const T*>(sizeof(T) == 8 ? P->op.dinv64.ptr : P->op.dinv32.ptr);
+    a.omega = T(P->mg.omega);
+    if (mode != KU_RESID) {
+      const Level& C = P->mg.lv[1];
+      a.xc = static_cast<const T*>(C.vx.ptr);
+      a.cnx = C.g.nx; a.cny = C.g.ny; a.cnz = C.g.nz;
+    }
+  }
+  return fine_mode<NDPN, T>(P, a, mode, b64, out64, src, nb);
 }
 
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
@@ -618,10 +763,12 @@ int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, co
 }
 
 template <int NDPN, typename T>
-static int coarse_call(tl_problem* P, int mode, const T* x, const T* b, T* y, const int* done) {
+static int coarse_call(tl_problem* P, int mode, const T* x, const T* xc, const T* b, T* y,
+                       const int* done) {
   const Level& L = P->mg.lv[1];
   SymArgs<T> a{};
   a.u = x;
+  a.xc = xc;
   a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
                         : reinterpret_cast<const T*>(P->op.sp32.ptr);
   a.mask = L.mask.as<uint8_t>();
@@ -633,21 +780,28 @@ static int coarse_call(tl_problem* P, int mode, const T* x, const T* b, T* y, co
   a.fnelx = P->g.nelx;
   a.fnely = P->g.nely;
   for (int g = 0; g < 16; ++g) a.kv[g] = T(P->mg.symkv[g]);
-  if (mode == 0) return sym_launch<NDPN, T, KU_RESID, T, T, false, true>(P->stream, L.g, a, nullptr);
-  return sym_launch<NDPN, T, KU_JACOBI, T, T, false, true>(P->stream, L.g, a, nullptr);
+  hipStream_t s = P->stream;
+  if (mode == 0) return sym_launch<NDPN, T, KU_RESID, T, T, SRC_U, true>(s, L.g, a, nullptr);
+  if (!xc) return sym_launch<NDPN, T, KU_JACOBI, T, T, SRC_U, true>(s, L.g, a, nullptr);
+  const Grid& gc = P->mg.lv[2].g;
+  a.cnx = gc.nx; a.cny = gc.ny; a.cnz = gc.nz;
+  return sym_launch<NDPN, T, KU_JACOBI, T, T, SRC_CORR, true>(s, L.g, a, nullptr);
 }
 
-int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* b, void* y,
-                     const int* done) {
-  if (P->ndpn == 3)
-    return f64 ? coarse_call<3, double>(P, mode, static_cast<const double*>(x),
-                                        static_cast<const double*>(b), static_cast<double*>(y), done)
-               : coarse_call<3, float>(P, mode, static_cast<const float*>(x),
-                                       static_cast<const float*>(b), static_cast<float*>(y), done);
-  return f64 ? coarse_call<1, double>(P, mode, static_cast<const double*>(x),
-                                      static_cast<const double*>(b), static_cast<double*>(y), done)
-             : coarse_call<1, float>(P, mode, static_cast<const float*>(x),
-                                     static_cast<const float*>(b), static_cast<float*>(y), done);
+// Level 1: y = b - A x (mode 0) or y = x' + omega D^-1 (b - A x') (mode 1), x' = x
+// or, with xc, x plus the coarse correction.
+int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* xc,
+                     const void* b, void* y, const int* done) {
+  auto go = [&](auto ndpn, auto t) {
+    using T = decltype(t);
+    return coarse_call<decltype(ndpn)::value, T>(P, mode, static_cast<const T*>(x),
+                                                 static_cast<const T*>(xc),
+                                                 static_cast<const T*>(b), static_cast<T*>(y), done);
+  };
+  using N1 = std::integral_constant<int, 1>;
+  using N3 = std::integral_constant<int, 3>;
+  if (P->ndpn == 3) return f64 ? go(N3{}, double{}) : go(N3{}, float{});
+  return f64 ? go(N1{}, double{}) : go(N1{}, float{});
 }
 
 }  // namespace tl
