@@ -111,11 +111,13 @@ __global__ void simp_pad_kernel(const double* __restrict__ x, double* __restrict
 // fine operator kernels
 // ----------------------------------------------------------------------------
 struct KuArgs {
-  const void* u;        // input (T); with FUSEP: z
-  const void* pin;      // FUSEP: previous p (T)
-  void* pout;           // FUSEP: new p (T)
-  const double* beta;   // FUSEP: device scalar, or the partials of rho
+  const void* u;        // input (T); with SRC_P: z
+  const void* pin;      // SRC_P: previous p (T)
+  void* pout;           // SRC_P: new p (T)
+  const double* beta;   // SRC_P: device scalar, or the partials of rho
   FoldIn rho;
+  const void* xc;       // SRC_SEED_CORR: the coarse level's correction (T)
+  int cny;              // and its node count in y
   const void* sp;       // padded scale (T)
   const void* KE;       // element matrix (T), nd x nd row-major
   const uint8_t* mask;  // per node
@@ -184,10 +186,25 @@ __device__ inline void ku_epilogue(const KuArgs& a, int64_t node, const T (&uc)[
   }
 }
 
-template <typename T>
-__device__ inline T stage_val(const KuArgs& a, int64_t g, bool fusep, T beta) {
-  if (fusep) return ldval<T>(a.u, g) + beta * ldval<T>(a.pin, g);
-  return ldval<T>(a.u, g);
+// Entry c of 2D node (ix, iy) as the operator's input (SRC_*).  The trilinear
+// correction averages the four coarse nodes around: in a direction with an
+// even coordinate both are the coinciding one.
+template <int NDPN, typename T, typename TB, int SRC>
+__device__ inline T stage_val(const KuArgs& a, int ix, int iy, int c, T beta) {
+  const int64_t node = int64_t(ix) * a.ny + iy, g = node * NDPN + c;
+  if constexpr (SRC == SRC_U) return ldval<T>(a.u, g);
+  else if constexpr (SRC == SRC_P) return ldval<T>(a.u, g) + beta * ldval<T>(a.pin, g);
+  else {
+    T v = zero_guess_sweep<T, TB>(T(a.omega), ldval<T>(a.dinv, g), ldval<TB>(a.b, g));
+    if constexpr (SRC == SRC_SEED_CORR) {
+      const int64_t x0 = int64_t(ix >> 1) * a.cny, x1 = int64_t((ix + 1) >> 1) * a.cny;
+      const int y0 = iy >> 1, y1 = (iy + 1) >> 1;
+      const T s = T(0.25) * ((ldval<T>(a.xc, (x0 + y0) * NDPN + c) + ldval<T>(a.xc, (x0 + y1) * NDPN + c)) +
+                             (ldval<T>(a.xc, (x1 + y0) * NDPN + c) + ldval<T>(a.xc, (x1 + y1) * NDPN + c)));
+      if (!((a.mask[node] >> c) & 1)) v += s;
+    }
+    return v;
+  }
 }
 
 // Contribution of the 4 (2D) / 8 (3D) elements around a node.
@@ -249,17 +266,19 @@ __device__ inline void node_sum(const KuArgs& a, const T (&U)[3][9][NDPN],
   }
 }
 
-template <int NDPN, typename T>
-__device__ inline void stage_plane(const KuArgs& a, T* lds, int pz, int64_t j0, bool fusep,
-                                   T beta) {
+// Nodes j0 - ny - 1 .. j0 + BS + ny of a 2D grid (0 outside it).
+template <int NDPN, typename T, typename TB, int SRC>
+__device__ inline void stage_line(const KuArgs& a, T* lds, int64_t j0, T beta) {
   const int L = BS + 2 * a.ny + 2;
   const int64_t base = j0 - a.ny - 1;
-  const bool zin = pz >= 0 && pz < a.nz;
   for (int t = threadIdx.x; t < L * NDPN; t += BS) {
     const int64_t jj = base + t / NDPN;
     T v = T(0);
-    if (zin && jj >= 0 && jj < a.plane)
-      v = stage_val<T>(a, (int64_t(pz) * a.plane + jj) * NDPN + (t % NDPN), fusep, beta);
+    if (jj >= 0 && jj < a.plane) {
+      // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
+      const int ix = int(uint32_t(jj) / uint32_t(a.ny));
+      v = stage_val<NDPN, T, TB, SRC>(a, ix, int(jj) - ix * a.ny, t % NDPN, beta);
+    }
     lds[t] = v;
   }
 }
@@ -588,7 +607,7 @@ __global__ __launch_bounds__(BS) void ku3d_kernel(KuArgs a) {
 }
 
 // lds: (BS + 2 ny + 2) * NDPN values of T
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool FAST>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds) {
   if (a.done && *a.done) return;
   const int64_t j0 = int64_t(bid) * BS;
@@ -601,8 +620,8 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
   T S[3][4];
   __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
-  if constexpr (FUSEP) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
-  stage_plane<NDPN, T>(a, lds, 0, j0, FUSEP, beta);
+  if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
+  stage_line<NDPN, T, TB, SRC>(a, lds, j0, beta);
   // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
   {
     const T* sp = static_cast<const T*>(a.sp);
@@ -621,7 +640,7 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
     T uc[NDPN];
 #pragma unroll
     for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
-    if constexpr (FUSEP) {
+    if constexpr (SRC == SRC_P) {
 #pragma unroll
       for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
     }
@@ -634,10 +653,10 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
   }
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool FAST>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 __global__ __launch_bounds__(BS) void ku2d_kernel(KuArgs a) {
   extern __shared__ double lds_raw[];
-  ku2d_body<NDPN, T, MODE, TB, TO, FUSEP, FAST>(a, blockIdx.x, reinterpret_cast<T*>(lds_raw));
+  ku2d_body<NDPN, T, MODE, TB, TO, SRC, FAST>(a, blockIdx.x, reinterpret_cast<T*>(lds_raw));
 }
 
 static int launch_fold(tl_problem* P, unsigned nb, int fin, double* out, const int* done);
@@ -652,7 +671,7 @@ template <int TY>
 constexpr int ku2t_halo_nodes() { return (BS / TY + 2) * (TY + 2); }
 
 // lds: ku2t_halo_nodes<TY>() * NDPN values of T
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, int TY>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int TY>
 __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds) {
   if (a.done && *a.done) return;
   constexpr int TX = BS / TY;
@@ -665,13 +684,13 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
   const bool active = ix < a.nx && iy < a.ny;
   __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
-  if constexpr (FUSEP) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
+  if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
   for (int t = threadIdx.x; t < HN * NDPN; t += BS) {
     const int h = t / NDPN, c = t % NDPN;
     const int hx = x0 - 1 + h / HY, hy = y0 - 1 + h % HY;
     T v = T(0);
     if (hx >= 0 && hx < a.nx && hy >= 0 && hy < a.ny)
-      v = stage_val<T>(a, (int64_t(hx) * a.ny + hy) * NDPN + c, FUSEP, beta);
+      v = stage_val<NDPN, T, TB, SRC>(a, hx, hy, c, beta);
     lds[t] = v;
   }
   T U[3][9][NDPN];
@@ -702,7 +721,7 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
     T uc[NDPN];
 #pragma unroll
     for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
-    if constexpr (FUSEP) {
+    if constexpr (SRC == SRC_P) {
 #pragma unroll
       for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
     }
@@ -715,10 +734,10 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
   }
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, int TY>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int TY>
 __global__ __launch_bounds__(BS) void ku2t_kernel(KuArgs a) {
   __shared__ T lds[ku2t_halo_nodes<TY>() * NDPN];
-  ku2t_body<NDPN, T, MODE, TB, TO, FUSEP, TY>(a, blockIdx.x, lds);
+  ku2t_body<NDPN, T, MODE, TB, TO, SRC, TY>(a, blockIdx.x, lds);
 }
 
 // Multi-instance form of the 2D operator for lockstep batched solves (see
@@ -726,7 +745,7 @@ __global__ __launch_bounds__(BS) void ku2t_kernel(KuArgs a) {
 // that system's workgroup shape (node line or 16/32/64-high tile), so one
 // launch serves systems whatever shape their autotuning chose.  All shapes
 // stage into one dynamic LDS buffer, sized for the largest among the systems.
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool FAST>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 __global__ __launch_bounds__(BS) void ku2_multi_kernel(const KuArgs* __restrict__ descs,
                                                        const uint2* __restrict__ tiles) {
   extern __shared__ double lds_raw[];
@@ -735,19 +754,19 @@ __global__ __launch_bounds__(BS) void ku2_multi_kernel(const KuArgs* __restrict_
   const KuArgs& a = descs[t.x];
   if constexpr (NDPN <= 2 && FAST) {
     switch (a.ty) {
-      case 16: ku2t_body<NDPN, T, MODE, TB, TO, FUSEP, 16>(a, t.y, lds); return;
-      case 32: ku2t_body<NDPN, T, MODE, TB, TO, FUSEP, 32>(a, t.y, lds); return;
-      case 64: ku2t_body<NDPN, T, MODE, TB, TO, FUSEP, 64>(a, t.y, lds); return;
+      case 16: ku2t_body<NDPN, T, MODE, TB, TO, SRC, 16>(a, t.y, lds); return;
+      case 32: ku2t_body<NDPN, T, MODE, TB, TO, SRC, 32>(a, t.y, lds); return;
+      case 64: ku2t_body<NDPN, T, MODE, TB, TO, SRC, 64>(a, t.y, lds); return;
       default: break;
     }
   }
-  ku2d_body<NDPN, T, MODE, TB, TO, FUSEP, FAST>(a, t.y, lds);
+  ku2d_body<NDPN, T, MODE, TB, TO, SRC, FAST>(a, t.y, lds);
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool FAST>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 static int ku2_multi_launch(hipStream_t s, const void* descs, const uint2* tiles, unsigned nb,
                             size_t lds) {
-  hipLaunchKernelGGL((ku2_multi_kernel<NDPN, T, MODE, TB, TO, FUSEP, FAST>), dim3(nb), dim3(BS),
+  hipLaunchKernelGGL((ku2_multi_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nb), dim3(BS),
                      lds, s, static_cast<const KuArgs*>(descs), tiles);
   TL_CHECK_LAUNCH();
   return TL_OK;
@@ -779,7 +798,13 @@ static int resident_slots(const void* kernel, size_t lds, int64_t& slots) {
   return TL_OK;
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, int TY>
+// 2D workgroup shape by rule: the 8 x 32 node tile from 64 nodes in y on (the
+// line's halo of 2 ny + 2 nodes then reaches half of what it computes; below,
+// both take the launch latency).  FP64 products: 1536x512 elasticity 16.1 (line)
+// and 8.7 us (tile), 448x224 3.8 and 3.2, 300x100 3.4 and 2.9, 150x50 both 2.8.
+static int default_tile2d(const Grid& g) { return g.ny >= 64 ? 32 : 0; }
+
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int TY>
 static int launch_ku2t(const tl_problem* P, const KuArgs& a) {
   constexpr int TX = BS / TY;
   const int64_t nb = int64_t((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
@@ -790,10 +815,10 @@ static int launch_ku2t(const tl_problem* P, const KuArgs& a) {
   if (P->rec) {
     KuArgs ar = a;
     ar.ty = TY;
-    P->rec->add(P->rec_phase, P->rec_level, &ku2_multi_launch<NDPN, T, MODE, TB, TO, FUSEP, true>,
+    P->rec->add(P->rec_phase, P->rec_level, &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, true>,
                 ar, unsigned(nb), size_t(ku2t_halo_nodes<TY>()) * NDPN * sizeof(T));
   } else {
-    hipLaunchKernelGGL((ku2t_kernel<NDPN, T, MODE, TB, TO, FUSEP, TY>), dim3(unsigned(nb)),
+    hipLaunchKernelGGL((ku2t_kernel<NDPN, T, MODE, TB, TO, SRC, TY>), dim3(unsigned(nb)),
                        dim3(BS), 0, P->stream, a);
     TL_CHECK_LAUNCH();
   }
@@ -802,7 +827,7 @@ static int launch_ku2t(const tl_problem* P, const KuArgs& a) {
   return TL_OK;
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP, bool FAST>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 static int launch_ku_impl(const tl_problem* P, KuArgs a) {
 
   const Grid& g = P->g;
@@ -818,8 +843,8 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
     // p = z + beta p is a separate pass before the 3D product (the fused
     // form needed a second copy stream and an in-LDS combine and was
     // slower: 96 vs 64 + 19 us per product at 192x96x96)
-    if constexpr (FUSEP) {
-      set_error("internal: the 3D operator has no fused search-direction update");
+    if constexpr (SRC != SRC_U) {
+      set_error("internal: the general 3D operator stages its input as it is");
       return TL_EINVAL;
     } else {
     // one workgroup per resident slot, at least 4 planes each
@@ -851,10 +876,17 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
   } else {
     a.ncol = 0;
     if constexpr (NDPN <= 2 && FAST) {
-      switch (P->op.tile2d[sizeof(T) == 8 ? 0 : 1]) {
-        case 16: return launch_ku2t<NDPN, T, MODE, TB, TO, FUSEP, 16>(P, a);
-        case 32: return launch_ku2t<NDPN, T, MODE, TB, TO, FUSEP, 32>(P, a);
-        case 64: return launch_ku2t<NDPN, T, MODE, TB, TO, FUSEP, 64>(P, a);
+      int ty = P->op.tile2d[sizeof(T) == 8 ? 0 : 1];
+      if (ty < 0) {
+        ty = default_tile2d(g);
+        // tiles round the grid up: a reduction that fits the slots as lines may not
+        const int64_t nt = int64_t((g.nx + 7) / 8) * ((g.ny + 31) / 32);
+        if ((MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) && nt > kMaxRedBlocks) ty = 0;
+      }
+      switch (ty) {
+        case 16: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 16>(P, a);
+        case 32: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 32>(P, a);
+        case 64: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 64>(P, a);
         default: break;
       }
     }
@@ -866,10 +898,10 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
       KuArgs ar = a;
       ar.ty = 0;
       P->rec->add(P->rec_phase, P->rec_level,
-                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, FUSEP, FAST>, ar, nbx,
+                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, FAST>, ar, nbx,
                   size_t(L) * NDPN * sizeof(T));
     } else {
-      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, FUSEP, FAST>), dim3(nbx), dim3(BS),
+      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nbx), dim3(BS),
                          size_t(L) * NDPN * sizeof(T), P->stream, a);
     }
     if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
@@ -881,34 +913,43 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
   return TL_OK;
 }
 
-template <int NDPN, typename T, int MODE, typename TB, typename TO, bool FUSEP>
+template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC>
 static int launch_ku(const tl_problem* P, KuArgs a) {
-  if (P->op.fast_ke) return launch_ku_impl<NDPN, T, MODE, TB, TO, FUSEP, true>(P, a);
-  return launch_ku_impl<NDPN, T, MODE, TB, TO, FUSEP, false>(P, a);
+  if (P->op.fast_ke) return launch_ku_impl<NDPN, T, MODE, TB, TO, SRC, true>(P, a);
+  return launch_ku_impl<NDPN, T, MODE, TB, TO, SRC, false>(P, a);
 }
 
 template <int NDPN, typename T>
 static int dispatch_mode(const tl_problem* P, const KuArgs& a, int mode, bool fusep, bool b64,
                          bool out64) {
-  // (mode, fusep, b type, out type) combinations used by the solver
+  // (mode, source, b type, out type) combinations used by the solver
+  if (!a.u) {  // V(1,1) cycles: the first sweep on the fly, the correction in the last one
+    if constexpr (NDPN <= 2) {
+      if (mode == KU_RESID) return launch_ku<NDPN, T, KU_RESID, double, T, SRC_SEED>(P, a);
+      if (mode == KU_JACOBI_DOT)
+        return launch_ku<NDPN, T, KU_JACOBI_DOT, double, double, SRC_SEED_CORR>(P, a);
+    }
+    set_error("internal: unsupported operator source");
+    return TL_EINVAL;
+  }
   if (mode == KU_STORE) {
-    if (out64) return launch_ku<NDPN, T, KU_STORE, double, double, false>(P, a);
-    return launch_ku<NDPN, T, KU_STORE, T, T, false>(P, a);
+    if (out64) return launch_ku<NDPN, T, KU_STORE, double, double, SRC_U>(P, a);
+    return launch_ku<NDPN, T, KU_STORE, T, T, SRC_U>(P, a);
   }
   if (mode == KU_STORE_DOT) {
-    if (fusep) return launch_ku<NDPN, T, KU_STORE_DOT, T, T, true>(P, a);
-    return launch_ku<NDPN, T, KU_STORE_DOT, T, T, false>(P, a);
+    if (fusep) return launch_ku<NDPN, T, KU_STORE_DOT, T, T, SRC_P>(P, a);
+    return launch_ku<NDPN, T, KU_STORE_DOT, T, T, SRC_U>(P, a);
   }
   if (mode == KU_RESID) {
-    if (b64) return launch_ku<NDPN, T, KU_RESID, double, T, false>(P, a);
-    return launch_ku<NDPN, T, KU_RESID, T, T, false>(P, a);
+    if (b64) return launch_ku<NDPN, T, KU_RESID, double, T, SRC_U>(P, a);
+    return launch_ku<NDPN, T, KU_RESID, T, T, SRC_U>(P, a);
   }
   if (mode == KU_JACOBI) {
-    if (b64) return launch_ku<NDPN, T, KU_JACOBI, double, T, false>(P, a);
-    return launch_ku<NDPN, T, KU_JACOBI, T, T, false>(P, a);
+    if (b64) return launch_ku<NDPN, T, KU_JACOBI, double, T, SRC_U>(P, a);
+    return launch_ku<NDPN, T, KU_JACOBI, T, T, SRC_U>(P, a);
   }
   if (mode == KU_JACOBI_DOT) {
-    if (b64) return launch_ku<NDPN, T, KU_JACOBI_DOT, double, double, false>(P, a);
+    if (b64) return launch_ku<NDPN, T, KU_JACOBI_DOT, double, double, SRC_U>(P, a);
   }
   set_error("unsupported operator mode");
   return TL_EINVAL;
@@ -940,6 +981,12 @@ int fine_apply_ex(tl_problem* P, const void* u, void* y, int prec, int mode, con
   a.st = P->state.as<PcgState>();
   a.fin = fin;
   a.done = done;
+  if (!u) {  // seed (and correction) formed inside the operator (mg_seeds_x0)
+    a.dinv = prec == TL_PREC_FP64 ? P->op.dinv64.ptr : P->op.dinv32.ptr;
+    a.omega = P->mg.omega;
+    a.xc = P->mg.lv[1].vx.ptr;
+    a.cny = P->mg.lv[1].g.ny;
+  }
   if (zfuse_pin && P->rho_nb) a.rho = {fin_partials(P, FIN_RHO), P->rho_nb, a.st};
   for (int g = 0; g < 8; ++g) {
     a.kv64[g] = P->op.kv[g];
@@ -1900,7 +1947,7 @@ int tl_autotune(tl_problem* P, int32_t reps, int32_t* tile_out, double* us_out) 
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc != TL_OK) {
-    P->op.tile2d[0] = P->op.tile2d[1] = 0;
+    P->op.tile2d[0] = P->op.tile2d[1] = -1;
     return rc;
   }
   {

@@ -239,8 +239,9 @@ struct FineOp {
   bool sym = false;            // 3D: the tiled reflection-symmetric operator applies (tl_sym.hip)
   double symkv[16] = {};       // its group values
   // 2D operator workgroup shape per precision [fp64, fp32]: 0 = node line
-  // (BS consecutive nodes), TY = 16/32/64: (BS/TY) x TY node tile
-  int tile2d[2] = {0, 0};
+  // (BS consecutive nodes), TY = 16/32/64: (BS/TY) x TY node tile; -1: by rule
+  // (default_tile2d)
+  int tile2d[2] = {-1, -1};
   // FP64 3D elasticity operator: true = MFMA column walk, false = vector FMAs
   bool mfma64 = false;
 };
@@ -335,8 +336,9 @@ int fine_diag(tl_problem* P);
 int prof_begin(tl_problem* P, int kind, ProfEvent& ev);
 int prof_end(tl_problem* P, ProfEvent& ev);
 // Whether the V-cycle forms its fine level's first (zero-guess) sweep, and the
-// iterate after the coarse correction, inside its two tiled operator calls:
-// no fine iterate is stored.  3D V(1,1) cycles in FP64 or FP32.
+// iterate after the coarse correction, inside its two operator calls:
+// no fine iterate is stored.  V(1,1) cycles in FP64 or FP32, in 2D and on the
+// tiled 3D operators.
 bool mg_seeds_x0(const tl_problem* P);
 // x0_ready: the fine level's first (zero-guess) smoothing sweep is already
 // in lv[0].vx (written by the PCG's residual update, see pcg_fuses_x0)
@@ -369,6 +371,17 @@ template <typename T, typename TB>
 __device__ inline T zero_guess_sweep(T omega, T dinv, TB b) {
   return omega * dinv * T(b);
 }
+
+// What a matrix-free operator stages as its input x:
+enum {
+  SRC_U = 0,          // u
+  SRC_P = 1,          // z + beta p, the new search direction (written out for the own nodes)
+  SRC_SEED = 2,       // omega D^-1 b, the first sweep from a zero guess
+  SRC_CORR = 3,       // u + (P xc) on the free DOFs: the iterate after the coarse correction
+  SRC_SEED_CORR = 4,  // omega D^-1 b + (P xc)
+};
+constexpr bool src_seed(int s) { return s == SRC_SEED || s == SRC_SEED_CORR; }
+constexpr bool src_corr(int s) { return s == SRC_CORR || s == SRC_SEED_CORR; }
 
 // modes of the fine matrix-free operator epilogue
 enum {

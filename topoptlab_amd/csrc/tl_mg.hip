@@ -1667,7 +1667,7 @@ int vcycle_fine(tl_problem* P, const double* r, double* z, const int* done, bool
   // the coarse correction (one pass over each instead of a stored iterate that
   // the PCG update writes, the residual reads, the prolongation rewrites and
   // the sweep reads again: 87 MB less in the update, 87 MB and a launch of 33 us
-  // less for the prolongation at 192x96x96)
+  // less for the prolongation at 192x96x96; a launch less in 2D)
   const bool seed = x0_ready && mg_seeds_x0(P);
   // fine-level operator: fp64, fp32, or MFMA with bf16/fp16 inputs (fp32 vectors)
   const int prec = std::is_same<T, double>::value
@@ -1719,7 +1719,7 @@ int vcycle_fine(tl_problem* P, const double* r, double* z, const int* done, bool
 
 bool mg_seeds_x0(const tl_problem* P) {
   const MgState& M = P->mg;
-  return P->op.sym && !P->op.mfma64 && M.nu1 == 1 && M.nu2 == 1 &&
+  return (P->g.dim == 2 || (P->op.sym && !P->op.mfma64)) && M.nu1 == 1 && M.nu2 == 1 &&
          (M.prec == TL_PREC_FP64 || M.prec == TL_PREC_FP32);
 }
 

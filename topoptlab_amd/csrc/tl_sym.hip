@@ -43,16 +43,6 @@ constexpr int TN = TE - 1;   // nodes produced per tile side
 constexpr int TS = TE + 1;   // nodes staged per tile side
 static_assert(TE * TE == BS, "one element column per thread");
 
-// What a staged node value is (the operator's input x):
-enum {
-  SRC_U = 0,          // u
-  SRC_P = 1,          // z + beta p, the new search direction (written out for the own nodes)
-  SRC_SEED = 2,       // omega D^-1 b, the first sweep from a zero guess
-  SRC_CORR = 3,       // u + (P xc) on the free DOFs: the iterate after the coarse correction
-  SRC_SEED_CORR = 4,  // omega D^-1 b + (P xc)
-};
-constexpr bool src_seed(int s) { return s == SRC_SEED || s == SRC_SEED_CORR; }
-constexpr bool src_corr(int s) { return s == SRC_CORR || s == SRC_SEED_CORR; }
 constexpr int TC = 10;  // coarse nodes per tile side that 17 staged nodes interpolate from
 constexpr int CR = 4;   // coarse tiles kept in LDS
 
