@@ -48,7 +48,7 @@ void DevBuf::release() {
 
 constexpr int BS = 256;  // threads per workgroup of the vector/stencil kernels
 
-enum { FIN_STORE = 0, FIN_RHO = 1, FIN_PQ = 2, FIN_RR = 3, FIN_BB = 4, FIN_RR0 = 5 };
+enum { FIN_STORE = 0, FIN_RHO = 1, FIN_PQ = 2, FIN_RR = 3, FIN_BB = 4, FIN_RR0 = 5, FIN_RRC = 6 };
 
 __device__ inline void finalize(int fin, PcgState* st, double tot, double* out) {
   switch (fin) {
@@ -67,6 +67,10 @@ __device__ inline void finalize(int fin, PcgState* st, double tot, double* out) 
       st->rr = tot;
       st->rho_prev = st->rho;
       st->it += 1;
+      st->done = (tot < st->tol2 || st->it >= st->maxiter) ? 1 : 0;
+      break;
+    case FIN_RRC:  // the x/r update has counted the iteration
+      st->rr = tot;
       st->done = (tot < st->tol2 || st->it >= st->maxiter) ? 1 : 0;
       break;
     case FIN_BB:
@@ -116,6 +120,7 @@ struct KuArgs {
   void* pout;           // SRC_P: new p (T)
   const double* beta;   // SRC_P: device scalar, or the partials of rho
   FoldIn rho;
+  FoldIn rr;            // SRC_SEED: partials of r.r of the iteration before, or none
   const void* xc;       // SRC_SEED_CORR: the coarse level's correction (T)
   int cny;              // and its node count in y
   const void* sp;       // padded scale (T)
@@ -132,6 +137,7 @@ struct KuArgs {
   const int* done;
   int nelx, nely, nelz, nx, ny, nz, plane, ncol;  // ncol: 3D tile columns
   int ty;  // 2D workgroup shape the launch uses (0: node line), for the multi-instance form
+  unsigned nblk;  // 2D: workgroups (each takes tiles bid, bid + nblk, ...)
   // group values of a pattern-matched element matrix (see ke_pattern.hpp)
   double kv64[8];
   float kv32[8];
@@ -610,41 +616,47 @@ __global__ __launch_bounds__(BS) void ku3d_kernel(KuArgs a) {
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds) {
   if (a.done && *a.done) return;
-  const int64_t j0 = int64_t(bid) * BS;
-  const int64_t j = j0 + threadIdx.x;
-  const bool active = j < a.plane;
-  const int64_t jc = active ? j : a.plane - 1;
-  // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
-  const int ix = int(uint32_t(jc) / uint32_t(a.ny)), iy = int(jc) - ix * a.ny;
-  T U[3][9][NDPN];
-  T S[3][4];
   __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
   if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
-  stage_line<NDPN, T, TB, SRC>(a, lds, j0, beta);
-  // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
-  {
-    const T* sp = static_cast<const T*>(a.sp);
-#pragma unroll
-    for (int ox = -1; ox <= 0; ++ox)
-#pragma unroll
-      for (int oy = -1; oy <= 0; ++oy)
-        S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(ix + ox + 1) * (a.nely + 2) + iy + oy + 1];
-  }
-  __syncthreads();
-  read_nbrs<NDPN, T, 1>(a, lds, U);
-  T acc[NDPN];
-  node_sum<NDPN, T, 0, 1, 2, false, FAST>(a, U, S, 0, 1, acc);
+  if constexpr (SRC == SRC_SEED)
+    if (a.rr.partials && fold_in_done(a.rr, bid == 0 && threadIdx.x == 0, sh)) return;
   double dot = 0.0;
-  if (active) {
-    T uc[NDPN];
+  const unsigned nline = unsigned((int64_t(a.plane) + BS - 1) / BS);
+  for (unsigned tile = bid; tile < nline; tile += a.nblk) {
+    if (tile != bid) __syncthreads();  // the previous tile has been read
+    const int64_t j0 = int64_t(tile) * BS;
+    const int64_t j = j0 + threadIdx.x;
+    const bool active = j < a.plane;
+    const int64_t jc = active ? j : a.plane - 1;
+    // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
+    const int ix = int(uint32_t(jc) / uint32_t(a.ny)), iy = int(jc) - ix * a.ny;
+    T U[3][9][NDPN];
+    T S[3][4];
+    stage_line<NDPN, T, TB, SRC>(a, lds, j0, beta);
+    // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
+    {
+      const T* sp = static_cast<const T*>(a.sp);
 #pragma unroll
-    for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
-    if constexpr (SRC == SRC_P) {
+      for (int ox = -1; ox <= 0; ++ox)
 #pragma unroll
-      for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
+        for (int oy = -1; oy <= 0; ++oy)
+          S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(ix + ox + 1) * (a.nely + 2) + iy + oy + 1];
     }
-    ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
+    __syncthreads();
+    read_nbrs<NDPN, T, 1>(a, lds, U);
+    T acc[NDPN];
+    node_sum<NDPN, T, 0, 1, 2, false, FAST>(a, U, S, 0, 1, acc);
+    if (active) {
+      T uc[NDPN];
+#pragma unroll
+      for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
+      if constexpr (SRC == SRC_P) {
+#pragma unroll
+        for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
+      }
+      ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
+    }
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
     double v[1] = {dot};
@@ -678,54 +690,60 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
   constexpr int HY = TY + 2, HN = (TX + 2) * HY;
   static_assert(TX * TY == BS, "tile must hold BS nodes");
   const int ntx = (a.nx + TX - 1) / TX;
-  const int x0 = int(bid % unsigned(ntx)) * TX, y0 = int(bid / unsigned(ntx)) * TY;
+  const unsigned ntile = unsigned(ntx) * unsigned((a.ny + TY - 1) / TY);
   const int lx = threadIdx.x / TY, ly = threadIdx.x % TY;
-  const int ix = x0 + lx, iy = y0 + ly;
-  const bool active = ix < a.nx && iy < a.ny;
   __shared__ double sh[BS / 64 + 2];
   T beta = T(0);
   if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
-  for (int t = threadIdx.x; t < HN * NDPN; t += BS) {
-    const int h = t / NDPN, c = t % NDPN;
-    const int hx = x0 - 1 + h / HY, hy = y0 - 1 + h % HY;
-    T v = T(0);
-    if (hx >= 0 && hx < a.nx && hy >= 0 && hy < a.ny)
-      v = stage_val<NDPN, T, TB, SRC>(a, hx, hy, c, beta);
-    lds[t] = v;
-  }
-  T U[3][9][NDPN];
-  T S[3][4];
-  {
-    // padded scale: (nelx+2) rows of (nely+2); inactive threads read node 0's
-    const T* sp = static_cast<const T*>(a.sp);
-    const int cx = active ? ix : 0, cy = active ? iy : 0;
-#pragma unroll
-    for (int ox = -1; ox <= 0; ++ox)
-#pragma unroll
-      for (int oy = -1; oy <= 0; ++oy)
-        S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(cx + ox + 1) * (a.nely + 2) + cy + oy + 1];
-  }
-  __syncthreads();
-#pragma unroll
-  for (int dx = -1; dx <= 1; ++dx)
-#pragma unroll
-    for (int dy = -1; dy <= 1; ++dy)
-#pragma unroll
-      for (int c = 0; c < NDPN; ++c)
-        U[1][(dx + 1) * 3 + (dy + 1)][c] = lds[((lx + 1 + dx) * HY + ly + 1 + dy) * NDPN + c];
-  T acc[NDPN];
-  node_sum<NDPN, T, 0, 1, 2, false, true>(a, U, S, 0, 1, acc);
+  if constexpr (SRC == SRC_SEED)
+    if (a.rr.partials && fold_in_done(a.rr, bid == 0 && threadIdx.x == 0, sh)) return;
   double dot = 0.0;
-  if (active) {
-    const int64_t j = int64_t(ix) * a.ny + iy;
-    T uc[NDPN];
-#pragma unroll
-    for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
-    if constexpr (SRC == SRC_P) {
-#pragma unroll
-      for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
+  for (unsigned tile = bid; tile < ntile; tile += a.nblk) {
+    if (tile != bid) __syncthreads();  // the previous tile has been read
+    const int x0 = int(tile % unsigned(ntx)) * TX, y0 = int(tile / unsigned(ntx)) * TY;
+    const int ix = x0 + lx, iy = y0 + ly;
+    const bool active = ix < a.nx && iy < a.ny;
+    for (int t = threadIdx.x; t < HN * NDPN; t += BS) {
+      const int h = t / NDPN, c = t % NDPN;
+      const int hx = x0 - 1 + h / HY, hy = y0 - 1 + h % HY;
+      T v = T(0);
+      if (hx >= 0 && hx < a.nx && hy >= 0 && hy < a.ny)
+        v = stage_val<NDPN, T, TB, SRC>(a, hx, hy, c, beta);
+      lds[t] = v;
     }
-    ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
+    T U[3][9][NDPN];
+    T S[3][4];
+    {
+      // padded scale: (nelx+2) rows of (nely+2); inactive threads read node 0's
+      const T* sp = static_cast<const T*>(a.sp);
+      const int cx = active ? ix : 0, cy = active ? iy : 0;
+#pragma unroll
+      for (int ox = -1; ox <= 0; ++ox)
+#pragma unroll
+        for (int oy = -1; oy <= 0; ++oy)
+          S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(cx + ox + 1) * (a.nely + 2) + cy + oy + 1];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int dx = -1; dx <= 1; ++dx)
+#pragma unroll
+      for (int dy = -1; dy <= 1; ++dy)
+#pragma unroll
+        for (int c = 0; c < NDPN; ++c)
+          U[1][(dx + 1) * 3 + (dy + 1)][c] = lds[((lx + 1 + dx) * HY + ly + 1 + dy) * NDPN + c];
+    T acc[NDPN];
+    node_sum<NDPN, T, 0, 1, 2, false, true>(a, U, S, 0, 1, acc);
+    if (active) {
+      const int64_t j = int64_t(ix) * a.ny + iy;
+      T uc[NDPN];
+#pragma unroll
+      for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
+      if constexpr (SRC == SRC_P) {
+#pragma unroll
+        for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
+      }
+      ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
+    }
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
     double v[1] = {dot};
@@ -804,14 +822,28 @@ static int resident_slots(const void* kernel, size_t lds, int64_t& slots) {
 // and 8.7 us (tile), 448x224 3.8 and 3.2, 300x100 3.4 and 2.9, 150x50 both 2.8.
 static int default_tile2d(const Grid& g) { return g.ny >= 64 ? 32 : 0; }
 
+// Workgroups of a 2D operator call over `tiles` tiles.  Where a scalar is
+// folded before or after it (dot products, the seeded residual) a workgroup
+// takes several tiles, evenly, so that the partials stay within what a
+// consumer folds itself; otherwise one each.
+template <int MODE, int SRC>
+static int64_t ku2_groups(int64_t tiles) {
+  if (MODE != KU_STORE_DOT && MODE != KU_JACOBI_DOT && SRC != SRC_SEED) return tiles;
+  const int64_t per = (tiles + kFoldInBlocks - 1) / kFoldInBlocks;
+  return (tiles + per - 1) / per;
+}
+
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int TY>
-static int launch_ku2t(const tl_problem* P, const KuArgs& a) {
+static int launch_ku2t(const tl_problem* P, KuArgs a) {
   constexpr int TX = BS / TY;
-  const int64_t nb = int64_t((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
-  if (nb > kMaxRedBlocks && (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT)) {
+  const int64_t tiles = int64_t((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
+  if (tiles > kMaxRedBlocks && P->op.tile2d[sizeof(T) == 8 ? 0 : 1] == TY &&
+      (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT)) {
     set_error("fine operator grid exceeds the reduction slot count");
     return TL_EINVAL;
   }
+  const int64_t nb = ku2_groups<MODE, SRC>(tiles);
+  a.nblk = unsigned(nb);
   if (P->rec) {
     KuArgs ar = a;
     ar.ty = TY;
@@ -879,9 +911,7 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
       int ty = P->op.tile2d[sizeof(T) == 8 ? 0 : 1];
       if (ty < 0) {
         ty = default_tile2d(g);
-        // tiles round the grid up: a reduction that fits the slots as lines may not
-        const int64_t nt = int64_t((g.nx + 7) / 8) * ((g.ny + 31) / 32);
-        if ((MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) && nt > kMaxRedBlocks) ty = 0;
+        if ((MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) && nbx > unsigned(kMaxRedBlocks)) ty = 0;
       }
       switch (ty) {
         case 16: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 16>(P, a);
@@ -894,19 +924,21 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
       set_error("fine operator grid exceeds the reduction slot count");
       return TL_EINVAL;
     }
+    const unsigned nb = unsigned(ku2_groups<MODE, SRC>(nbx));
+    a.nblk = nb;
     if (P->rec) {
       KuArgs ar = a;
       ar.ty = 0;
       P->rec->add(P->rec_phase, P->rec_level,
-                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, FAST>, ar, nbx,
+                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, FAST>, ar, nb,
                   size_t(L) * NDPN * sizeof(T));
     } else {
-      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nbx), dim3(BS),
+      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nb), dim3(BS),
                          size_t(L) * NDPN * sizeof(T), P->stream, a);
     }
     if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
       TL_CHECK_LAUNCH();
-      return launch_fold(const_cast<tl_problem*>(P), nbx, a.fin, a.dot_out, a.done);
+      return launch_fold(const_cast<tl_problem*>(P), nb, a.fin, a.dot_out, a.done);
     }
   }
   TL_CHECK_LAUNCH();
@@ -962,7 +994,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
 // because a consumer may still fold one while the next is written.
 static double* fin_partials(tl_problem* P, int fin) {
   double* p = P->partials.as<double>();
-  return fin == FIN_PQ ? p + kMaxRedBlocks : (fin == FIN_RR ? p + 2 * kMaxRedBlocks : p);
+  return fin == FIN_PQ ? p + kMaxRedBlocks : (fin == FIN_RR || fin == FIN_RRC ? p + 2 * kMaxRedBlocks : p);
 }
 
 // Generic entry used by the solver and the V-cycle.  prec selects T; b is
@@ -987,6 +1019,7 @@ int fine_apply_ex(tl_problem* P, const void* u, void* y, int prec, int mode, con
     a.xc = P->mg.lv[1].vx.ptr;
     a.cny = P->mg.lv[1].g.ny;
   }
+  if (!u && mode == KU_RESID && P->rr_nb) a.rr = {fin_partials(P, FIN_RR), P->rr_nb, a.st};
   if (zfuse_pin && P->rho_nb) a.rho = {fin_partials(P, FIN_RHO), P->rho_nb, a.st};
   for (int g = 0; g < 8; ++g) {
     a.kv64[g] = P->op.kv[g];
@@ -1039,7 +1072,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
     }
     unsigned nb = 0;
     TL_TRY(sym_fine_apply(P, a.u, a.y, prec, mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
-                          a.rho, a.partials, a.done, out64, &nb));
+                          a.rho, a.rr, a.partials, a.done, out64, &nb));
     if (mode == KU_STORE_DOT || mode == KU_JACOBI_DOT)
       return launch_fold(P, nb, a.fin, a.dot_out, a.done);
     return TL_OK;
@@ -1257,6 +1290,7 @@ struct UpdateArgs {
   const int* done;
   unsigned nb;  // blocks of the system's grid-stride loop
   FoldIn pq;    // partials of p.q, or none: alpha is in the state
+  PcgState* count;  // counts the iteration (r.r is folded by the next residual), or null
 };
 
 template <typename TS>
@@ -1264,6 +1298,10 @@ __device__ __forceinline__ void update_body(const UpdateArgs<TS>& a, unsigned bi
   if (*a.done) return;
   __shared__ double sh[BS / 64 + 4];
   const double alpha = fold_in_alpha(a.pq, a.st, sh);
+  if (a.count && bid == 0 && threadIdx.x == 0) {  // fields no workgroup reads here
+    a.count->it += 1;
+    a.count->rho_prev = a.count->rho;
+  }
   double s = 0.0;
   for (int64_t i = bid * int64_t(BS) + threadIdx.x; i < a.n; i += int64_t(a.nb) * BS) {
     const double xv = __builtin_nontemporal_load(&a.x[i]) + alpha * __builtin_nontemporal_load(&a.p[i]);
@@ -1627,6 +1665,7 @@ struct PcgCtx {
 
 int pcg_context(tl_problem* P, PcgCtx& c) {
   const int64_t n = P->ndof;
+  P->rho_nb = P->pq_nb = P->rr_nb = 0;
   for (DevBuf* b : {&P->r, &P->z, &P->p, &P->p2, &P->q, &P->t}) TL_TRY(b->alloc(sizeof(double) * n));
   c.n = n;
   c.r = P->r.as<double>(); c.z = P->z.as<double>(); c.q = P->q.as<double>(); c.t = P->t.as<double>();
@@ -1751,13 +1790,17 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
   FoldIn pq;
   if (P->pq_nb) pq = {fin_partials(P, FIN_PQ), P->pq_nb, c.st};
   double* rrp = fin_partials(P, FIN_RR);
+  // seeded cycles: the next residual folds r.r and ends the solve (a lockstep
+  // batch folds all of its systems in one launch instead)
+  const bool lazy = fx0 && mg_seeds_x0(P) && !P->rec;
+  const unsigned ub = lazy ? std::min(c.rb, kFoldInBlocks) : c.rb;
   auto upd = [&](auto ua) -> int {
     using TS = std::remove_pointer_t<decltype(ua.xs)>;
     if (P->rec) {
-      P->rec->add(2, 0, &update_multi_launch<TS>, ua, c.rb, 0);
+      P->rec->add(2, 0, &update_multi_launch<TS>, ua, ub, 0);
       return TL_OK;
     }
-    hipLaunchKernelGGL(update_kernel<TS>, dim3(c.rb), dim3(BS), 0, s, ua);
+    hipLaunchKernelGGL(update_kernel<TS>, dim3(ub), dim3(BS), 0, s, ua);
     TL_CHECK_LAUNCH();
     return TL_OK;
   };
@@ -1765,15 +1808,25 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
   if (xs && P->mg.prec == TL_PREC_FP64)
     TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                   P->mg.lv[0].vx.as<double>(), P->op.dinv64.as<double>(),
-                                  P->mg.omega, c.done, c.rb, pq}));
+                                  P->mg.omega, c.done, ub, pq, nullptr}));
   else if (xs)
     TL_TRY(upd(UpdateArgs<float>{x, c.r, pout, c.q, c.n, rrp, c.st,
                                  P->mg.lv[0].vx.as<float>(), P->op.dinv32.as<float>(),
-                                 float(P->mg.omega), c.done, c.rb, pq}));
+                                 float(P->mg.omega), c.done, ub, pq, nullptr}));
   else
     TL_TRY(upd(UpdateArgs<double>{x, c.r, pout, c.q, c.n, rrp, c.st, nullptr, nullptr,
-                                  0.0, c.done, c.rb, pq}));
-  return launch_fold(P, c.rb, FIN_RR, nullptr, c.done);
+                                  0.0, c.done, ub, pq, lazy ? c.st : nullptr}));
+  P->rr_nb = lazy ? ub : 0u;
+  return lazy ? int(TL_OK) : launch_fold(P, ub, FIN_RR, nullptr, c.done);
+}
+
+// End of a chunk of iterations: the state is brought up to date for the host
+// and for the next chunk's first iteration.
+int pcg_chunk_end(tl_problem* P, const PcgCtx& c) {
+  if (!P->rr_nb) return TL_OK;
+  const unsigned nb = P->rr_nb;
+  P->rr_nb = 0;
+  return launch_fold(P, nb, FIN_RRC, nullptr, c.done);
 }
 
 // True residual |t - K x|^2 into *tr2_dev (a device slot), state unchanged.
@@ -1827,6 +1880,7 @@ int tl_solve(tl_problem* P, const double* f, double* u, const tl_solve_opts* o,
   int64_t kk = 0;
   for (int launched = 0; !hs.done;) {
     for (int k = 0; k < chunk; ++k) TL_TRY(pcg_iteration(P, c, u, o->precond, kk++));
+    TL_TRY(pcg_chunk_end(P, c));
     launched += chunk;
     TL_HIP(hipMemcpyAsync(&hs, c.st, sizeof(PcgState), hipMemcpyDeviceToHost, s));
     TL_HIP(hipStreamSynchronize(s));
@@ -1982,6 +2036,7 @@ int chunk_graph(tl_problem* P, const PcgCtx& c, int precond, int chunk) {
   int rc = TL_OK;
   for (int k = 0; k < chunk && rc == TL_OK; ++k)
     rc = pcg_iteration(P, c, P->xb.as<double>(), precond, k);
+  if (rc == TL_OK) rc = pcg_chunk_end(P, c);
   hipGraph_t g = nullptr;
   const hipError_t ec = hipStreamEndCapture(s, &g);
   if (rc != TL_OK) {
@@ -2427,6 +2482,7 @@ int tl_batch_solve(int32_t n, tl_problem* const* hs, const double* const* f, dou
       TL_HIP(hipGraphLaunch(P->chunk_exec, P->stream));
     } else {
       for (int k = 0; k < chunk; ++k) TL_TRY(pcg_iteration(P, ctx[i], P->xb.as<double>(), o->precond, k));
+      TL_TRY(pcg_chunk_end(P, ctx[i]));
     }
     launched[i] += chunk;
     TL_HIP(hipMemcpyAsync(&slots[i].hs, ctx[i].st, sizeof(PcgState), hipMemcpyDeviceToHost, P->stream));

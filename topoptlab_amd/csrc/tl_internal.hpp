@@ -172,9 +172,10 @@ struct PcgState {
 
 // A PCG scalar whose block partials the consuming kernel folds itself (every
 // workgroup in the same fixed order as fold_kernel) instead of a one-block
-// kernel in between: a launch of 3.5-4.8 us less per scalar.  Beyond
+// kernel in between: a launch of 2-6 us and a gap less per scalar.  Beyond
 // kFoldInBlocks partials the reads of all workgroups together cost more than
-// the launch.  partials == nullptr: the scalar is in the state.
+// the launch.  partials == nullptr: the scalar is in the state.  No workgroup
+// reads a state field that one of the same kernel writes.
 constexpr unsigned kFoldInBlocks = 1024;
 struct FoldIn {
   const double* partials = nullptr;
@@ -199,6 +200,20 @@ __device__ __forceinline__ double fold_in_alpha(const FoldIn& f, const PcgState*
   double tot[1];
   fold_partials<1>(f.partials, f.nb, tot, sh);
   return st->rho / tot[0];
+}
+
+// r.r of the iteration before, and whether the solve has ended (the x/r update
+// has counted the iteration already, see UpdateArgs::count).  Folding the same
+// partials again changes nothing.
+__device__ __forceinline__ bool fold_in_done(const FoldIn& f, bool writer, double* sh) {
+  double tot[1];
+  fold_partials<1>(f.partials, f.nb, tot, sh);
+  const bool end = tot[0] < f.st->tol2 || f.st->it >= f.st->maxiter;
+  if (writer) {
+    f.st->rr = tot[0];
+    f.st->done = end ? 1 : 0;
+  }
+  return end;
 }
 
 struct Level {
@@ -317,8 +332,8 @@ struct tl_problem {
   hipGraphExec_t chunk_exec = nullptr;
   int64_t chunk_key[5] = {-1, -1, -1, -1, -1};
   tl::DevBuf partials, state;
-  // rho and p.q partials left for their consumer to fold (0: in the state)
-  unsigned rho_nb = 0, pq_nb = 0;
+  // rho, p.q and r.r partials left for their consumer to fold (0: in the state)
+  unsigned rho_nb = 0, pq_nb = 0, rr_nb = 0;
   // launch timing of the fine operator (tl_profile)
   bool prof_on = false;
   std::vector<tl::ProfEvent> prof_used, prof_free;
@@ -358,8 +373,8 @@ bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]);
 bool sym_fits(const Grid& g, int ndpn);
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
-                   const double* beta, const FoldIn& rho, double* partials, const int* done,
-                   bool out64, unsigned* nblocks_out);
+                   const double* beta, const FoldIn& rho, const FoldIn& rr, double* partials,
+                   const int* done, bool out64, unsigned* nblocks_out);
 int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* xc,
                      const void* b, void* y, const int* done);
 }  // namespace tl

@@ -53,6 +53,7 @@ struct SymArgs {
   T* pout;             // SRC_P: new search direction
   const double* beta;  // SRC_P: device scalar, or the partials of rho
   FoldIn rho;
+  FoldIn rr;           // SRC_SEED: partials of r.r of the iteration before, or none
   const T* xc;         // SRC_*CORR: the coarse level's correction
   int cnx, cny, cnz;   // and its node counts
   const T* sp;         // zero-bordered scales of the fine grid
@@ -530,6 +531,8 @@ __global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kerne
   unsigned u0 = __builtin_amdgcn_readfirstlane(units * w / nb);
   const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
   __shared__ double sh[BS / 64 + 2];
+  if constexpr (SRC == SRC_SEED)
+    if (a.rr.partials && fold_in_done(a.rr, blockIdx.x == 0 && threadIdx.x == 0, sh)) return;
   T beta = T(0);
   if constexpr (SRC == SRC_P)
     beta = T(fold_in_beta(a.rho, a.beta, blockIdx.x == 0 && threadIdx.x == 0, sh));
@@ -704,14 +707,15 @@ static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, boo
 template <int NDPN, typename T>
 static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void* b, bool b64,
                      const void* dinv, double omega, const void* pin, void* pout,
-                     const double* beta, const FoldIn& rho, double* partials, const int* done,
-                     bool out64, unsigned* nb) {
+                     const double* beta, const FoldIn& rho, const FoldIn& rr, double* partials,
+                     const int* done, bool out64, unsigned* nb) {
   SymArgs<T> a{};
   a.u = static_cast<const T*>(u);
   a.pin = static_cast<const T*>(pin);
   a.pout = static_cast<T*>(pout);
   a.beta = beta;
   a.rho = rho;
+  a.rr = rr;
   a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
                         : reinterpret_cast<const T*>(P->op.sp32.ptr);
   a.mask = P->op.mask.as<uint8_t>();
@@ -738,18 +742,17 @@ static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void
 
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
-                   const double* beta, const FoldIn& rho, double* partials, const int* done,
-                   bool out64, unsigned* nb) {
+                   const double* beta, const FoldIn& rho, const FoldIn& rr, double* partials,
+                   const int* done, bool out64, unsigned* nb) {
+  auto go = [&](auto ndpn, auto t) {
+    return fine_call<decltype(ndpn)::value, decltype(t)>(P, u, y, mode, b, b64, dinv, omega, pin, pout,
+                                                         beta, rho, rr, partials, done, out64, nb);
+  };
+  using N1 = std::integral_constant<int, 1>;
+  using N3 = std::integral_constant<int, 3>;
   const bool f64 = prec == TL_PREC_FP64;
-  if (P->ndpn == 3)
-    return f64 ? fine_call<3, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
-                                      partials, done, out64, nb)
-               : fine_call<3, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
-                                     partials, done, out64, nb);
-  return f64 ? fine_call<1, double>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
-                                    partials, done, out64, nb)
-             : fine_call<1, float>(P, u, y, mode, b, b64, dinv, omega, pin, pout, beta, rho,
-                                   partials, done, out64, nb);
+  if (P->ndpn == 3) return f64 ? go(N3{}, double{}) : go(N3{}, float{});
+  return f64 ? go(N1{}, double{}) : go(N1{}, float{});
 }
 
 template <int NDPN, typename T>
