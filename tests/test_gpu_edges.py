@@ -155,3 +155,11 @@ def test_oc_sizes(gpu, n, l2):
     got, ggt = oc_top88(t(x), 0.3, t(dc), t(dv), g, el_flags=t(fl), l2=l2)
     assert np.array_equal(got.cpu().numpy(), ref)
     assert abs(ggt - gt) <= 1e-12 * np.abs(dv * (ref - x)).sum() + 1e-15
+
+
+# one block, partial blocks, more elements than 1,024 blocks hold at once
+@pytest.mark.parametrize("it,n", [(0, 2), (5, 255), (0, 257), (5, 131072), (0, 300001)])
+def test_mma_sizes(gpu, it, n):
+    """MMA step against the oracle, inputs and tolerances of its parity test."""
+    from tests.test_gpu_parity import test_mma_update_matches_oracle as check
+    check(gpu, it, n)

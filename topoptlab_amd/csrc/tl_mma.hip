@@ -16,24 +16,34 @@
 //    norm decreases (at most 50 halvings, 200 Newton steps per epsi).
 //
 // Elementwise work and the global sums / maxima run on the device; the few
-// scalars of the m = 1 system (y, z, lam, mu, zet, s) live on the host,
-// which reads 3-4 reduced values per Newton step.
+// scalars of the m = 1 system (y, z, lam, mu, zet, s) live on the host, which
+// reads the folded values of two passes per Newton step (the direction, and
+// the residual of the step together with the next step's Newton sums) from
+// pinned memory as they arrive.  The round trips bound an update (about 60 of
+// them, kernels of 8-10 us at 221,184 elements); with a pass of its own for
+// the Newton sums and a stream synchronisation per pass there were 84 of 25 us.
+// (Block partials written straight to the host instead of a one-block fold:
+// each of those small writes costs about 20 ns at the end of the kernel.)
 #include "tl_internal.hpp"
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 
 namespace tl {
 namespace {
 
 constexpr int BS = 256;
-constexpr int NR = 4;  // reduced values per pass
+constexpr int NR = 5;        // reduced values per pass
+// Bits of a slot that no kernel has written yet: a NaN that arithmetic does not
+// produce (its results carry the canonical payload or an input's).
+constexpr uint64_t kEmpty = 0x7ff8a5a5c3c35a5aull;
 
 struct MmaWork {
   DevBuf vec, partials;
-  // the folded scalars, written by the fold kernel straight into pinned,
-  // coherent host memory: the host reads them after the stream synchronises,
-  // with no copy in between (one per fold, ~90 folds per update)
+  // the folded values, written by the fold kernel straight into pinned,
+  // coherent host memory; two sets in turn
   double* hout = nullptr;
   int64_t n = 0;
   int ensure(int64_t nn) {
@@ -42,7 +52,7 @@ struct MmaWork {
       n = nn;
     }
     if (!partials.ptr) TL_TRY(partials.alloc(sizeof(double) * NR * kMaxRedBlocks));
-    if (!hout) TL_HIP(hipHostMalloc(reinterpret_cast<void**>(&hout), sizeof(double) * NR,
+    if (!hout) TL_HIP(hipHostMalloc(reinterpret_cast<void**>(&hout), sizeof(double) * 2 * NR,
                                     hipHostMallocCoherent));
     return TL_OK;
   }
@@ -81,9 +91,9 @@ __device__ inline void store_red(const double (&v)[NR], double* partials) {
     for (int k = 0; k < NR; ++k) partials[k * kMaxRedBlocks + blockIdx.x] = v[k];
 }
 
+// one block: the folded values into the host's slots
 __global__ __launch_bounds__(BS) void mma_fold_kernel(const double* __restrict__ partials,
-                                                      unsigned nb, unsigned maxmask,
-                                                      double* __restrict__ out) {
+                                                      unsigned nb, unsigned maxmask, double* out) {
   __shared__ double sh[NR * (BS / 64)];
   double v[NR];
 #pragma unroll
@@ -97,9 +107,12 @@ __global__ __launch_bounds__(BS) void mma_fold_kernel(const double* __restrict__
     v[k] = r;
   }
   block_reduce(v, maxmask, sh);
-  if (threadIdx.x == 0)
+  if (threadIdx.x < NR) {
+    double r = v[0];
 #pragma unroll
-    for (int k = 0; k < NR; ++k) out[k] = v[k];
+    for (int k = 1; k < NR; ++k) r = int(threadIdx.x) == k ? v[k] : r;
+    __hip_atomic_store(&out[threadIdx.x], r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
 struct MmaVec {
@@ -114,9 +127,9 @@ __global__ __launch_bounds__(BS) void mma_prep_kernel(
     const double* __restrict__ xold2, const double* __restrict__ xmin_a,
     const double* __restrict__ xmax_a, const double* __restrict__ df0dx,
     const double* __restrict__ dfdx, double* __restrict__ low, double* __restrict__ upp, int iter,
-    tl_mma_opts o, MmaVec w, double* __restrict__ partials) {
+    tl_mma_opts o, MmaVec w, double* partials) {
   __shared__ double sh[NR * (BS / 64)];
-  double red[NR] = {0.0, 0.0, 0.0, 0.0};
+  double red[NR] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS) {
     const double xv = xval[i];
     const double xmn = xmin_a ? xmin_a[i] : 0.0, xmx = xmax_a ? xmax_a[i] : 1.0;
@@ -162,15 +175,17 @@ __global__ __launch_bounds__(BS) void mma_prep_kernel(
 }
 
 // Residual of the relaxed KKT system, vector part, at x = x0 + steg*dx (and
-// xsi, eta likewise) written to set `to` (steg = 0: no update, set `from`).
-// Reduced: [0] sum of squares, [1] max |.|, [2] gvec = sum P/ux + Q/xl.
+// xsi, eta likewise) written to set `to` (steg = 0: no update, set `from`), and
+// the sums of the Newton system there.
+// Reduced: [0] sum of squares, [1] max |.|, [2] gvec = sum P/ux + Q/xl,
+// [3] sum GG delx/diagx, [4] sum GG^2/diagx.
 __global__ __launch_bounds__(BS) void mma_resid_kernel(int64_t n, MmaVec w, int from, int to,
                                                        double steg, double lam, double epsi,
                                                        const double* __restrict__ low,
                                                        const double* __restrict__ upp,
-                                                       double* __restrict__ partials) {
+                                                       double* partials) {
   __shared__ double sh[NR * (BS / 64)];
-  double red[NR] = {0.0, 0.0, 0.0, 0.0};
+  double red[NR] = {0.0, 0.0, 0.0, 0.0, 0.0};
   for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS) {
     double x = w.x[from][i], xsi = w.xsi[from][i], eta = w.eta[from][i];
     if (to != from) {
@@ -180,39 +195,24 @@ __global__ __launch_bounds__(BS) void mma_resid_kernel(int64_t n, MmaVec w, int 
       w.x[to][i] = x; w.xsi[to][i] = xsi; w.eta[to][i] = eta;
     }
     const double ux1 = upp[i] - x, xl1 = x - low[i];
-    const double plam = w.p0[i] + w.P[i] * lam, qlam = w.q0[i] + w.Q[i] * lam;
-    const double rex = plam / (ux1 * ux1) - qlam / (xl1 * xl1) - xsi + eta;
-    const double rexsi = xsi * (x - w.alfa[i]) - epsi;
-    const double reeta = eta * (w.beta[i] - x) - epsi;
+    const double ux2 = ux1 * ux1, xl2 = xl1 * xl1;
+    const double P = w.P[i], Q = w.Q[i];
+    const double plam = w.p0[i] + P * lam, qlam = w.q0[i] + Q * lam;
+    const double xa = x - w.alfa[i], bx = w.beta[i] - x;
+    const double grad = plam / ux2 - qlam / xl2;
+    const double rex = grad - xsi + eta;
+    const double rexsi = xsi * xa - epsi;
+    const double reeta = eta * bx - epsi;
     red[0] += rex * rex + rexsi * rexsi + reeta * reeta;
     red[1] = fmax(red[1], fmax(fabs(rex), fmax(fabs(rexsi), fabs(reeta))));
-    red[2] += w.P[i] / ux1 + w.Q[i] / xl1;
+    red[2] += P / ux1 + Q / xl1;
+    const double GG = P / ux2 - Q / xl2;
+    const double delx = grad - epsi / xa + epsi / bx;
+    const double diagx = 2.0 * (plam / (ux1 * ux2) + qlam / (xl1 * xl2)) + xsi / xa + eta / bx;
+    red[3] += GG * (delx / diagx);
+    red[4] += GG * GG / diagx;
   }
   block_reduce(red, 2u, sh);
-  store_red(red, partials);
-}
-
-// Newton system sums at set `cur`: [0] gvec, [1] sum GG delx/diagx, [2] sum GG^2/diagx
-__global__ __launch_bounds__(BS) void mma_newton_kernel(int64_t n, MmaVec w, int cur, double lam,
-                                                        double epsi, const double* __restrict__ low,
-                                                        const double* __restrict__ upp,
-                                                        double* __restrict__ partials) {
-  __shared__ double sh[NR * (BS / 64)];
-  double red[NR] = {0.0, 0.0, 0.0, 0.0};
-  for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS) {
-    const double x = w.x[cur][i], xsi = w.xsi[cur][i], eta = w.eta[cur][i];
-    const double ux1 = upp[i] - x, xl1 = x - low[i];
-    const double ux2 = ux1 * ux1, xl2 = xl1 * xl1;
-    const double plam = w.p0[i] + w.P[i] * lam, qlam = w.q0[i] + w.Q[i] * lam;
-    const double GG = w.P[i] / ux2 - w.Q[i] / xl2;
-    const double xa = x - w.alfa[i], bx = w.beta[i] - x;
-    const double delx = plam / ux2 - qlam / xl2 - epsi / xa + epsi / bx;
-    const double diagx = 2.0 * (plam / (ux1 * ux2) + qlam / (xl1 * xl2)) + xsi / xa + eta / bx;
-    red[0] += w.P[i] / ux1 + w.Q[i] / xl1;
-    red[1] += GG * (delx / diagx);
-    red[2] += GG * GG / diagx;
-  }
-  block_reduce(red, 0u, sh);
   store_red(red, partials);
 }
 
@@ -222,9 +222,9 @@ __global__ __launch_bounds__(BS) void mma_dir_kernel(int64_t n, MmaVec w, int cu
                                                      double dlam, double epsi,
                                                      const double* __restrict__ low,
                                                      const double* __restrict__ upp,
-                                                     double* __restrict__ partials) {
+                                                     double* partials) {
   __shared__ double sh[NR * (BS / 64)];
-  double red[NR] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  double red[NR] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY, -INFINITY};
   for (int64_t i = blockIdx.x * int64_t(BS) + threadIdx.x; i < n; i += int64_t(gridDim.x) * BS) {
     const double x = w.x[cur][i], xsi = w.xsi[cur][i], eta = w.eta[cur][i];
     const double ux1 = upp[i] - x, xl1 = x - low[i];
@@ -276,19 +276,40 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
   for (int k = 0; k < 15; ++k) *slots[k] = base + size_t(k) * size_t(n);
   const unsigned nb = unsigned(std::min<int64_t>((n + BS - 1) / BS, 1024));
   double* partials = W.partials.as<double>();
-  double* out = W.hout;
-  double h[NR];
+  double* out = W.hout;  // the set that the next fold writes
+  double h[NR] = {};
+  auto empty = [&](double* set) {
+    for (int k = 0; k < NR; ++k) reinterpret_cast<volatile uint64_t*>(set)[k] = kEmpty;
+    std::atomic_thread_fence(std::memory_order_seq_cst);
+  };
+  // Folds the pass just launched and waits for its values: a bounded spin on
+  // the slots, then the stream.
   auto fold = [&](unsigned maxmask) -> int {
     hipLaunchKernelGGL(mma_fold_kernel, dim3(1), dim3(BS), 0, s, partials, nb, maxmask, out);
     TL_CHECK_LAUNCH();
-    TL_HIP(hipStreamSynchronize(s));
-    for (int k = 0; k < NR; ++k) h[k] = static_cast<volatile double*>(out)[k];
+    auto* q = reinterpret_cast<volatile uint64_t*>(out);
+    out = out == W.hout ? W.hout + NR : W.hout;
+    empty(out);
+    using clock = std::chrono::steady_clock;
+    const auto until = clock::now() + std::chrono::milliseconds(2);
+    bool synced = false;
+    for (int k = 0; k < NR; ++k) {
+      uint64_t bits = q[k];
+      for (unsigned spin = 0; !synced && bits == kEmpty; ++spin) {
+        if ((spin & 255u) == 255u && clock::now() > until) {
+          TL_HIP(hipStreamSynchronize(s));
+          synced = true;
+        }
+        bits = q[k];
+      }
+      std::memcpy(&h[k], &bits, sizeof(double));
+    }
     return TL_OK;
   };
+  empty(out);
   // approximation and the subproblem's start point
   hipLaunchKernelGGL(mma_prep_kernel, dim3(nb), dim3(BS), 0, s, n, x, xold1, xold2, xmin, xmax,
                      df0dx, dfdx, low, upp, int(iter), *o, w, partials);
-  TL_CHECK_LAUNCH();
   TL_TRY(fold(0u));
   const double b = h[0] - fval;
   const double a0 = o->a0, a = o->a, c = o->c, d = o->d;
@@ -307,19 +328,14 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
   for (double epsi = 1.0; epsi > 1e-7; epsi *= 0.1) {
     hipLaunchKernelGGL(mma_resid_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, cur, 0.0, lam, epsi,
                        low, upp, partials);
-    TL_CHECK_LAUNCH();
     TL_TRY(fold(2u));
+    double gvec = h[2], S1 = h[3], S2 = h[4];
     double sq, mx;
     scal_res(h[2], epsi, y, z, lam, mu, zet, sl, sq, mx);
     double residunorm = std::sqrt(h[0] + sq);
     double residumax = std::max(h[1], mx);
     for (int ittt = 0; residumax > 0.9 * epsi && ittt < 200; ++ittt) {
       ++its;
-      hipLaunchKernelGGL(mma_newton_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, lam, epsi, low,
-                         upp, partials);
-      TL_CHECK_LAUNCH();
-      TL_TRY(fold(0u));
-      const double gvec = h[0], S1 = h[1], S2 = h[2];
       const double dely = c + d * y - lam - epsi / y;
       const double delz = a0 - a * lam - epsi / z;
       const double dellam = gvec - a * z - y - b + epsi / lam;
@@ -336,9 +352,8 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
       const double dmu = -mu + epsi / y - (mu * dy) / y;
       const double dzet = -zet + epsi / z - zet * dz / z;
       const double ds = -sl + epsi / lam - (sl * dlam) / lam;
-      hipLaunchKernelGGL(mma_dir_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, lam, dlam, epsi,
+        hipLaunchKernelGGL(mma_dir_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, lam, dlam, epsi,
                          low, upp, partials);
-      TL_CHECK_LAUNCH();
       TL_TRY(fold(15u));
       double stm = std::max({h[0], h[1], h[2], h[3], 1.0});
       const double sv[6] = {y, z, lam, mu, zet, sl}, dv[6] = {dy, dz, dlam, dmu, dzet, ds};
@@ -350,10 +365,10 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
       for (int itto = 0; resinew > residunorm && itto < 50; ++itto) {
         y = y0 + steg * dy; z = z0 + steg * dz; lam = l0 + steg * dlam;
         mu = m0 + steg * dmu; zet = ze0 + steg * dzet; sl = s0 + steg * ds;
-        hipLaunchKernelGGL(mma_resid_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, trial, steg, lam,
+            hipLaunchKernelGGL(mma_resid_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, trial, steg, lam,
                            epsi, low, upp, partials);
-        TL_CHECK_LAUNCH();
         TL_TRY(fold(2u));
+        gvec = h[2]; S1 = h[3]; S2 = h[4];
         scal_res(h[2], epsi, y, z, lam, mu, zet, sl, sq, mx);
         resinew = std::sqrt(h[0] + sq);
         residumax = std::max(h[1], mx);
