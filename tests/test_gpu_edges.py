@@ -96,6 +96,37 @@ def test_level1_from_densities(gpu, dims, nlevels, ndpn):
     op.close()
 
 
+# small 3D levels: the residual restricted in the same pass (up to 8,192 nodes)
+# and the correction added inside the first sweep (up to 16,384); workgroups
+# of 16 nodes over node lines of 2 to 33 nodes, node counts that 16 does not
+# divide, and a level (9,801 nodes) with the second form alone
+@pytest.mark.parametrize("dims,ndpn,nlevels,gamma,nu", [
+    ((16, 8, 24), 3, 4, 2, 2), ((8, 128, 8), 3, 4, 1, 1), ((48, 24, 24), 1, 4, 2, 1),
+    ((40, 8, 16), 1, 4, 1, 2), ((128, 128, 32), 1, 4, 1, 1)])
+def test_small_stencil_levels(gpu, dims, ndpn, nlevels, gamma, nu):
+    """First PCG iterate of the FP64 and FP32 cycles against the oracle's
+    (rounding times the condition, as in the V-cycle parity test); with an
+    element matrix of no symmetry pattern level 1 is a stencil too."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    say("small stencil levels", dims, ndpn, nlevels, gamma, nu)
+    KE, edof, ndof, fixed, free, x = _problem(dims, ndpn)
+    b = np.random.default_rng(3).standard_normal(len(free))
+    s = np.random.default_rng(4).uniform(0.9, 1.1, KE.shape[0])
+    for ke in (KE, s[:, None] * KE * s):
+        K = fem.apply_bc(fem.assemble_K(ke, edof, fem.simp(x), ndof), free).tocsr()
+        h = mg.Hierarchy(K, *dims, ndpn, fixed, nlevels, nu1=nu, nu2=nu)
+        ref, _, _ = mg.pcg(K, b, lambda r: h.vcycle(r, 0, gamma, 1), maxiter=1)
+        op = StiffnessOperator(*dims, KE=ke, fixed=fixed, device=gpu)
+        op.set_density(x)
+        for prec, tol in (("fp64", 1e-8), ("fp32", 2e-3)):
+            op.setup_mg(nlevels=nlevels, precision=prec, gamma=gamma, gamma_from=1, nu1=nu, nu2=nu)
+            got, _ = op.solve(op.full(torch.as_tensor(b, device=gpu)), maxiter=1,
+                              raise_on_fail=False)
+            assert rel(got[op._free_t].cpu().numpy(), ref) < tol, prec
+        op.close()
+
+
 # convolution layers: result channels and nodes in tiles of 16, source channels
 # in 1, 2, 4, 8 or 16 groups of 4; one channel, partial and several tiles, one
 # node, more node tiles than workgroups

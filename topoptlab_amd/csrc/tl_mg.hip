@@ -570,69 +570,174 @@ __global__ __launch_bounds__(BS) void st_apply_kernel(GridD g, const T* __restri
 // On larger levels (30,625 nodes) the one-lane form with three pairs per
 // load group is faster: it already has waves enough, and the quad's extra
 // threads and exchanges cost more than the shorter chains save.
-template <int NDPN, typename T, int MODE>
+template <int NDPN, typename T>
+struct QuadRow {
+  static constexpr int NN = NDPN * NDPN, NT = 7;  // terms per lane (lane 3: 6)
+  T w[NT][NN];
+  int ix, iy, iz;
+  // block A(n, m) of the lane's terms: the forward block of n (K >= 13), else the
+  // transposed forward block of m; m is clamped, a missing neighbour's block is 0
+  __device__ __forceinline__ void load(const GridD& g, const T* __restrict__ sth, int64_t n, int q) {
+    node_xyz(g, n, ix, iy, iz);
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int K = min(q + 4 * j, 26);  // lane 3's seventh slot repeats term 26 with weight 0
+      const int rz = K / 9 - 1, rx = K / 3 % 3 - 1, ry = K % 3 - 1;
+      const bool fwd = K >= 13;
+      const bool ok = q + 4 * j <= 26 && (fwd || node_in(g, ix + rx, iy + ry, iz + rz));
+      const T* h = sth + int64_t(fwd ? K - 13 : 13 - K) * NN * g.nnodes + (fwd ? n : neighbour(g, K));
+#pragma unroll
+      for (int d = 0; d < NDPN; ++d)
+#pragma unroll
+        for (int c = 0; c < NDPN; ++c) {
+          const T v = h[int64_t(fwd ? d * NDPN + c : c * NDPN + d) * g.nnodes];
+          w[j][d * NDPN + c] = ok ? v : T(0);
+        }
+    }
+  }
+  __device__ __forceinline__ int64_t neighbour(const GridD& g, int K) const {
+    const int rz = K / 9 - 1, rx = K / 3 % 3 - 1, ry = K % 3 - 1;
+    return node_id(g, min(max(ix + rx, 0), g.nx - 1), min(max(iy + ry, 0), g.ny - 1),
+                   min(max(iz + rz, 0), g.nz - 1));
+  }
+  // DOF min(q, NDPN - 1) of (A x)_n from the terms' x values
+  __device__ __forceinline__ T sum(const T (&xm)[NT][NDPN], int q) const {
+    T a = T(0);
+#pragma unroll
+    for (int d = 0; d < NDPN; ++d) {
+      T s = T(0);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int c = 0; c < NDPN; ++c) s += w[j][d * NDPN + c] * xm[j][c];
+      s += __shfl_xor(s, 1, 64);
+      s += __shfl_xor(s, 2, 64);
+      a = q >= d ? s : a;
+    }
+    return a;
+  }
+  // x of the terms' neighbours read from memory, then the sum
+  __device__ __forceinline__ T apply(const GridD& g, const T* __restrict__ x, int q) const {
+    T xm[NT][NDPN];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      const int64_t m = neighbour(g, min(q + 4 * j, 26));
+#pragma unroll
+      for (int c = 0; c < NDPN; ++c) xm[j][c] = x[m * NDPN + c];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    return sum(xm, q);
+  }
+};
+
+// PRO (MODE 1): x is the iterate before the coarse correction cc.  The 16 nodes
+// of a workgroup read at most nine runs of 18 consecutive nodes; their
+// corrected values are formed once, in LDS (a run that leaves its node line
+// only meets blocks that are 0).  A prolongation of its own costs a launch:
+// 3.1-3.9 us and a gap on these levels.
+template <int NDPN, typename T, int MODE, bool PRO>
 __global__ __launch_bounds__(64) void st_apply_quad_kernel(GridD g, const T* __restrict__ sth,
                                                            const T* __restrict__ x,
                                                            const T* __restrict__ b,
                                                            const T* __restrict__ dinv, T omega,
                                                            const uint8_t* __restrict__ mask,
-                                                           T* __restrict__ y, const int* done) {
-  constexpr int NN = NDPN * NDPN, NT = 7;  // terms per lane (lane 3: 6)
+                                                           T* __restrict__ y, const int* done,
+                                                           CoarseCorr<T> cc) {
   if (*done) return;
+  constexpr int RUN = 18, NS = 9 * RUN;
+  __shared__ T xs[PRO ? NS * NDPN : 1];
   const unsigned nb = gridDim.x, hw = blockIdx.x;
   const unsigned xcd = hw & 7u, qq = nb >> 3, rr = nb & 7u;
   const unsigned logical = xcd * qq + min(xcd, rr) + (hw >> 3);
-  const int64_t n = (int64_t(logical) * 64 + threadIdx.x) >> 2;
+  const int64_t n0 = int64_t(logical) * 16, n = n0 + (threadIdx.x >> 2);
   const int q = int(threadIdx.x & 3u);
-  if (n >= g.nnodes) return;  // a whole quad: its four lanes share n
-  int ix, iy, iz;
-  node_xyz(g, n, ix, iy, iz);
-  T xm[NT][NDPN], w[NT][NN];
+  const bool in = n < g.nnodes;  // a whole quad: its four lanes share n
+  QuadRow<NDPN, T> row;
+  row.load(g, sth, in ? n : g.nnodes - 1, q);
+  T a, own = T(0);
+  const int64_t i = (in ? n : 0) * NDPN + min(q, NDPN - 1);
+  if constexpr (PRO) {
 #pragma unroll
-  for (int j = 0; j < NT; ++j) {
-    const int K = min(q + 4 * j, 26);  // lane 3's seventh slot repeats term 26 with weight 0
-    const bool live = q + 4 * j <= 26;
-    const int rz = K / 9 - 1, rx = K / 3 % 3 - 1, ry = K % 3 - 1;
-    const int64_t m = node_id(g, min(max(ix + rx, 0), g.nx - 1), min(max(iy + ry, 0), g.ny - 1),
-                              min(max(iz + rz, 0), g.nz - 1));
+    for (int k = 0; k < (NS + 63) / 64; ++k) {
+      const int e = int(threadIdx.x) + 64 * k;
+      if (e < NS) {
+        const int rz = e / (3 * RUN) - 1, rx = e / RUN % 3 - 1;
+        int64_t m = n0 + e % RUN - 1 + (int64_t(rz) * g.nx + rx) * g.ny;
+        m = m < 0 ? 0 : (m >= g.nnodes ? g.nnodes - 1 : m);
+        int mx, my, mz;
+        node_xyz(g, m, mx, my, mz);
+        T pc[NDPN];
+        prolong_at<NDPN, T, true>(cc.gc, cc.xc, mx, my, mz, pc);
+        const uint8_t mk = mask[m];
 #pragma unroll
-    for (int c = 0; c < NDPN; ++c) xm[j][c] = x[m * NDPN + c];
-    // forward block of n (K >= 13), else the transposed forward block of m
-    const bool fwd = K >= 13;
-    const bool ok = live && (fwd || node_in(g, ix + rx, iy + ry, iz + rz));
-    const T* h = sth + int64_t(fwd ? K - 13 : 13 - K) * NN * g.nnodes + (fwd ? n : m);
-#pragma unroll
-    for (int d = 0; d < NDPN; ++d)
-#pragma unroll
-      for (int c = 0; c < NDPN; ++c) {
-        const T v = h[int64_t(fwd ? d * NDPN + c : c * NDPN + d) * g.nnodes];
-        w[j][d * NDPN + c] = ok ? v : T(0);
+        for (int c = 0; c < NDPN; ++c) {
+          const T v = x[m * NDPN + c];
+          xs[e * NDPN + c] = ((mk >> c) & 1) ? v : v + pc[c];
+        }
       }
+    }
+    __syncthreads();
+    T xm[QuadRow<NDPN, T>::NT][NDPN];
+#pragma unroll
+    for (int j = 0; j < QuadRow<NDPN, T>::NT; ++j) {
+      const int K = min(q + 4 * j, 26);
+      const int e = K / 3 * RUN + int(threadIdx.x >> 2) + K % 3;  // run (rz, rx), place ry
+#pragma unroll
+      for (int c = 0; c < NDPN; ++c) xm[j][c] = xs[e * NDPN + c];
+    }
+    a = row.sum(xm, q);
+    own = xs[(4 * RUN + int(threadIdx.x >> 2) + 1) * NDPN + min(q, NDPN - 1)];
+  } else {
+    a = row.apply(g, x, q);
+    if constexpr (MODE == 1) own = x[i];
   }
-  __builtin_amdgcn_sched_barrier(0);
-  T acc[NDPN];
-#pragma unroll
-  for (int d = 0; d < NDPN; ++d) acc[d] = T(0);
-#pragma unroll
-  for (int j = 0; j < NT; ++j)
-#pragma unroll
-    for (int d = 0; d < NDPN; ++d)
-#pragma unroll
-      for (int c = 0; c < NDPN; ++c) acc[d] += w[j][d * NDPN + c] * xm[j][c];
-#pragma unroll
-  for (int d = 0; d < NDPN; ++d) {
-    acc[d] += __shfl_xor(acc[d], 1, 64);
-    acc[d] += __shfl_xor(acc[d], 2, 64);
-  }
-  if (q >= NDPN) return;
-  T a = acc[0];
-#pragma unroll
-  for (int d = 1; d < NDPN; ++d) a = q == d ? acc[d] : a;
-  const int64_t i = n * NDPN + q;
+  if (!in || q >= NDPN) return;
   T v;
   if (MODE == 0) v = b[i] - a;
-  else v = x[i] + omega * dinv[i] * (b[i] - a);
+  else v = own + omega * dinv[i] * (b[i] - a);
   y[i] = ((mask[n] >> q) & 1) ? T(0) : v;
+}
+
+// Residual and restriction of a small 3D level in one pass: a workgroup per
+// coarse node, a quad per fine node around it (27 of them; a fine row is formed
+// by up to eight workgroups, 3.4 on average, from the L2).  The weighted sum
+// takes the 27 residuals in the order of the separate restriction.  With xc
+// set, also the coarse level's first sweep.  Worth it while the redundant rows
+// cost less than a launch (restrict_quad): up to 8,192 fine nodes.
+template <int NDPN, typename T>
+__global__ __launch_bounds__(128) void st_restrict_quad_kernel(
+    GridD g, const T* __restrict__ sth, const T* __restrict__ x, const T* __restrict__ b,
+    const uint8_t* __restrict__ mask, GridD gc, const uint8_t* __restrict__ maskc,
+    T* __restrict__ bc, const T* __restrict__ dinvc, T omega, T* __restrict__ xc, const int* done) {
+  if (*done) return;
+  __shared__ T res[27 * NDPN];
+  const int64_t nc = blockIdx.x;
+  int cx, cy, cz;
+  node_xyz(gc, nc, cx, cy, cz);
+  const int f = int(threadIdx.x >> 2), q = int(threadIdx.x & 3u);
+  const int K = min(f, 26);
+  const int dz = K / 9 - 1, dx = K / 3 % 3 - 1, dy = K % 3 - 1;
+  const int fx = 2 * cx + dx, fy = 2 * cy + dy, fz = 2 * cz + dz;
+  const bool in = f < 27 && node_in(g, fx, fy, fz);
+  const int64_t n = in ? node_id(g, fx, fy, fz) : 0;
+  QuadRow<NDPN, T> row;
+  row.load(g, sth, n, q);
+  const T a = row.apply(g, x, q);
+  if (f < 27 && q < NDPN) {
+    const int64_t i = n * NDPN + q;
+    const T v = b[i] - a;
+    const T w = T((dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0));
+    res[K * NDPN + q] = !in || ((mask[n] >> q) & 1) ? T(0) : w * v;
+  }
+  __syncthreads();
+  if (int(threadIdx.x) >= NDPN) return;
+  const int d = int(threadIdx.x);
+  T s = T(0);
+#pragma unroll
+  for (int k = 0; k < 27; ++k) s += res[k * NDPN + d];
+  const T v = ((maskc[nc] >> d) & 1) ? T(0) : s;
+  bc[nc * NDPN + d] = v;
+  if (xc) xc[nc * NDPN + d] = zero_guess_sweep<T, T>(omega, dinvc[nc * NDPN + d], v);
 }
 
 // x = omega*dinv*b  (first smoothing sweep from a zero guess); b may be fp64
@@ -1448,6 +1553,19 @@ int st_dimu(const Grid& g) {
 // levels 2-3: 120-480 workgroups instead of 17-120).
 constexpr unsigned kStBlock3d = 64;
 
+// Four lanes per node on the smallest 3D levels (never recorded for a lockstep
+// batch).
+template <int NDPN>
+bool quad_level(const tl_problem* P, const Grid& g) {
+  return st_dimu<NDPN>(g) == 5 && !P->rec && g.nnodes <= 16384;
+}
+
+// Residual and restriction of a quad level in one launch.
+template <int NDPN>
+bool restrict_quad(const tl_problem* P, const Grid& g) {
+  return quad_level<NDPN>(P, g) && g.nnodes <= 8192;
+}
+
 template <int NDPN, typename T>
 int st_apply(tl_problem* P, int l, int mode, const T* x, const T* b, T* y, const int* done) {
   Level& L = P->mg.lv[l];
@@ -1494,17 +1612,15 @@ int st_apply(tl_problem* P, int l, int mode, const T* x, const T* b, T* y, const
   using I5 = std::integral_constant<int, 5>;
   if (dimu == 4) {
     if constexpr (NDPN != 2) { if (mode == 0) go(I0{}, I4{}); else go(I1{}, I4{}); }
-  } else if (dimu == 5 && !P->rec && L.g.nnodes <= 16384) {
-    // four lanes per node on the smallest levels (3D levels are never
-    // recorded for a lockstep batch)
+  } else if (quad_level<NDPN>(P, L.g)) {
     if constexpr (NDPN != 2) {
-      const unsigned nq = unsigned((4 * L.g.nnodes + kStBlock3d - 1) / kStBlock3d);
+      const unsigned nq = unsigned((L.g.nnodes + 15) / 16);
       if (mode == 0)
-        hipLaunchKernelGGL((st_apply_quad_kernel<NDPN, T, 0>), dim3(nq), dim3(kStBlock3d), 0,
-                           P->stream, gd, st, x, b, dinv, om, mk, y, done);
+        hipLaunchKernelGGL((st_apply_quad_kernel<NDPN, T, 0, false>), dim3(nq), dim3(64), 0, P->stream,
+                           gd, st, x, b, dinv, om, mk, y, done, CoarseCorr<T>{});
       else
-        hipLaunchKernelGGL((st_apply_quad_kernel<NDPN, T, 1>), dim3(nq), dim3(kStBlock3d), 0,
-                           P->stream, gd, st, x, b, dinv, om, mk, y, done);
+        hipLaunchKernelGGL((st_apply_quad_kernel<NDPN, T, 1, false>), dim3(nq), dim3(64), 0, P->stream,
+                           gd, st, x, b, dinv, om, mk, y, done, CoarseCorr<T>{});
     }
   } else if (dimu == 5) {
     if constexpr (NDPN != 2) { if (mode == 0) go(I0{}, I5{}); else go(I1{}, I5{}); }
@@ -1518,13 +1634,14 @@ int st_apply(tl_problem* P, int l, int mode, const T* x, const T* b, T* y, const
 }
 
 // Whether the prolongation into level l is fused with its first post-smoothing
-// sweep: on the small (unrolled-form) 2D levels.  In 3D the 27 neighbours'
-// extra coarse gathers exceed the registers (3 DOFs per node: 2 KB of scratch
-// per lane in FP64; 1 DOF: 256 VGPRs, one wave per SIMD), so the two passes
-// stay separate there.
+// sweep: on the small (unrolled-form) 2D levels and on the four-lane 3D ones
+// (through LDS).  In the one-lane 3D forms the 27 neighbours' extra coarse
+// gathers exceed the registers (3 DOFs per node: 2 KB of scratch per lane in
+// FP64; 1 DOF: 256 VGPRs, one wave per SIMD), so the two passes stay separate
+// there.
 template <int NDPN>
-bool fuse_correction(const Grid& g) {
-  return NDPN != 3 && st_dimu<NDPN>(g) == 2;
+bool fuse_correction(const tl_problem* P, const Grid& g) {
+  return (NDPN != 3 && st_dimu<NDPN>(g) == 2) || quad_level<NDPN>(P, g);
 }
 
 // y = x' + omega D^-1 (b - A x'), x' = x + P xc on the free DOFs: the
@@ -1536,7 +1653,7 @@ int st_smooth_corrected(tl_problem* P, int l, const T* x, const T* xc, const T* 
   Level& L = P->mg.lv[l];
   TL_ARG(l >= 1 && l + 1 < P->mg.nlevels, "internal: stencil level out of range");
   const int dimu = st_dimu<NDPN>(L.g);
-  TL_ARG(fuse_correction<NDPN>(L.g), "internal: fused correction on a level without it");
+  TL_ARG(fuse_correction<NDPN>(P, L.g), "internal: fused correction on a level without it");
   TL_NONNULL(L.sth64.ptr); TL_NONNULL(L.st32.ptr); TL_NONNULL(L.dinv64.ptr);
   TL_NONNULL(L.dinv32.ptr); TL_NONNULL(L.mask.ptr); TL_NONNULL(x); TL_NONNULL(xc);
   TL_NONNULL(b); TL_NONNULL(y);
@@ -1554,7 +1671,13 @@ int st_smooth_corrected(tl_problem* P, int l, const T* x, const T* xc, const T* 
   cc.mask = L.mask.as<uint8_t>();
   const GridD gd = to_d(L.g);
   const T om = T(P->mg.omega);
-  (void)dimu;  // 2: fuse_correction levels are 2D
+  if (dimu == 5) {
+    if constexpr (NDPN != 2)
+      hipLaunchKernelGGL((st_apply_quad_kernel<NDPN, T, 1, true>), dim3(unsigned((L.g.nnodes + 15) / 16)),
+                         dim3(64), 0, P->stream, gd, st, x, b, dinv, om, cc.mask, y, done, cc);
+    TL_CHECK_LAUNCH();
+    return prof_end(P, ev);
+  }
   if constexpr (NDPN != 3) {
     if (P->rec) {
       P->rec->add(P->rec_phase, P->rec_level, &st_apply_multi_launch<NDPN, T, 1, 2, true>,
@@ -1564,6 +1687,32 @@ int st_smooth_corrected(tl_problem* P, int l, const T* x, const T* xc, const T* 
     hipLaunchKernelGGL((st_apply_kernel<NDPN, T, 1, 2, true>), dim3(nb), dim3(BS), 0, P->stream,
                        gd, st, x, b, dinv, om, cc.mask, y, done, cc);
   }
+  TL_CHECK_LAUNCH();
+  return prof_end(P, ev);
+}
+
+// Level l's residual restricted into level l+1, with its first sweep unless it
+// is the coarsest (restrict_quad levels only).
+template <int NDPN, typename T>
+int resid_restrict(tl_problem* P, int l, const T* x, const T* b, const int* done) {
+  MgState& M = P->mg;
+  Level& L = M.lv[l];
+  Level& C = M.lv[l + 1];
+  TL_ARG(restrict_quad<NDPN>(P, L.g), "internal: fused restriction on a level without it");
+  TL_NONNULL(L.sth64.ptr); TL_NONNULL(L.st32.ptr); TL_NONNULL(L.mask.ptr); TL_NONNULL(C.mask.ptr);
+  TL_NONNULL(C.vb.ptr); TL_NONNULL(x); TL_NONNULL(b);
+  const bool seed = l + 1 < M.nlevels - 1;
+  if (seed) { TL_NONNULL(C.vx.ptr); TL_NONNULL(C.dinv64.ptr); TL_NONNULL(C.dinv32.ptr); }
+  constexpr bool f64 = std::is_same<T, double>::value;
+  ProfEvent ev{};
+  ev.kind = -1;
+  if (l == 1) TL_TRY(prof_begin(P, 3, ev));
+  if constexpr (NDPN != 2)
+    hipLaunchKernelGGL((st_restrict_quad_kernel<NDPN, T>), dim3(unsigned(C.g.nnodes)), dim3(128), 0,
+                       P->stream, to_d(L.g), static_cast<const T*>(f64 ? L.sth64.ptr : L.st32.ptr), x,
+                       b, L.mask.as<uint8_t>(), to_d(C.g), C.mask.as<uint8_t>(), vp<T>(C.vb),
+                       static_cast<const T*>(f64 ? C.dinv64.ptr : C.dinv32.ptr), T(M.omega),
+                       seed ? vp<T>(C.vx) : static_cast<T*>(nullptr), done);
   TL_CHECK_LAUNCH();
   return prof_end(P, ev);
 }
@@ -1617,9 +1766,13 @@ int vcycle_level(tl_problem* P, int l, const int* done) {
       std::swap(L.vx.ptr, L.vt.ptr);
       x = vp<T>(L.vx); t = vp<T>(L.vt);
     }
-    TL_TRY((st_apply<NDPN, T>(P, l, 0, x, b, vp<T>(L.vr), done)));
     Level& C = M.lv[l + 1];
-    TL_TRY((restrict_to<NDPN, T>(P, l, L.g, vp<T>(L.vr), done)));
+    if (restrict_quad<NDPN>(P, L.g) && !(l == 1 && M.sym1)) {
+      TL_TRY((resid_restrict<NDPN, T>(P, l, x, b, done)));
+    } else {
+      TL_TRY((st_apply<NDPN, T>(P, l, 0, x, b, vp<T>(L.vr), done)));
+      TL_TRY((restrict_to<NDPN, T>(P, l, L.g, vp<T>(L.vr), done)));
+    }
     TL_TRY((vcycle_level<NDPN, T>(P, l + 1, done)));
     P->rec_phase = 1;  // up the cycle at level l
     P->rec_level = l;
@@ -1634,7 +1787,7 @@ int vcycle_level(tl_problem* P, int l, const int* done) {
       std::swap(L.vx.ptr, L.vt.ptr);
       x = vp<T>(L.vx); t = vp<T>(L.vt);
       s0 = 1;
-    } else if (fuse_correction<NDPN>(L.g)) {
+    } else if (fuse_correction<NDPN>(P, L.g)) {
       TL_TRY((st_smooth_corrected<NDPN, T>(P, l, x, vp<T>(C.vx), b, t, done)));
       std::swap(L.vx.ptr, L.vt.ptr);
       x = vp<T>(L.vx); t = vp<T>(L.vt);
