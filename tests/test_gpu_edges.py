@@ -96,10 +96,9 @@ def test_level1_from_densities(gpu, dims, nlevels, ndpn):
     op.close()
 
 
-# small 3D levels: the residual restricted in the same pass (up to 8,192 nodes)
-# and the correction added inside the first sweep (up to 16,384); workgroups
-# of 16 nodes over node lines of 2 to 33 nodes, node counts that 16 does not
-# divide, and a level (9,801 nodes) with the second form alone
+# small 3D levels (up to 16,384 nodes): the correction added inside the first
+# sweep; workgroups of 16 nodes over node lines of 2 to 33 nodes, node counts
+# that 16 does not divide, one of 9,801
 @pytest.mark.parametrize("dims,ndpn,nlevels,gamma,nu", [
     ((16, 8, 24), 3, 4, 2, 2), ((8, 128, 8), 3, 4, 1, 1), ((48, 24, 24), 1, 4, 2, 1),
     ((40, 8, 16), 1, 4, 1, 2), ((128, 128, 32), 1, 4, 1, 1)])

@@ -633,8 +633,9 @@ struct QuadRow {
 // PRO (MODE 1): x is the iterate before the coarse correction cc.  The 16 nodes
 // of a workgroup read at most nine runs of 18 consecutive nodes; their
 // corrected values are formed once, in LDS (a run that leaves its node line
-// only meets blocks that are 0).  A prolongation of its own costs a launch:
-// 3.1-3.9 us and a gap on these levels.
+// only meets blocks that are 0).  A prolongation of its own costs a launch,
+// 3.1-3.9 us and a gap on these levels, and the sweep 3.4; the corrected sweep
+// takes 4.2 us (FP32, 25 x 13 x 13 nodes).
 template <int NDPN, typename T, int MODE, bool PRO>
 __global__ __launch_bounds__(64) void st_apply_quad_kernel(GridD g, const T* __restrict__ sth,
                                                            const T* __restrict__ x,
@@ -696,48 +697,6 @@ __global__ __launch_bounds__(64) void st_apply_quad_kernel(GridD g, const T* __r
   if (MODE == 0) v = b[i] - a;
   else v = own + omega * dinv[i] * (b[i] - a);
   y[i] = ((mask[n] >> q) & 1) ? T(0) : v;
-}
-
-// Residual and restriction of a small 3D level in one pass: a workgroup per
-// coarse node, a quad per fine node around it (27 of them; a fine row is formed
-// by up to eight workgroups, 3.4 on average, from the L2).  The weighted sum
-// takes the 27 residuals in the order of the separate restriction.  With xc
-// set, also the coarse level's first sweep.  Worth it while the redundant rows
-// cost less than a launch (restrict_quad): up to 8,192 fine nodes.
-template <int NDPN, typename T>
-__global__ __launch_bounds__(128) void st_restrict_quad_kernel(
-    GridD g, const T* __restrict__ sth, const T* __restrict__ x, const T* __restrict__ b,
-    const uint8_t* __restrict__ mask, GridD gc, const uint8_t* __restrict__ maskc,
-    T* __restrict__ bc, const T* __restrict__ dinvc, T omega, T* __restrict__ xc, const int* done) {
-  if (*done) return;
-  __shared__ T res[27 * NDPN];
-  const int64_t nc = blockIdx.x;
-  int cx, cy, cz;
-  node_xyz(gc, nc, cx, cy, cz);
-  const int f = int(threadIdx.x >> 2), q = int(threadIdx.x & 3u);
-  const int K = min(f, 26);
-  const int dz = K / 9 - 1, dx = K / 3 % 3 - 1, dy = K % 3 - 1;
-  const int fx = 2 * cx + dx, fy = 2 * cy + dy, fz = 2 * cz + dz;
-  const bool in = f < 27 && node_in(g, fx, fy, fz);
-  const int64_t n = in ? node_id(g, fx, fy, fz) : 0;
-  QuadRow<NDPN, T> row;
-  row.load(g, sth, n, q);
-  const T a = row.apply(g, x, q);
-  if (f < 27 && q < NDPN) {
-    const int64_t i = n * NDPN + q;
-    const T v = b[i] - a;
-    const T w = T((dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0));
-    res[K * NDPN + q] = !in || ((mask[n] >> q) & 1) ? T(0) : w * v;
-  }
-  __syncthreads();
-  if (int(threadIdx.x) >= NDPN) return;
-  const int d = int(threadIdx.x);
-  T s = T(0);
-#pragma unroll
-  for (int k = 0; k < 27; ++k) s += res[k * NDPN + d];
-  const T v = ((maskc[nc] >> d) & 1) ? T(0) : s;
-  bc[nc * NDPN + d] = v;
-  if (xc) xc[nc * NDPN + d] = zero_guess_sweep<T, T>(omega, dinvc[nc * NDPN + d], v);
 }
 
 // x = omega*dinv*b  (first smoothing sweep from a zero guess); b may be fp64
@@ -1560,12 +1519,6 @@ bool quad_level(const tl_problem* P, const Grid& g) {
   return st_dimu<NDPN>(g) == 5 && !P->rec && g.nnodes <= 16384;
 }
 
-// Residual and restriction of a quad level in one launch.
-template <int NDPN>
-bool restrict_quad(const tl_problem* P, const Grid& g) {
-  return quad_level<NDPN>(P, g) && g.nnodes <= 8192;
-}
-
 template <int NDPN, typename T>
 int st_apply(tl_problem* P, int l, int mode, const T* x, const T* b, T* y, const int* done) {
   Level& L = P->mg.lv[l];
@@ -1691,32 +1644,6 @@ int st_smooth_corrected(tl_problem* P, int l, const T* x, const T* xc, const T* 
   return prof_end(P, ev);
 }
 
-// Level l's residual restricted into level l+1, with its first sweep unless it
-// is the coarsest (restrict_quad levels only).
-template <int NDPN, typename T>
-int resid_restrict(tl_problem* P, int l, const T* x, const T* b, const int* done) {
-  MgState& M = P->mg;
-  Level& L = M.lv[l];
-  Level& C = M.lv[l + 1];
-  TL_ARG(restrict_quad<NDPN>(P, L.g), "internal: fused restriction on a level without it");
-  TL_NONNULL(L.sth64.ptr); TL_NONNULL(L.st32.ptr); TL_NONNULL(L.mask.ptr); TL_NONNULL(C.mask.ptr);
-  TL_NONNULL(C.vb.ptr); TL_NONNULL(x); TL_NONNULL(b);
-  const bool seed = l + 1 < M.nlevels - 1;
-  if (seed) { TL_NONNULL(C.vx.ptr); TL_NONNULL(C.dinv64.ptr); TL_NONNULL(C.dinv32.ptr); }
-  constexpr bool f64 = std::is_same<T, double>::value;
-  ProfEvent ev{};
-  ev.kind = -1;
-  if (l == 1) TL_TRY(prof_begin(P, 3, ev));
-  if constexpr (NDPN != 2)
-    hipLaunchKernelGGL((st_restrict_quad_kernel<NDPN, T>), dim3(unsigned(C.g.nnodes)), dim3(128), 0,
-                       P->stream, to_d(L.g), static_cast<const T*>(f64 ? L.sth64.ptr : L.st32.ptr), x,
-                       b, L.mask.as<uint8_t>(), to_d(C.g), C.mask.as<uint8_t>(), vp<T>(C.vb),
-                       static_cast<const T*>(f64 ? C.dinv64.ptr : C.dinv32.ptr), T(M.omega),
-                       seed ? vp<T>(C.vx) : static_cast<T*>(nullptr), done);
-  TL_CHECK_LAUNCH();
-  return prof_end(P, ev);
-}
-
 // Solve A_l x_l = b_l approximately (x_l := V-cycle(b_l) from the zero guess; the
 // caller's restriction has already written the first sweep into x_l).
 template <int NDPN, typename T>
@@ -1766,13 +1693,9 @@ int vcycle_level(tl_problem* P, int l, const int* done) {
       std::swap(L.vx.ptr, L.vt.ptr);
       x = vp<T>(L.vx); t = vp<T>(L.vt);
     }
+    TL_TRY((st_apply<NDPN, T>(P, l, 0, x, b, vp<T>(L.vr), done)));
     Level& C = M.lv[l + 1];
-    if (restrict_quad<NDPN>(P, L.g) && !(l == 1 && M.sym1)) {
-      TL_TRY((resid_restrict<NDPN, T>(P, l, x, b, done)));
-    } else {
-      TL_TRY((st_apply<NDPN, T>(P, l, 0, x, b, vp<T>(L.vr), done)));
-      TL_TRY((restrict_to<NDPN, T>(P, l, L.g, vp<T>(L.vr), done)));
-    }
+    TL_TRY((restrict_to<NDPN, T>(P, l, L.g, vp<T>(L.vr), done)));
     TL_TRY((vcycle_level<NDPN, T>(P, l + 1, done)));
     P->rec_phase = 1;  // up the cycle at level l
     P->rec_level = l;
