@@ -71,6 +71,25 @@ def test_tiled_operator(gpu, dims, ndpn):
     op.close()
 
 
+@pytest.mark.parametrize("dims,ndpn", [((5, 4, 3), 3), ((17, 31, 4), 1)])
+def test_tiled_operator_keeps_translation_stiffness(gpu, dims, ndpn):
+    """An element matrix whose translations cost 4e-14 of its largest entry is
+    still taken as reflection-symmetric (to 1e-13); K times a translation is
+    then 8 t per element of a node (rounding of the 8 n terms: below 1e-16 of
+    the largest entry, 1 % of it)."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    KE, edof, ndof, _, _, x = _problem(dims, ndpn)
+    t = 5e-15 * np.abs(KE).max()
+    op = StiffnessOperator(*dims, KE=KE + 8 * t * np.eye(len(KE)), fixed=[], device=gpu)
+    op.set_density(x)
+    want = np.zeros(ndof)
+    np.add.at(want, edof.ravel(), np.repeat(8 * t * fem.simp(x), edof.shape[1]))
+    got = op.matvec_full(torch.ones(ndof, dtype=torch.float64, device=gpu)).cpu().numpy()
+    assert np.abs(got - want).max() < 0.03 * want.max()
+    op.close()
+
+
 @pytest.mark.parametrize("dims,nlevels", [((28, 28, 4), 3), ((32, 28, 8), 3), ((60, 32, 4), 3),
                                           ((64, 60, 8), 3), ((16, 8, 24), 4)])
 @pytest.mark.parametrize("ndpn", [3, 1])

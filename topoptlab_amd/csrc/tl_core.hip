@@ -335,6 +335,16 @@ struct PlaneDma {
   __host__ __device__ static size_t buf_bytes(int ny) { return size_t(rounds(ny)) * BS * UB; }
 };
 
+// Grids whose FP64 products the general 3D operator takes (its two LDS planes,
+// its reduction slots).  The tiled operator could take more, but keeps to the
+// same ones, so that the sizes accepted do not depend on the element matrix.
+static bool ku3d_serves(const Grid& g, int ndpn) {
+  const size_t lds = 2 * (ndpn == 1 ? PlaneDma<1, double>::buf_bytes(g.ny)
+                                    : PlaneDma<3, double>::buf_bytes(g.ny));
+  return lds <= size_t(160) * 1024 &&
+         (int64_t(g.nx) * g.ny + BS - 1) / BS <= int64_t(kMaxRedBlocks);
+}
+
 template <int NDPN, typename T>
 __device__ inline void dma_plane(const KuArgs& a, const void* src, T* lds, int pz, int64_t j0) {
   constexpr int UB = PlaneDma<NDPN, T>::UB;
@@ -1072,7 +1082,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
     }
     unsigned nb = 0;
     TL_TRY(sym_fine_apply(P, a.u, a.y, prec, mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
-                          a.rho, a.rr, a.partials, a.done, out64, &nb));
+                          a.rho, a.rr, a.partials, a.done, &nb));
     if (mode == KU_STORE_DOT || mode == KU_JACOBI_DOT)
       return launch_fold(P, nb, a.fin, a.dot_out, a.done);
     return TL_OK;
@@ -1107,7 +1117,9 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
       case 3: return dispatch_mode<3, double>(P, a, mode, fusep, b64, out64);
     }
   } else {
-    if (P->op.sym && (mode == KU_STORE || mode == KU_STORE_DOT || b64)) return sym();
+    // the V-cycle's FP32 modes; FP32 products (tl_apply_K) keep the general form
+    // and its order of sums, which is what their callers compare runs by
+    if (P->op.sym && b64) return sym();
     a.sp = P->op.sp32.ptr; a.KE = P->op.KE32.ptr;
     switch (P->ndpn) {
       case 1: return dispatch_mode<1, float>(P, a, mode, fusep, b64, out64);
@@ -1510,7 +1522,14 @@ int tl_create(const tl_grid_desc* d, tl_problem** out) {
   }
   P->fixed_h.assign(d->fixed, d->fixed + d->nfixed);
   detect_ke_pattern(P);
-  P->op.sym = sym_fits(P->g, P->ndpn) && sym_detect(P->ndpn, P->KEh.data(), P->op.symkv);
+  std::vector<double> ks = P->KEh;  // the matrix that the general operator applies
+  if (P->op.fast_ke && d->ndim == 3)
+    for (int i = 0; i < nd * nd; ++i) {
+      const int p = d->ndpn == 3 ? kPat_h8_elast(i) : kPat_h8_poisson(i);
+      ks[i] = p > 0 ? P->op.kv[p - 1] : -P->op.kv[-p - 1];
+    }
+  P->op.sym = sym_fits(P->g, P->ndpn) && ku3d_serves(P->g, P->ndpn) &&
+              sym_detect(P->ndpn, ks.data(), P->op.symkv, P->op.symkt);
   P->op.mfma64 = false;  // the vector kernel is faster (tl_set_fp64_operator selects)
   std::vector<float> ke32(nd * nd);
   for (int i = 0; i < nd * nd; ++i) ke32[i] = float(P->KEh[i]);

@@ -253,6 +253,7 @@ struct FineOp {
   double kv[8] = {};           // group values of the pattern
   bool sym = false;            // 3D: the tiled reflection-symmetric operator applies (tl_sym.hip)
   double symkv[16] = {};       // its group values
+  double symkt = 0.0;          // and its stiffness against a translation
   // 2D operator workgroup shape per precision [fp64, fp32]: 0 = node line
   // (BS consecutive nodes), TY = 16/32/64: (BS/TY) x TY node tile; -1: by rule
   // (default_tile2d)
@@ -368,13 +369,13 @@ int fine_apply_mfma64(tl_problem* P, const double* u, double* y, int mode, const
                       const double* beta, double* partials, const int* done,
                       unsigned* nblocks_out);
 // tiled 3D operators in the reflection-symmetric form (tl_sym.hip)
-bool sym_detect(int ndpn, const double* KE, double (&kv)[16]);
+bool sym_detect(int ndpn, const double* KE, double (&kv)[16], double& kt);
 bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]);
 bool sym_fits(const Grid& g, int ndpn);
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
                    bool b64, const void* dinv, double omega, const void* pin, void* pout,
                    const double* beta, const FoldIn& rho, const FoldIn& rr, double* partials,
-                   const int* done, bool out64, unsigned* nblocks_out);
+                   const int* done, unsigned* nblocks_out);
 int sym_coarse_apply(tl_problem* P, bool f64, int mode, const void* x, const void* xc,
                      const void* b, void* y, const int* done);
 }  // namespace tl
