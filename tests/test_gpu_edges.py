@@ -212,3 +212,63 @@ def test_mma_sizes(gpu, it, n):
     """MMA step against the oracle, inputs and tolerances of its parity test."""
     from tests.test_gpu_parity import test_mma_update_matches_oracle as check
     check(gpu, it, n)
+
+
+# cycles whose first sweep, correction and scalars are formed inside the
+# operators: 2D node lines (up to 63 nodes in y) and tiles (from 64 on), one
+# node line of many workgroups; tiled 3D operators with 16, 17 and 31 nodes
+SEEDED = [((32, 60, None), 2, 3), ((12, 64, None), 2, 3), ((36, 68, None), 1, 3),
+          ((260, 8, None), 2, 3), ((16, 16, 8), 3, 3), ((32, 28, 8), 1, 3)]
+
+
+@pytest.mark.parametrize("dims,ndpn,nlevels", SEEDED)
+def test_seeded_cycle_iterates(gpu, dims, ndpn, nlevels):
+    """PCG iterates 1 and 3 of the FP64 cycle against the oracle's (bounds of
+    the V-cycle parity test: rounding times the condition)."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    say("seeded cycle", dims, ndpn)
+    KE, edof, ndof, fixed, free, x = _problem(dims, ndpn)
+    K = fem.apply_bc(fem.assemble_K(KE, edof, fem.simp(x), ndof), free).tocsr()
+    b = np.random.default_rng(3).standard_normal(len(free))
+    h = mg.Hierarchy(K, *dims, ndpn, fixed, nlevels)
+    op = StiffnessOperator(*dims, KE=KE, fixed=fixed, device=gpu)
+    op.set_density(x)
+    op.setup_mg(nlevels=nlevels, precision="fp64")
+    for k, tol in ((1, 1e-8), (3, 1e-7)):
+        ref, _, _ = mg.pcg(K, b, h.vcycle, rtol=1e-10, maxiter=k)
+        got, _ = op.solve(op.full(torch.as_tensor(b, device=gpu)), rtol=1e-10, maxiter=k,
+                          raise_on_fail=False)
+        assert rel(got[op._free_t].cpu().numpy(), ref) < tol, k
+    op.close()
+
+
+# besides, more 2D tiles than the 1,024 partials that a consumer folds itself
+# (1,256 and 2,512), and the FP32 cycles
+@pytest.mark.parametrize("dims,ndpn,nlevels", SEEDED + [((1248, 240, None), 1, 5),
+                                                        ((1248, 480, None), 2, 5)])
+def test_solve_ends_alike_within_a_chunk(gpu, dims, ndpn, nlevels):
+    """r.r is folded by the next iteration's residual, or at the end of a
+    chunk: whatever the chunk length, the solve stops at the same iteration
+    with the same bits, also when repeated on one handle."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    say("chunk lengths", dims, ndpn)
+    KE, edof, ndof, fixed, free, x = _problem(dims, ndpn)
+    f = torch.zeros(ndof, dtype=torch.float64, device=gpu)
+    f[torch.as_tensor(free, device=gpu)] = torch.as_tensor(
+        np.random.default_rng(3).standard_normal(len(free)), device=gpu)
+    op = StiffnessOperator(*dims, KE=KE, fixed=fixed, device=gpu)
+    op.set_density(x)
+    for prec in ("fp64", "fp32"):
+        op.setup_mg(nlevels=nlevels, precision=prec)
+        want, inf = op.solve(f, rtol=1e-6, check_every=1)
+        assert inf["relres_recursive"] < 1e-6
+        for every in (3, 64, 1):
+            got, i2 = op.solve(f, rtol=1e-6, check_every=every)
+            assert i2["iterations"] == inf["iterations"], (prec, every)
+            assert torch.equal(got, want), (prec, every)
+        # started from the solution: ended before its first iteration
+        again, i3 = op.solve(f, u0=want, rtol=1e-2, check_every=8)
+        assert i3["iterations"] == 0 and torch.equal(again, want)
+    op.close()

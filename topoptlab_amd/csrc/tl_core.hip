@@ -625,12 +625,10 @@ __global__ __launch_bounds__(BS) void ku3d_kernel(KuArgs a) {
 // lds: (BS + 2 ny + 2) * NDPN values of T
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool FAST>
 __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds) {
-  if (a.done && *a.done) return;
   __shared__ double sh[BS / 64 + 2];
+  if (op_ended<SRC == SRC_SEED>(a.rr, a.done, bid == 0 && threadIdx.x == 0, sh)) return;
   T beta = T(0);
   if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
-  if constexpr (SRC == SRC_SEED)
-    if (a.rr.partials && fold_in_done(a.rr, bid == 0 && threadIdx.x == 0, sh)) return;
   double dot = 0.0;
   const unsigned nline = unsigned((int64_t(a.plane) + BS - 1) / BS);
   for (unsigned tile = bid; tile < nline; tile += a.nblk) {
@@ -695,7 +693,6 @@ constexpr int ku2t_halo_nodes() { return (BS / TY + 2) * (TY + 2); }
 // lds: ku2t_halo_nodes<TY>() * NDPN values of T
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int TY>
 __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds) {
-  if (a.done && *a.done) return;
   constexpr int TX = BS / TY;
   constexpr int HY = TY + 2, HN = (TX + 2) * HY;
   static_assert(TX * TY == BS, "tile must hold BS nodes");
@@ -703,10 +700,9 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
   const unsigned ntile = unsigned(ntx) * unsigned((a.ny + TY - 1) / TY);
   const int lx = threadIdx.x / TY, ly = threadIdx.x % TY;
   __shared__ double sh[BS / 64 + 2];
+  if (op_ended<SRC == SRC_SEED>(a.rr, a.done, bid == 0 && threadIdx.x == 0, sh)) return;
   T beta = T(0);
   if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
-  if constexpr (SRC == SRC_SEED)
-    if (a.rr.partials && fold_in_done(a.rr, bid == 0 && threadIdx.x == 0, sh)) return;
   double dot = 0.0;
   for (unsigned tile = bid; tile < ntile; tile += a.nblk) {
     if (tile != bid) __syncthreads();  // the previous tile has been read

@@ -204,16 +204,29 @@ __device__ __forceinline__ double fold_in_alpha(const FoldIn& f, const PcgState*
 
 // r.r of the iteration before, and whether the solve has ended (the x/r update
 // has counted the iteration already, see UpdateArgs::count).  Folding the same
-// partials again changes nothing.
+// partials again changes nothing.  `done` is read by one thread for its whole
+// workgroup: the grid's writer may set it meanwhile, and the waves of a
+// workgroup have to leave together.  sh: blockDim/64 + 2 doubles.
 __device__ __forceinline__ bool fold_in_done(const FoldIn& f, bool writer, double* sh) {
+  const int flag = blockDim.x >> 6;  // behind the sums' slots
+  if (threadIdx.x == 0) sh[flag] = f.st->done ? 1.0 : 0.0;
   double tot[1];
   fold_partials<1>(f.partials, f.nb, tot, sh);
+  if (sh[flag] != 0.0) return true;
   const bool end = tot[0] < f.st->tol2 || f.st->it >= f.st->maxiter;
   if (writer) {
     f.st->rr = tot[0];
     f.st->done = end ? 1 : 0;
   }
   return end;
+}
+
+// Whether a workgroup of an operator call has nothing to do (SEED: the call
+// folds r.r itself where its partials are given).
+template <bool SEED>
+__device__ __forceinline__ bool op_ended(const FoldIn& rr, const int* done, bool writer, double* sh) {
+  if (SEED && rr.partials) return fold_in_done(rr, writer, sh);
+  return done && *done;
 }
 
 struct Level {

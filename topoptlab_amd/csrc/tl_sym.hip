@@ -532,7 +532,8 @@ constexpr int sym_waves() {
 // (the sweep spills, the rest is unchanged: the moves are not what bounds it).
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
 __global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kernel(SymArgs<T> a) {
-  if (a.done && *a.done) return;
+  __shared__ double sh[BS / 64 + 2];
+  if (op_ended<SRC == SRC_SEED>(a.rr, a.done, blockIdx.x == 0 && threadIdx.x == 0, sh)) return;
   __shared__ T plane[2][TS * TS * NDPN];
   __shared__ T xch[2][NDPN * BS];
   __shared__ T ring[src_corr(SRC) ? CR * TC * TC * NDPN : 1];
@@ -543,9 +544,6 @@ __global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kerne
   const unsigned units = a.ncol * unsigned(a.nz);  // units * (nb + 1) < 2^32 (launcher)
   unsigned u0 = __builtin_amdgcn_readfirstlane(units * w / nb);
   const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
-  __shared__ double sh[BS / 64 + 2];
-  if constexpr (SRC == SRC_SEED)
-    if (a.rr.partials && fold_in_done(a.rr, blockIdx.x == 0 && threadIdx.x == 0, sh)) return;
   T beta = T(0);
   if constexpr (SRC == SRC_P)
     beta = T(fold_in_beta(a.rho, a.beta, blockIdx.x == 0 && threadIdx.x == 0, sh));
