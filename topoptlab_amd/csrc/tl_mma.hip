@@ -352,7 +352,7 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
       const double dmu = -mu + epsi / y - (mu * dy) / y;
       const double dzet = -zet + epsi / z - zet * dz / z;
       const double ds = -sl + epsi / lam - (sl * dlam) / lam;
-        hipLaunchKernelGGL(mma_dir_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, lam, dlam, epsi,
+      hipLaunchKernelGGL(mma_dir_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, lam, dlam, epsi,
                          low, upp, partials);
       TL_TRY(fold(15u));
       double stm = std::max({h[0], h[1], h[2], h[3], 1.0});
@@ -365,7 +365,7 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
       for (int itto = 0; resinew > residunorm && itto < 50; ++itto) {
         y = y0 + steg * dy; z = z0 + steg * dz; lam = l0 + steg * dlam;
         mu = m0 + steg * dmu; zet = ze0 + steg * dzet; sl = s0 + steg * ds;
-            hipLaunchKernelGGL(mma_resid_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, trial, steg, lam,
+        hipLaunchKernelGGL(mma_resid_kernel, dim3(nb), dim3(BS), 0, s, n, w, cur, trial, steg, lam,
                            epsi, low, upp, partials);
         TL_TRY(fold(2u));
         gvec = h[2]; S1 = h[3]; S2 = h[4];
