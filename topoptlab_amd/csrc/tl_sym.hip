@@ -68,6 +68,7 @@ struct SymArgs {
   int fnelx, fnely;                  // CG: the fine grid below it
   int ncy;                           // tile columns along y
   unsigned ncol;                     // tile columns
+  unsigned nseg;                     // equal z ranges per column, or 0 (see sym_segments)
   T kv[16];                          // group values of the pattern
   T kt;                              // products: stiffness against a translation
 };
@@ -513,8 +514,11 @@ constexpr int sym_waves() {
   return NDPN == 3 && sizeof(T) == 8 && CG && src_corr(SRC) ? 1 : 2;
 }
 
-// The ncol * nz (tile column, node plane) units are split evenly over the
-// workgroups, in column order; each walks one or more column segments, and a
+// Split: every column into the same nseg z ranges, a workgroup each, numbered
+// range by range, so that the workgroups of an XCD walk the same planes side by
+// side and find their neighbours' halo lines in its L2; or, where that leaves
+// too many workgroups idle (sym_segments), the ncol * nz (tile column, node
+// plane) units evenly over the workgroups, in column order.  A
 // segment costs one extra element layer (the one below its first plane).  Two
 // waves per SIMD: 170-184 VGPRs in FP64 (256 for the level-1 form); a bound of
 // three spills (192x96x96, FP64: residual 40.2 instead of 39.9 us, level-1
@@ -528,6 +532,10 @@ constexpr int sym_waves() {
 // seed 45, last sweep from the seed and the coarse correction 57.5 (45.7 and a
 // prolongation of 33 before), level-1 sweep with the correction 24 (17.2 + 7),
 // and 9 us less in the PCG update, which no longer writes the seed.
+// Side by side instead of evenly: 95x61x47 product 16.1 -> 14.0 us; at 192x96x96
+// plain product 34.3 -> 32.7 (L2 misses 121 -> 66 MB), level-1 residual and sweep
+// 18.7 and 26.0 -> 17.5 and 24.7, the fine kernels with two staged inputs
+// unchanged within 1% (61.4, 51.9 and 63.2 us).
 // Measured and not kept: two layers per loop turn without the register moves
 // (the sweep spills, the rest is unchanged: the moves are not what bounds it).
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
@@ -542,8 +550,17 @@ __global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kerne
   const unsigned xcd = hw & 7u, q = nb >> 3, r = nb & 7u;
   const unsigned w = xcd * q + min(xcd, r) + (hw >> 3);
   const unsigned units = a.ncol * unsigned(a.nz);  // units * (nb + 1) < 2^32 (launcher)
-  unsigned u0 = __builtin_amdgcn_readfirstlane(units * w / nb);
-  const unsigned u1 = __builtin_amdgcn_readfirstlane(units * (w + 1) / nb);
+  unsigned u0, u1;
+  if (a.nseg) {
+    const unsigned seg = w / a.ncol, first = (w - seg * a.ncol) * unsigned(a.nz);
+    u0 = first + unsigned(a.nz) * seg / a.nseg;
+    u1 = first + unsigned(a.nz) * (seg + 1) / a.nseg;
+  } else {
+    u0 = units * w / nb;
+    u1 = units * (w + 1) / nb;
+  }
+  u0 = __builtin_amdgcn_readfirstlane(u0);
+  u1 = __builtin_amdgcn_readfirstlane(u1);
   T beta = T(0);
   if constexpr (SRC == SRC_P)
     beta = T(fold_in_beta(a.rho, a.beta, blockIdx.x == 0 && threadIdx.x == 0, sh));
@@ -584,6 +601,16 @@ int64_t tile_cols(const Grid& g) {
   return int64_t((g.nx + TN - 1) / TN) * ((g.ny + TN - 1) / TN);
 }
 
+// z ranges per column of the side-by-side split, 0 for the even one: taken where
+// its longest walk (with the layer below) is no longer than the even split's,
+// whose workgroups start a second column on the way.
+unsigned sym_segments(int64_t ncol, int64_t nz, int64_t slots) {
+  const int64_t nseg = std::min(slots / ncol, nz);
+  if (nseg < 1) return 0;
+  const int64_t even = (ncol * nz + slots - 1) / slots + 2;
+  return (nz + nseg - 1) / nseg + 1 <= even ? unsigned(nseg) : 0;
+}
+
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
 int sym_launch(hipStream_t s, const Grid& g, SymArgs<T> a, unsigned* nblocks) {
   auto* kern = sym_kernel<NDPN, T, MODE, TB, TO, SRC, CG>;
@@ -594,7 +621,9 @@ int sym_launch(hipStream_t s, const Grid& g, SymArgs<T> a, unsigned* nblocks) {
   int64_t slots = 0;
   TL_TRY(sym_slots(reinterpret_cast<const void*>(kern), slots));
   const int64_t units = int64_t(a.ncol) * g.nz;
-  const int64_t nwg = std::max<int64_t>(1, std::min<int64_t>({slots, units, int64_t(kMaxRedBlocks)}));
+  slots = std::max<int64_t>(1, std::min(slots, int64_t(kMaxRedBlocks)));
+  a.nseg = sym_segments(a.ncol, g.nz, slots);
+  const int64_t nwg = a.nseg ? int64_t(a.ncol) * a.nseg : std::min(slots, units);
   TL_ARG(units * (nwg + 1) < (int64_t(1) << 32), "internal: grid too large for the tiled operator");
   if (nblocks) *nblocks = unsigned(nwg);
   hipLaunchKernelGGL(kern, dim3(unsigned(nwg)), dim3(BS), 0, s, a);
