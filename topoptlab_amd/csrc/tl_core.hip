@@ -1414,8 +1414,12 @@ static unsigned grid_for(int64_t n) {
 
 static int launch_fold(tl_problem* P, unsigned nb, int fin, double* out, const int* done) {
   if (fin == FIN_RHO || fin == FIN_PQ) {
-    // left to the consumer; the FP64 MFMA product reads beta from the state
-    const bool in = nb <= kFoldInBlocks && !(fin == FIN_RHO && P->op.mfma64);
+    // left to the consumer; the FP64 MFMA product reads beta from the state.
+    // A lockstep batch folds all systems' scalars in one launch, and its
+    // operators fill the chip: every workgroup reading the partials first cost
+    // more than that launch (136 systems, 13.9M DOF: 594 ms per batch solve,
+    // 537 with the launch).
+    const bool in = nb <= kFoldInBlocks && !P->rec && !(fin == FIN_RHO && P->op.mfma64);
     (fin == FIN_RHO ? P->rho_nb : P->pq_nb) = in ? nb : 0u;
     if (in) return TL_OK;
   }
