@@ -35,7 +35,6 @@ sys.path.insert(0, str(ROOT))
 METRIC = "ms per FEM solve to relres 1e-8 + HBM TB/s, 192×96×96 H8 (5.45M DOF)"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3
 
 
 def log(*a):
@@ -45,21 +44,21 @@ def log(*a):
 def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4):
     """Algorithmic HBM bytes of one solve (each array touched once per kernel).
 
-    Fine level per PCG iteration: p = z + beta p 24 B/DOF, product q = K p
-    16 B/DOF + 8 B/el, x/r update 48 B/DOF plus the next V-cycle's
-    zero-guess sweep (dinv -> x) that it writes; V-cycle fine level:
-    residual (x, r -> r0), prolongation-add (x), final smoothing writing z in
-    FP64 (x, r, dinv -> z).  Coarse levels: stencil bytes twice (residual and
-    smoothing) plus their vectors; coarsest dense inverse once.
+    Fine level per PCG iteration: p = z + beta p inside the product q = K p
+    32 B/DOF + 8 B/el, x/r update 48 B/DOF; V-cycle fine level: residual from
+    the first sweep formed on the fly (r, dinv -> r0), final smoothing from the
+    same and the coarse correction, writing z in FP64 (r, dinv, xc -> z).
+    Level 1 is applied from the fine densities (residual and smoothing), deeper
+    levels read their stencils twice, plus the levels' vectors; coarsest dense
+    inverse once.
     """
     nelx, nely, nelz = dims
     ndpn = 3
     nel = nelx * nely * nelz
     ndof = ndpn * (nelx + 1) * (nely + 1) * (nelz + 1)
     w = vprec_bytes
-    fine_pcg = 24 * ndof + 16 * ndof + 8 * nel + (48 + 2 * w) * ndof
-    fine_v = (w + 8 + w) * ndof + w * nel + 2 * w * ndof \
-        + (w + 8 + w + 8) * ndof + w * nel
+    fine_pcg = 32 * ndof + 8 * nel + 48 * ndof
+    fine_v = (8 + 2 * w) * ndof + w * nel + (16 + w) * ndof + w * nel
     coarse = 0
     d = [nelx, nely, nelz]
     for lvl in range(1, nlevels):
@@ -69,7 +68,8 @@ def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4):
         if lvl == nlevels - 1:
             coarse += 8 * nd * nd + 2 * w * nd
         else:
-            st = 14 * ndpn * ndpn * nn * w  # forward half of the block stencil
+            # fine densities, or the forward half of the block stencil
+            st = nel * w if lvl == 1 else 14 * ndpn * ndpn * nn * w
             coarse += 2 * st + 12 * w * nd
     return iters * (fine_pcg + fine_v + coarse)
 
@@ -240,41 +240,37 @@ def kernel_kinds(dims, vcycle, nlevels, fp64_mfma=False):
     flops_ku = 1152.0 * nel
     vb = 8 if vcycle == "fp64" else 4  # V-cycle vector bytes (bf16/fp16: fp32 vectors)
     mfma = vcycle in ("bf16", "fp16")
-    # compute-bound kinds carry bound "mfma" (the compute roof) with the
-    # peak of the unit that runs them: FP64 vector FMAs and FP64 MFMA share
-    # 78.6 TFLOP/s on MI355X, FP32 vector FMAs 157.3 (a figure that counts
-    # packed FP32; the library is built without packed FP32 instructions, so
-    # half of it is the ceiling these kernels can reach and the fraction
-    # reported against 157.3 is the conservative one)
+    # the vector operators execute about 160 operations per element where the
+    # element product has 1152, so memory bounds them; only the FP64 MFMA walk is
+    # held against a compute peak (78.6 TFLOP/s)
     if mfma:
         vk = f"kucol_kernel {vcycle.upper()}-input MFMA (fp32 accumulate)"
         vbound, vpeak = "hbm", HBM_PEAK_GBS
     elif vcycle == "fp64" and fp64_mfma:
         vk = "kucol64_kernel FP64 MFMA (v_mfma_f64_16x16x4f64)"
         vbound, vpeak = "mfma", FP64_PEAK_TFLOPS
-    elif vcycle == "fp64":
-        vk = "ku3d_kernel FP64 (vector FMAs)"
-        vbound, vpeak = "mfma", FP64_PEAK_TFLOPS
     else:
-        vk = "ku3d_kernel FP32 (vector FMAs)"
-        vbound, vpeak = "mfma", FP32_PEAK_TFLOPS
-    sb = 14 * 9 * nn1 * vb  # level-1 block stencil bytes (forward half: centre + 13 blocks)
+        vk = f"sym_kernel {vcycle.upper()} (reflection-symmetric form)"
+        vbound, vpeak = "hbm", HBM_PEAK_GBS
+    # the tiled operators form the cycle's first sweep (r, dinv) themselves and
+    # add the level-1 correction in the last one; the MFMA walks read a stored x
+    corr = 0 if mfma or fp64_mfma else vb * nd1
+    sweep = (2 * vb + 16) if mfma or fp64_mfma else (vb + 16)
+    l1 = "fp32" if mfma else vcycle
     return {
-        # the MFMA walk fuses p = z + beta p (reads z and p, writes p and q);
-        # the vector operator takes p from a separate pointwise pass
-        0: ("kucol64_kernel FP64 MFMA fused PCG product (p = z + beta p; q = K p; p.q)" if fp64_mfma
-            else "ku3d_kernel FP64 PCG product (q = K p; p.q)",
-            (32 if fp64_mfma else 16) * ndof + 8 * nel + ndof // 3, flops_ku, "mfma",
-            FP64_PEAK_TFLOPS),
+        # both forms take p = z + beta p along (read z and p, write p and q)
+        0: (f"{'kucol64_kernel FP64 MFMA' if fp64_mfma else 'sym_kernel FP64'} fused PCG product "
+            "(p = z + beta p; q = K p; p.q)",
+            32 * ndof + 8 * nel + ndof // 3, flops_ku, "mfma" if fp64_mfma else "hbm",
+            FP64_PEAK_TFLOPS if fp64_mfma else HBM_PEAK_GBS),
         1: (f"{vk} V-cycle residual (r = b - K x)",
             (2 * vb + 8) * ndof + vb * nel + ndof // 3, flops_ku, vbound, vpeak),
         2: (f"{vk} V-cycle damped-Jacobi sweep (z in FP64, r.z)",
-            (2 * vb + 16) * ndof + vb * nel + ndof // 3, flops_ku, vbound, vpeak),
-        3: (f"st_apply_kernel {vcycle if not mfma else 'fp32'} level-1 residual (27-point block "
-            f"stencil, symmetric half stored)",
-            sb + 3 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
-        4: (f"st_apply_kernel {vcycle if not mfma else 'fp32'} level-1 damped-Jacobi sweep",
-            sb + 4 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
+            sweep * ndof + corr + vb * nel + ndof // 3, flops_ku, vbound, vpeak),
+        3: (f"sym_kernel {l1} level-1 residual (Galerkin operator from the fine densities)",
+            vb * nel + 3 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
+        4: (f"sym_kernel {l1} level-1 damped-Jacobi sweep with the level-2 correction",
+            vb * nel + 4 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
     }
 
 
