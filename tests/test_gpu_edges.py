@@ -184,6 +184,51 @@ def test_conv_tiles(gpu, stride, shape, cin, cout):
     assert rel(gw.cpu().numpy(), gw_ref) < 1e-5 and rel(gb.cpu().numpy(), gb_ref) < 1e-5
 
 
+@pytest.mark.parametrize("stride,shape,cin,cout", [(1, (3, 4, 18), 5, 20), (2, (5, 5, 9), 9, 33)])
+def test_conv_skips_taps_without_source(gpu, stride, shape, cin, cout):
+    """Infinite and NaN weights (overflowed fp16) reach the nodes whose tap has
+    a source node and no others, forward and in the data gradient: the values
+    of a loop that skips the other taps, finite ones to the 1e-5 above."""
+    import ctypes as C
+    import torch
+    from oracle import nn
+    from topoptlab_amd._lib import check, lib
+    say("conv special weights", stride, shape, cin, cout)
+    rng = np.random.default_rng(cin)
+    a = rng.standard_normal((cin,) + shape).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, 27)) * 0.2).astype(np.float16)
+    b = np.zeros(cout, np.float32)
+    w[1, 2, 0], w[2, 0, 26], w[18, 4, 3], w[0, 1, 13] = np.inf, -np.inf, np.nan, np.inf
+    oshape = nn.out_shape(shape, stride)
+    gy = rng.standard_normal((cout,) + oshape).astype(np.float32)
+    y_ref, ga_ref = np.zeros((cout,) + oshape), np.zeros(a.shape)
+    with np.errstate(invalid="ignore"):
+        for t, off in enumerate(nn.OFFS):
+            # outputs o whose source stride o + off lies in the grid
+            o = [np.array([i for i in range(m) if 0 <= stride * i + d < n], dtype=int)
+                 for m, n, d in zip(oshape, shape, off)]
+            to = (slice(None),) + np.ix_(*o)
+            ti = (slice(None),) + np.ix_(*[stride * i + d for i, d in zip(o, off)])
+            wt = w[:, :, t].astype(np.float64)
+            for co in range(cout):
+                for ci in range(cin):
+                    y_ref[co][to[1:]] += wt[co, ci] * a[ci][ti[1:]]
+                    ga_ref[ci][ti[1:]] += wt[co, ci] * gy[co][to[1:]]
+    t = lambda v: torch.as_tensor(np.ascontiguousarray(v), device=gpu)
+    p = lambda v: C.c_void_p(v.data_ptr())
+    s = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+    da, dw, db, dgy = t(a), t(w), t(b), t(gy)
+    y, ga = torch.empty(y_ref.shape, device=gpu), torch.empty(a.shape, device=gpu)
+    check(lib().tl_nn_conv3d(cin, cout, *shape, stride, 0, p(da), p(dw), p(db), p(y), s))
+    check(lib().tl_nn_conv3d_bwd_data(cin, cout, *shape, stride, p(dgy), p(dw), p(ga), 0, s))
+    for got, ref in ((y.cpu().numpy(), y_ref), (ga.cpu().numpy(), ga_ref)):
+        fin = np.isfinite(ref)
+        assert fin.any() and not fin.all()
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+        assert np.isfinite(got[fin]).all() and rel(got[fin], ref[fin]) < 1e-5
+
+
 # one workgroup up to 8,192 elements (256 threads to 2,048, else 1,024), three
 # steps per pass beyond; partial rows, blocks and grids
 @pytest.mark.parametrize("n", [2, 255, 257, 2048, 2049, 8191, 8192, 8193, 131073])

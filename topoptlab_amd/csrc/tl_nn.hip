@@ -38,6 +38,11 @@ __device__ inline int tap_dy(int t) { return t % 3 - 1; }
 // idle: 186 us (forward) and 148 us (gradient) per layer on average at that
 // size against 25 and 12 now (a design of 192x96x96: forward pass 2.5 -> 0.69
 // ms, forward and backward 26.3 -> 12.8 ms).
+//
+// A tap that has no source node for a result node is a product with 0 there,
+// which an infinite or NaN weight (an fp16 overflow) would turn into a NaN.
+// The staging looks for such weights; a workgroup that holds one skips those
+// terms on scalar FMAs instead, in the same order of sums.
 typedef float nn_f4 __attribute__((ext_vector_type(4)));
 // NG: channel groups of 4, at least kc / 4; a power of two, so that every load
 // of a tap is issued before its first product.
@@ -57,6 +62,7 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
   // weights in their memory order ([rows][k][t], BWD [k][rows][t]), a batch of
   // loads in flight
   constexpr int NW = 27 * kp * 16, NB = 9;
+  uint32_t top = 0;  // largest exponent and fraction among the staged weights
   for (int i0 = threadIdx.x; i0 < NW; i0 += CT * NB) {
     _Float16 r[NB];
 #pragma unroll
@@ -72,14 +78,15 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
     for (int b = 0; b < NB; ++b) {
       const int i = i0 + b * CT;
       const int k = BWD ? i / (27 * 16) : i / 27 % kp, m = BWD ? i / 27 % 16 : i / (27 * kp);
+      top = max(top, __builtin_bit_cast(uint16_t, r[b]) & 0x7fffu);
       if (i < NW) wl[i % 27 * TP + k * 16 + m] = r[b];
     }
   }
-  __syncthreads();
+  const bool special = __syncthreads_or(top >= 0x7c00u);  // one is infinite or NaN
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, j = l & 15, g = l >> 4;
   const int64_t nres = int64_t(rz) * rx * ry, nsrc = int64_t(sz) * sx * sy;
-  // source values of tap t for the lane's node (0 where the tap has none)
-  auto load = [&](int t, int Z, int X, int Y, float (&v)[NG]) {
+  // tap t's source node for result node (Z, X, Y); false where there is none
+  auto source = [&](int t, int Z, int X, int Y, const float*& p) {
     int z, x, y;
     bool ok;
     if constexpr (BWD) {
@@ -91,7 +98,13 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
       z = stride * Z + tap_dz(t); x = stride * X + tap_dx(t); y = stride * Y + tap_dy(t);
       ok = z >= 0 && z < sz && x >= 0 && x < sx && y >= 0 && y < sy;
     }
-    const float* p = src + (ok ? (int64_t(z) * sx + x) * sy + y : 0);
+    p = src + (ok ? (int64_t(z) * sx + x) * sy + y : 0);
+    return ok;
+  };
+  // source values of tap t for the lane's node (0 where the tap has none)
+  auto load = [&](int t, int Z, int X, int Y, float (&v)[NG]) {
+    const float* p;
+    const bool ok = source(t, Z, X, Y, p);
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
       const int c = 4 * q + g;
@@ -105,10 +118,42 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
     for (int q = 0; q < NG; ++q)
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(float(wt[q * 64]), v[q], acc, 0, 0, 0);
   };
+  // the same sums of the lane's four results without the terms that have no source
+  auto skip_product = [&](int t, int Z, int X, int Y, nn_f4& acc) {
+    const float* p;
+    if (!source(t, Z, X, Y, p)) return;
+    const _Float16* wt = wl + t * TP + 4 * g;
+    for (int c = 0; c < kc; ++c)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        acc[i] = fmaf(float(wt[c * 16 + i]), p[int64_t(c) * nsrc], acc[i]);
+  };
   auto node = [&](int64_t o, int& Z, int& X, int& Y) {
     o = o < nres ? o : nres - 1;
     Y = int(o % ry); X = int((o / ry) % rx); Z = int(o / (int64_t(ry) * rx));
   };
+  auto store = [&](int m, int64_t o, float v) {
+    if (m >= mc || o >= nres) return;
+    float* dst = out + int64_t(m) * nres + o;
+    if constexpr (BWD) {
+      *dst = accumulate ? *dst + v : v;
+    } else {
+      v += bias[m];
+      *dst = relu ? fmaxf(v, 0.f) : v;
+    }
+  };
+  if (special) {
+    for (int tile = int(blockIdx.x) * CW + wave; tile < ntiles; tile += int(gridDim.x) * CW) {
+      const int64_t o = int64_t(tile) * 16 + j;
+      int Z, X, Y;
+      node(o, Z, X, Y);
+      nn_f4 acc{0.f, 0.f, 0.f, 0.f};
+      for (int t = 0; t < 27; ++t) skip_product(t, Z, X, Y, acc);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) store(m0 + 4 * g + i, o, acc[i]);
+    }
+    return;
+  }
   if constexpr (!BWD) {
     // a wave per node tile, all taps in order: the sum of every output keeps
     // the order of a loop over taps and source channels
@@ -124,15 +169,8 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
 #pragma unroll
         for (int q = 0; q < 3; ++q) product(t + q, v[q], acc);
       }
-      if (o < nres) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = m0 + 4 * g + i;
-          if (m >= mc) continue;
-          const float v = acc[i] + bias[m];
-          out[int64_t(m) * nres + o] = relu ? fmaxf(v, 0.f) : v;
-        }
-      }
+      for (int i = 0; i < 4; ++i) store(m0 + 4 * g + i, o, acc[i]);
     }
   } else {
     // the waves share a node tile, taps in turn, sums added through LDS
@@ -150,13 +188,11 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
       for (int i = 0; i < 4; ++i) red[wave][4 * g + i][j] = acc[i];
       __syncthreads();
       const int m = threadIdx.x >> 4, n = threadIdx.x & 15;
-      const int64_t on = int64_t(tile) * 16 + n;
-      if (threadIdx.x < 256 && m0 + m < mc && on < nres) {
+      if (threadIdx.x < 256) {
         float v = 0.f;
 #pragma unroll
         for (int q = 0; q < CW; ++q) v += red[q][m][n];
-        float* dst = out + int64_t(m0 + m) * nres + on;
-        *dst = accumulate ? *dst + v : v;
+        store(m0 + m, int64_t(tile) * 16 + n, v);
       }
       __syncthreads();
     }
