@@ -184,6 +184,19 @@ def test_conv_tiles(gpu, stride, shape, cin, cout):
     assert rel(gw.cpu().numpy(), gw_ref) < 1e-5 and rel(gb.cpu().numpy(), gb_ref) < 1e-5
 
 
+# the data gradient's waves share a node tile below 512 tiles (768 with more than
+# 16 source channels): 497 and 525 tiles of 5 channels, 525 and 792 of 20; one
+# source channel forward (first) and in the gradient from 4,096 tiles (65,536
+# nodes) on, 9 result channels in groups of 8
+@pytest.mark.parametrize("stride,shape,cin,cout", [(1, (19, 19, 22), 3, 5), (1, (20, 20, 21), 3, 5),
+                                                   (1, (20, 20, 21), 3, 20), (1, (22, 24, 24), 3, 20),
+                                                   (1, (37, 41, 45), 1, 9), (1, (37, 41, 45), 9, 1),
+                                                   (2, (37, 41, 45), 2, 1)])
+def test_conv_split_rules(gpu, stride, shape, cin, cout):
+    """The same against the same bounds on both sides of the rules."""
+    test_conv_tiles(gpu, stride, shape, cin, cout)
+
+
 @pytest.mark.parametrize("stride,shape,cin,cout", [(1, (3, 4, 18), 5, 20), (2, (5, 5, 9), 9, 33)])
 def test_conv_skips_taps_without_source(gpu, stride, shape, cin, cout):
     """Infinite and NaN weights (overflowed fp16) reach the nodes whose tap has

@@ -27,17 +27,17 @@ __device__ inline int tap_dy(int t) { return t % 3 - 1; }
 //   BWD      ga[ci][n] (+)= sum_t sum_co w[co][ci][t] gy[co][o], stride*o + off_t = n
 // rows = 16 channels of the result (blockIdx.y), columns = 16 consecutive nodes
 // of the result grid, inner dimension = 4 source channels of one tap.  A lane
-// loads one source value per product, 16 lanes a run of y.  The waves of
-// a workgroup take the taps in turn and their sums are added through LDS;
-// the workgroup's weights are staged once in LDS (fp16, [t][k][16 rows]) for
-// all its node tiles.
+// loads one source value per product, 16 lanes a run of y.  A wave takes a node
+// tile, or on small grids (SPLIT) the waves of a workgroup share one, taps in
+// turn, and add their sums through LDS; the workgroup's weights are staged once
+// in LDS (fp16, [t][k][16 rows]) for all its node tiles.
 //
 // The grids are small (4,225 nodes for a 48x24x24 design), so the split is
 // over channels and taps as well as nodes.  One thread per node and 8 result
 // channels, looping over all taps and source channels, left most of the chip
 // idle: 186 us (forward) and 148 us (gradient) per layer on average at that
-// size against 25 and 12 now (a design of 192x96x96: forward pass 2.5 -> 0.69
-// ms, forward and backward 26.3 -> 12.8 ms).
+// size against 25 and 12 now (a design of 192x96x96: forward pass 2.5 -> 0.63
+// ms, forward and backward 26.2 -> 12.3 ms).
 //
 // A tap that has no source node for a result node is a product with 0 there,
 // which an infinite or NaN weight (an fp16 overflow) would turn into a NaN.
@@ -47,7 +47,7 @@ typedef float nn_f4 __attribute__((ext_vector_type(4)));
 // NG: channel groups of 4, at least kc / 4; a power of two, so that every load
 // of a tap is issued before its first product.
 constexpr int CT = 512, CW = CT / 64;  // threads and waves of a workgroup
-template <bool BWD, int NG>
+template <bool BWD, bool SPLIT, int NG, int TB>
 __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx, int ry, int sz,
                                                   int sx, int sy, int stride, int relu,
                                                   int accumulate, int ntiles,
@@ -85,31 +85,57 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
   const bool special = __syncthreads_or(top >= 0x7c00u);  // one is infinite or NaN
   const int wave = threadIdx.x >> 6, l = threadIdx.x & 63, j = l & 15, g = l >> 4;
   const int64_t nres = int64_t(rz) * rx * ry, nsrc = int64_t(sz) * sx * sy;
-  // tap t's source node for result node (Z, X, Y); false where there is none
-  auto source = [&](int t, int Z, int X, int Y, const float*& p) {
-    int z, x, y;
-    bool ok;
-    if constexpr (BWD) {
-      const int pz = Z - tap_dz(t), px = X - tap_dx(t), py = Y - tap_dy(t);
-      z = pz / stride; x = px / stride; y = py / stride;
-      ok = pz >= 0 && px >= 0 && py >= 0 && z < sz && x < sx && y < sy &&
-           !(stride == 2 && ((pz | px | py) & 1));
+  // Source node of the lane's result node for each offset of an axis (as an
+  // offset in memory) and, in bits of `ok`, whether there is one: axis z 0..2, x
+  // 3..5, y 6..8.  (Formed per tap, index arithmetic was most of a narrow layer:
+  // 6 to 3 channels on 49x97x49 nodes 43.9 us, 35.8 now.)
+  int64_t oz[3], ox[3], oy[3];
+  uint32_t ok;
+  auto node = [&](int64_t o) {
+    o = o < nres ? o : nres - 1;
+    int X, Y, Z;
+    if (nres < (int64_t(1) << 31)) {  // 32-bit divisions
+      const uint32_t u = uint32_t(o), line = u / uint32_t(ry);
+      Y = int(u - line * uint32_t(ry));
+      Z = int(line / uint32_t(rx));
+      X = int(line - uint32_t(Z) * uint32_t(rx));
     } else {
-      z = stride * Z + tap_dz(t); x = stride * X + tap_dx(t); y = stride * Y + tap_dy(t);
-      ok = z >= 0 && z < sz && x >= 0 && x < sx && y >= 0 && y < sy;
+      Y = int(o % ry); X = int((o / ry) % rx); Z = int(o / (int64_t(ry) * rx));
     }
-    p = src + (ok ? (int64_t(z) * sx + x) * sy + y : 0);
-    return ok;
+    ok = 0;
+    auto axis = [&](int a, int r, int n, int64_t step, int64_t (&off)[3]) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const int at = BWD ? r - (d - 1) : stride * r + d - 1;
+        const int s = BWD && stride == 2 ? at >> 1 : at;
+        const bool in = at >= 0 && s < n && !(BWD && stride == 2 && (at & 1));
+        off[d] = s * step;
+        ok |= uint32_t(in) << (3 * a + d);
+      }
+    };
+    axis(0, Z, sz, int64_t(sx) * sy, oz);
+    axis(1, X, sx, sy, ox);
+    axis(2, Y, sy, 1, oy);
+  };
+  auto pick = [](const int64_t (&v)[3], int d) { return d == 0 ? v[0] : (d == 1 ? v[1] : v[2]); };
+  // tap t's source node; false where there is none
+  auto source = [&](int t, const float*& p) {
+    const int a = t / 9, b = t / 3 % 3, c = t % 3;
+    const uint32_t m = (1u << a) | (8u << b) | (64u << c);
+    const bool in = (ok & m) == m;
+    const int64_t off = pick(oz, a) + pick(ox, b) + pick(oy, c);
+    p = src + (in ? off : 0);
+    return in;
   };
   // source values of tap t for the lane's node (0 where the tap has none)
-  auto load = [&](int t, int Z, int X, int Y, float (&v)[NG]) {
+  auto load = [&](int t, float (&v)[NG]) {
     const float* p;
-    const bool ok = source(t, Z, X, Y, p);
+    const bool in = source(t, p);
 #pragma unroll
     for (int q = 0; q < NG; ++q) {
       const int c = 4 * q + g;
       v[q] = p[int64_t(c < kc ? c : 0) * nsrc];
-      v[q] = ok && c < kc ? v[q] : 0.f;
+      v[q] = in && c < kc ? v[q] : 0.f;
     }
   };
   auto product = [&](int t, const float (&v)[NG], nn_f4& acc) {
@@ -119,18 +145,14 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
       acc = __builtin_amdgcn_mfma_f32_16x16x4f32(float(wt[q * 64]), v[q], acc, 0, 0, 0);
   };
   // the same sums of the lane's four results without the terms that have no source
-  auto skip_product = [&](int t, int Z, int X, int Y, nn_f4& acc) {
+  auto skip_product = [&](int t, nn_f4& acc) {
     const float* p;
-    if (!source(t, Z, X, Y, p)) return;
+    if (!source(t, p)) return;
     const _Float16* wt = wl + t * TP + 4 * g;
     for (int c = 0; c < kc; ++c)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         acc[i] = fmaf(float(wt[c * 16 + i]), p[int64_t(c) * nsrc], acc[i]);
-  };
-  auto node = [&](int64_t o, int& Z, int& X, int& Y) {
-    o = o < nres ? o : nres - 1;
-    Y = int(o % ry); X = int((o / ry) % rx); Z = int(o / (int64_t(ry) * rx));
   };
   auto store = [&](int m, int64_t o, float v) {
     if (m >= mc || o >= nres) return;
@@ -145,29 +167,28 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
   if (special) {
     for (int tile = int(blockIdx.x) * CW + wave; tile < ntiles; tile += int(gridDim.x) * CW) {
       const int64_t o = int64_t(tile) * 16 + j;
-      int Z, X, Y;
-      node(o, Z, X, Y);
+      node(o);
       nn_f4 acc{0.f, 0.f, 0.f, 0.f};
-      for (int t = 0; t < 27; ++t) skip_product(t, Z, X, Y, acc);
+      for (int t = 0; t < 27; ++t) skip_product(t, acc);
 #pragma unroll
       for (int i = 0; i < 4; ++i) store(m0 + 4 * g + i, o, acc[i]);
     }
     return;
   }
-  if constexpr (!BWD) {
+  if constexpr (!SPLIT) {
     // a wave per node tile, all taps in order: the sum of every output keeps
     // the order of a loop over taps and source channels
     for (int tile = int(blockIdx.x) * CW + wave; tile < ntiles; tile += int(gridDim.x) * CW) {
       const int64_t o = int64_t(tile) * 16 + j;
-      int Z, X, Y;
-      node(o, Z, X, Y);
+      node(o);
       nn_f4 acc{0.f, 0.f, 0.f, 0.f};
-      for (int t = 0; t < 27; t += 3) {
-        float v[3][NG];
+#pragma unroll NG <= 4 ? 27 / TB : 1
+      for (int t = 0; t < 27; t += TB) {
+        float v[TB][NG];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) load(t + q, Z, X, Y, v[q]);
+        for (int q = 0; q < TB; ++q) load(t + q, v[q]);
 #pragma unroll
-        for (int q = 0; q < 3; ++q) product(t + q, v[q], acc);
+        for (int q = 0; q < TB; ++q) product(t + q, v[q], acc);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) store(m0 + 4 * g + i, o, acc[i]);
@@ -176,12 +197,11 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
     // the waves share a node tile, taps in turn, sums added through LDS
     __shared__ float red[CW][16][16];
     for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-      int Z, X, Y;
-      node(int64_t(tile) * 16 + j, Z, X, Y);
+      node(int64_t(tile) * 16 + j);
       nn_f4 acc{0.f, 0.f, 0.f, 0.f};
       for (int t = wave; t < 27; t += CW) {
         float v[NG];
-        load(t, Z, X, Y, v);
+        load(t, v);
         product(t, v, acc);
       }
 #pragma unroll
@@ -199,10 +219,73 @@ __global__ __launch_bounds__(CT) void conv_kernel(int kc, int mc, int rz, int rx
   }
 }
 
+// One source channel on a large grid: a thread per node and 8 result channels,
+// taps in order (a tap without a source node is skipped).  The matrix tile would
+// have three of its four source channels empty and most of its 16 rows.
+constexpr int NR = 8;
+template <bool BWD>
+__global__ __launch_bounds__(BS) void conv_one_kernel(int mc, int rz, int rx, int ry, int sz, int sx,
+                                                      int sy, int stride, int relu, int accumulate,
+                                                      const float* __restrict__ src,
+                                                      const _Float16* __restrict__ w,
+                                                      const float* __restrict__ bias,
+                                                      float* __restrict__ out) {
+  __shared__ float wl[27][NR];
+  const int m0 = int(blockIdx.y) * NR;
+  for (int i = threadIdx.x; i < 27 * NR; i += BS)
+    wl[i % 27][i / 27] = m0 + i / 27 < mc ? float(w[int64_t(m0) * 27 + i]) : 0.f;
+  __syncthreads();
+  const int64_t nres = int64_t(rz) * rx * ry;
+  const int64_t o = int64_t(blockIdx.x) * BS + threadIdx.x;
+  if (o >= nres) return;
+  const int Y = int(o % ry), X = int((o / ry) % rx), Z = int(o / (int64_t(ry) * rx));
+  float acc[NR];
+#pragma unroll
+  for (int k = 0; k < NR; ++k) acc[k] = 0.f;
+#pragma unroll
+  for (int t = 0; t < 27; ++t) {
+    int z, x, y;
+    if constexpr (BWD) {
+      const int pz = Z - tap_dz(t), px = X - tap_dx(t), py = Y - tap_dy(t);
+      if (stride == 2 && ((pz | px | py) & 1)) continue;
+      z = stride == 2 ? pz >> 1 : pz; x = stride == 2 ? px >> 1 : px; y = stride == 2 ? py >> 1 : py;
+    } else {
+      z = stride * Z + tap_dz(t); x = stride * X + tap_dx(t); y = stride * Y + tap_dy(t);
+    }
+    if (z < 0 || z >= sz || x < 0 || x >= sx || y < 0 || y >= sy) continue;
+    const float v = src[(int64_t(z) * sx + x) * sy + y];
+#pragma unroll
+    for (int k = 0; k < NR; ++k) acc[k] = fmaf(wl[t][k], v, acc[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < NR; ++k) {
+    if (m0 + k >= mc) break;
+    float* dst = out + int64_t(m0 + k) * nres + o;
+    if constexpr (BWD) {
+      *dst = accumulate ? *dst + acc[k] : acc[k];
+    } else {
+      const float v = acc[k] + bias[m0 + k];
+      *dst = relu ? fmaxf(v, 0.f) : v;
+    }
+  }
+}
+
 // Workgroups per 16 result channels: a workgroup stages up to 55 KB of weights
 // before its first tile, so beyond two rounds of the chip (two workgroups of
 // that size per CU) a workgroup takes several tiles.
 constexpr int64_t kConvGroups = 1024;
+// The data gradient's waves share a node tile while there are fewer (node,
+// channel) tiles than about half the SIMDs, and with more source channels a
+// little longer, which take a wave of its own more time (16 source channels:
+// 265 tiles 10.6 us shared, 14.3 a wave each, 977 tiles 17.3 and 12.5; 64 source
+// channels: 530 tiles 33.2 and 39.1, 977 tiles 42.8 and 38.9).  Shared on every
+// grid it took 92 us for 6 source and 3 result channels on 49x97x49 nodes, 35
+// now.
+constexpr int64_t conv_split(int kc) { return kc > 16 ? 768 : 512; }
+// Node tiles from which one source channel takes a thread per node (1 result
+// channel forward: 4,424 tiles 11.4 us on the matrix cores; 14,557 tiles 22.4 and
+// 8.2).
+constexpr int64_t kConvOne = 4096;
 
 template <bool BWD>
 int conv_launch(int kc, int mc, int rz, int rx, int ry, int sz, int sx, int sy, int stride,
@@ -210,13 +293,28 @@ int conv_launch(int kc, int mc, int rz, int rx, int ry, int sz, int sx, int sy, 
                 const float* bias, float* out, void* stream) {
   const int64_t ntiles = (int64_t(rz) * rx * ry + 15) / 16, mt = (mc + 15) / 16;
   TL_ARG(ntiles < (int64_t(1) << 31) && mt < 65536, "grid too large for the convolution");
-  const int64_t groups = BWD ? ntiles : (ntiles + CW - 1) / CW;
-  const int64_t gx = std::min<int64_t>(groups, kConvGroups / std::min<int64_t>(mt, 4));
-  auto go = [&](auto ng) {
-    hipLaunchKernelGGL((conv_kernel<BWD, decltype(ng)::value>), dim3(unsigned(gx), unsigned(mt)),
-                       dim3(CT), 0, static_cast<hipStream_t>(stream), kc, mc, rz, rx, ry, sz, sx, sy,
-                       stride, relu, accumulate, int(ntiles), src,
+  if (kc == 1 && mc <= 64 && ntiles >= kConvOne) {
+    const dim3 grid(unsigned((int64_t(rz) * rx * ry + BS - 1) / BS), unsigned((mc + NR - 1) / NR));
+    hipLaunchKernelGGL(conv_one_kernel<BWD>, grid, dim3(BS), 0, static_cast<hipStream_t>(stream), mc,
+                       rz, rx, ry, sz, sx, sy, stride, relu, accumulate, src,
                        reinterpret_cast<const _Float16*>(w16), bias, out);
+    TL_CHECK_LAUNCH();
+    return TL_OK;
+  }
+  const bool split = BWD && ntiles * mt < conv_split(kc);
+  const int64_t groups = split ? ntiles : (ntiles + CW - 1) / CW;
+  const int64_t gx = std::min<int64_t>(groups, kConvGroups / std::min<int64_t>(mt, 4));
+  auto launch = [&](auto sp, auto ng) {
+    constexpr int NG = decltype(ng)::value;
+    hipLaunchKernelGGL((conv_kernel<BWD, decltype(sp)::value, NG, NG <= 4 ? 9 : 3>),
+                       dim3(unsigned(gx), unsigned(mt)), dim3(CT), 0,
+                       static_cast<hipStream_t>(stream), kc, mc, rz, rx, ry, sz, sx, sy, stride, relu,
+                       accumulate, int(ntiles), src, reinterpret_cast<const _Float16*>(w16), bias, out);
+  };
+  auto go = [&](auto ng) {
+    if constexpr (BWD)
+      if (split) return launch(std::true_type{}, ng);
+    launch(std::false_type{}, ng);
   };
   if (kc <= 4) go(std::integral_constant<int, 1>{});
   else if (kc <= 8) go(std::integral_constant<int, 2>{});
