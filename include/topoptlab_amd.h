@@ -277,7 +277,8 @@ typedef struct {
  * for iter <= 2).  xmin, xmax (device n) may be NULL: 0 and 1.  df0dx, dfdx
  * (device n): objective and constraint gradients; fval: constraint value.
  * *newton_its (may be NULL): Newton steps of the subproblem.  Synchronises
- * the stream (the subproblem's scalars live on the host). */
+ * the stream (the subproblem's scalars live on the host).  The work vectors
+ * are shared per device; concurrent host threads are serialised by a lock. */
 int tl_mma_update(int64_t n, double* x, const double* xold1, const double* xold2,
                   const double* xmin, const double* xmax, const double* df0dx, double fval,
                   const double* dfdx, double* low, double* upp, int32_t iter,

@@ -272,6 +272,49 @@ def test_mma_sizes(gpu, it, n):
     check(gpu, it, n)
 
 
+def test_mma_threads(gpu):
+    """Two host threads on streams of their own, designs of different sizes:
+    each step's design and asymptotes are the ones of the step done alone."""
+    import threading
+    import torch
+    from topoptlab_amd.optimizer import mma_defaultkws, mma_update
+    say("mma threads")
+    probs = []
+    for n in (3001, 40000):
+        rng = np.random.default_rng(n)
+        t = lambda a: torch.as_tensor(a, device=gpu)
+        probs.append((t(0.05 + 0.9 * rng.random(n)), t(-10.0 ** rng.uniform(-4, 1, n)),
+                      torch.full((n,), 1.0 / n, dtype=torch.float64, device=gpu)))
+
+    def step(x, dc, dv):
+        kw = mma_defaultkws(x.numel(), 1, device=gpu)
+        return [mma_update(x, None, None, dc, 0.01, dv, kw, iter=0), kw["low"], kw["upp"]]
+
+    want = [step(*p) for p in probs]
+    torch.cuda.synchronize()
+    got, errs = [[], []], []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream(device=gpu)):
+                for _ in range(8):
+                    got[i].append(step(*probs[i]))
+                torch.cuda.current_stream().synchronize()
+        except Exception as e:  # shown by the assertion below
+            errs.append(e)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not errs, errs
+    for i in range(2):
+        assert len(got[i]) == 8
+        for res in got[i]:
+            assert all(torch.equal(a, b) for a, b in zip(res, want[i]))
+
+
 # cycles whose first sweep, correction and scalars are formed inside the
 # operators: 2D node lines (up to 63 nodes in y) and tiles (from 64 on), one
 # node line of many workgroups; tiled 3D operators with 16, 17 and 31 nodes

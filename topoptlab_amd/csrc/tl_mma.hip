@@ -30,6 +30,7 @@
 #include <atomic>
 #include <chrono>
 #include <cmath>
+#include <mutex>
 
 namespace tl {
 namespace {
@@ -40,7 +41,11 @@ constexpr int NR = 5;        // reduced values per pass
 // produce (its results carry the canonical payload or an input's).
 constexpr uint64_t kEmpty = 0x7ff8a5a5c3c35a5aull;
 
+// One per device, for all callers: the mutex is held for the whole call, which
+// ends with a stream synchronisation, so that no caller resizes the vectors
+// under another's kernels or empties the slots that another one polls.
 struct MmaWork {
+  std::mutex mu;
   DevBuf vec, partials;
   // the folded values, written by the fold kernel straight into pinned,
   // coherent host memory; two sets in turn
@@ -267,6 +272,7 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
   TL_ARG(o->move > 0.0 && o->asyinit > 0.0 && o->albefa > 0.0 && o->albefa < 1.0,
          "MMA parameters out of range");
   MmaWork& W = work_for_device();
+  std::lock_guard<std::mutex> lock(W.mu);
   TL_TRY(W.ensure(n));
   hipStream_t s = static_cast<hipStream_t>(stream);
   double* base = W.vec.as<double>();
@@ -301,6 +307,10 @@ extern "C" int tl_mma_update(int64_t n, double* x, const double* xold1, const do
           synced = true;
         }
         bits = q[k];
+      }
+      if (bits == kEmpty) {
+        set_error("MMA: a folded value has not arrived");
+        return TL_EHIP;
       }
       std::memcpy(&h[k], &bits, sizeof(double));
     }
