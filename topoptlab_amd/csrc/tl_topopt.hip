@@ -210,6 +210,8 @@ __device__ __forceinline__ void oc_decide(OcState& st, double lmid, double gt) {
   if (!((st.l2 - st.l1) / (st.l1 + st.l2) > 1e-3)) st.done = 1;
 }
 
+constexpr int kOcSteps = 400;  // a bisection that has not ended by then is refused
+
 // Designs of up to kOcSmall elements: the whole bisection in one workgroup,
 // eight elements per thread in registers.  A step is one evaluation and one
 // block sum (about 2 us) where two launches per step cost 5.3 us of kernel
@@ -241,7 +243,7 @@ __global__ __launch_bounds__(1024) void oc_small_kernel(const double* __restrict
     }
   }
   const int ne = (n + bs - 1) / bs;
-  while (!st.done && st.steps < 400) {
+  while (!st.done && st.steps < kOcSteps) {
     const double lmid = 0.5 * (st.l2 + st.l1);
     double v[2] = {0.0, 0.0};
 #pragma unroll
@@ -333,7 +335,7 @@ __global__ __launch_bounds__(512) void oc_fold_kernel(const double* __restrict__
   __syncthreads();
   if (threadIdx.x == 0) {
     OcState st = *stp;
-    for (int j = 0, at = 0; j < 3 && !st.done; ++j) {
+    for (int j = 0, at = 0; j < 3 && !st.done && st.steps < kOcSteps; ++j) {
       const double gt = st.g + tot[at];
       oc_decide(st, 0.5 * (st.l2 + st.l1), gt);
       at = 2 * at + (gt > 0 ? 2 : 1);
@@ -441,7 +443,7 @@ int oc_bisect(int64_t n, const double* x, const double* dc, const double* dv,
     const unsigned nb =
         unsigned(std::min<int64_t>((n + kOcThreads - 1) / kOcThreads, kOcBlocks));
     // 48 steps before the first look at the state, then 12 at a time
-    for (int pass = 0, batch = 16; pass * 3 < 400; batch = 4) {
+    for (int pass = 0, batch = 16; pass * 3 < kOcSteps; batch = 4) {
       for (int k = 0; k < batch; ++k, ++pass) {
         hipLaunchKernelGGL(oc_pass_kernel, dim3(nb), dim3(kOcThreads), 0, s, x, dc, dv, el_flags, n,
                            st, partials, kOcBlocks);
