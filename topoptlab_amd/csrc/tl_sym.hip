@@ -15,7 +15,13 @@
 // scales, and in the same basis sum_m t_m B_m with t the Hadamard transform of
 // the child scales and B_m constant: 279 nonzeros together.  Applying it from
 // the densities reads about 25 MB at 192x96x96 in FP64 where the stored
-// half-stencil reads 252 MB.
+// half-stencil reads 252 MB.  Its arithmetic is FP64 in the FP32 cycles too
+// (vectors in FP32): the coefficients of a stored FP32 stencil are FP64 sums
+// rounded once, and formed in FP32 from FP32 scales they had up to a tenth more
+// error on rough fields (white noise, scales over nine decades: stored 8.4e-8,
+// FP32 9.1e-8, FP64 2.6e-8 with the output's rounding; on nearly constant fields
+// 1e-5, 2e-6 and 2.5e-8).  It costs a third: at 192x96x96 residual 12.6 -> 16.3
+// us, sweep 11.6 -> 15.9, sweep with the correction 15.9 -> 23.2.
 //
 // A workgroup owns a 16x16 tile of element columns (thread (tx, ty): element
 // column (X0 + tx - 1, Y0 + ty - 1), y fastest) and walks a range of element
@@ -46,7 +52,12 @@ static_assert(TE * TE == BS, "one element column per thread");
 constexpr int TC = 10;  // coarse nodes per tile side that 17 staged nodes interpolate from
 constexpr int CR = 4;   // coarse tiles kept in LDS
 
-template <typename T>
+// Arithmetic of an operator with vectors of type T.
+template <typename T, bool CG>
+using sym_arith = std::conditional_t<CG, double, T>;
+
+// T: vectors, A: arithmetic
+template <typename T, typename A>
 struct SymArgs {
   const T* u;          // input; SRC_P: z
   const T* pin;        // SRC_P: previous search direction
@@ -56,7 +67,7 @@ struct SymArgs {
   FoldIn rr;           // SRC_SEED: partials of r.r of the iteration before, or none
   const T* xc;         // SRC_*CORR: the coarse level's correction
   int cnx, cny, cnz;   // and its node counts
-  const T* sp;         // zero-bordered scales of the fine grid
+  const A* sp;         // zero-bordered scales of the fine grid
   const uint8_t* mask;
   const void* b;       // KU_RESID / KU_JACOBI*: right-hand side
   const T* dinv;
@@ -69,8 +80,8 @@ struct SymArgs {
   int ncy;                           // tile columns along y
   unsigned ncol;                     // tile columns
   unsigned nseg;                     // equal z ranges per column, or 0 (see sym_segments)
-  T kv[16];                          // group values of the pattern
-  T kt;                              // products: stiffness against a translation
+  A kv[16];                          // group values of the pattern
+  A kt;                              // products: stiffness against a translation
 };
 
 template <int NDPN, bool CG>
@@ -127,10 +138,11 @@ __device__ __forceinline__ void child_modes(T (&t)[8]) {
 
 // Element scales of the thread's column in one layer: the element's own
 // (fine) or its children's modes (CG).
-template <typename T, bool CG>
+template <typename A, bool CG>
 struct Scales {
-  T s[CG ? 8 : 1];
-  __device__ __forceinline__ void load(const SymArgs<T>& a, int ix, int iy, int ez) {
+  A s[CG ? 8 : 1];
+  template <typename T>
+  __device__ __forceinline__ void load(const SymArgs<T, A>& a, int ix, int iy, int ez) {
     if constexpr (CG) {
       // element (ix - 1, iy - 1, ez); zero outside the grid
       const bool in = ix >= 1 && ix <= a.nelx && iy >= 1 && iy <= a.nely && ez >= 0 && ez < a.nelz;
@@ -140,8 +152,8 @@ struct Scales {
       for (int k = 0; k < 8; ++k) {
         const int64_t i = (int64_t(2 * cz + (k >> 2) + 1) * (a.fnelx + 2) + 2 * cx - 1 + (k >> 1 & 1)) *
                               (a.fnely + 2) + 2 * cy - 1 + (k & 1);
-        const T v = a.sp[i];
-        s[k] = in ? v : T(0);
+        const A v = a.sp[i];
+        s[k] = in ? v : A(0);
       }
     } else {
       // the border of the padded array holds zeros
@@ -165,30 +177,30 @@ struct Scales {
 // solution: without it a 120x20x12 solve differs by 9e-9 from one with the
 // matrix as given.  12 operations per element: 95x61x47 product 15.6 -> 16.1 us,
 // 192x96x96 solve 28.3 -> 28.0 ms.
-template <int NDPN, typename T, bool CG, bool TR>
-__device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, CG>& S,
-                                          const T (&flo)[4 * NDPN], const T (&fhi)[4 * NDPN],
-                                          T (&tot)[4 * NDPN], T (&up)[4 * NDPN]) {
+template <int NDPN, typename T, typename A, bool CG, bool TR>
+__device__ __forceinline__ void sym_layer(const SymArgs<T, A>& a, const Scales<A, CG>& S,
+                                          const A (&flo)[4 * NDPN], const A (&fhi)[4 * NDPN],
+                                          A (&tot)[4 * NDPN], A (&up)[4 * NDPN]) {
   constexpr int ND = 8 * NDPN;
-  T U[ND];
+  A U[ND];
 #pragma unroll
   for (int i = 0; i < 4 * NDPN; ++i) {
     U[i] = flo[i] + fhi[i];
     U[4 * NDPN + i] = flo[i] - fhi[i];
   }
-  T ks[16];  // fine: the group values times the element's scale
+  A ks[16];  // fine: the group values times the element's scale
   if constexpr (!CG) {
 #pragma unroll
     for (int g = 0; g < (NDPN == 3 ? kGroupsSym_elast : kGroupsSym_poisson); ++g) ks[g] = S.s[0] * a.kv[g];
   }
 #pragma unroll
   for (int i = 0; i < 4 * NDPN; ++i) {
-    T y[2];
+    A y[2];
     bool any[2] = {false, false};
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int m = 4 * h + i / NDPN, c = i % NDPN, r = m * NDPN + c;
-      y[h] = T(0);
+      y[h] = A(0);
       if (TR && m == 0) {
         y[h] = S.s[0] * a.kt * U[r];
         any[h] = true;
@@ -199,7 +211,7 @@ __device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, C
           const int col = sym_mode<NDPN>(sym_class<NDPN>(m, c), k) * NDPN + k;
           const int p = sym_tab<NDPN, false>(r * ND + col);
           if (p == 0) continue;
-          const T v = ks[(p > 0 ? p : -p) - 1];
+          const A v = ks[(p > 0 ? p : -p) - 1];
           if (!any[h]) y[h] = p > 0 ? v * U[col] : -v * U[col];
           else y[h] = sym_fma(p > 0 ? v : -v, U[col], y[h]);
           any[h] = true;
@@ -207,14 +219,14 @@ __device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, C
       } else {
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
-          T t = T(0);
+          A t = A(0);
           bool anyq = false;
 #pragma unroll
           for (int k = 0; k < NDPN; ++k) {
             const int col = sym_mode<NDPN>(sym_class<NDPN>(m, c) ^ q, k) * NDPN + k;
             const int p = sym_tab<NDPN, true>((q * ND + r) * ND + col);
             if (p == 0) continue;
-            const T v = a.kv[(p > 0 ? p : -p) - 1];
+            const A v = a.kv[(p > 0 ? p : -p) - 1];
             if (!anyq) t = p > 0 ? v * U[col] : -v * U[col];
             else t = sym_fma(p > 0 ? v : -v, U[col], t);
             anyq = true;
@@ -244,7 +256,7 @@ __device__ __forceinline__ void sym_layer(const SymArgs<T>& a, const Scales<T, C
 // (`ring`, plane z at z % CR, already interpolated in z): in a direction with
 // an even coordinate both neighbours are the coinciding coarse node, so one
 // average serves every case.
-template <int NDPN, typename T, typename TB, int SRC>
+template <int NDPN, typename T, typename A, typename TB, int SRC>
 struct Stage {
   static constexpr int N = TS * TS * NDPN, NR = (N + BS - 1) / BS;
   static constexpr bool kTwo = SRC == SRC_P || src_seed(SRC), kCorr = src_corr(SRC);
@@ -258,7 +270,7 @@ struct Stage {
     int z;                       // the plane asked for (past the grid: the last one is held)
   };
   __device__ __forceinline__ bool has(int k) const { return k + 1 < NR || int(threadIdx.x) + k * BS < N; }
-  __device__ __forceinline__ void init(const SymArgs<T>& a, int x0, int y0) {
+  __device__ __forceinline__ void init(const SymArgs<T, A>& a, int x0, int y0) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
       const int e = int(threadIdx.x) + k * BS;
@@ -271,7 +283,7 @@ struct Stage {
     }
   }
   __device__ __forceinline__ static int coarse_base(int x0) { return max(x0 - 1, 0) >> 1; }
-  __device__ __forceinline__ void load(const SymArgs<T>& a, int z, Vals& q) const {
+  __device__ __forceinline__ void load(const SymArgs<T, A>& a, int z, Vals& q) const {
     q.z = z;
     const int64_t base = int64_t(min(max(z, 0), a.nz - 1)) * a.nx * a.ny * NDPN;
     const V* p = (src_seed(SRC) ? static_cast<const V*>(a.b) : reinterpret_cast<const V*>(a.u)) + base;
@@ -291,12 +303,12 @@ struct Stage {
         if (has(k)) q.mk[k] = m[off[k] / NDPN];
     }
   }
-  __device__ __forceinline__ T value(const SymArgs<T>& a, int k, const Vals& q, T beta) const {
+  __device__ __forceinline__ T value(const SymArgs<T, A>& a, int k, const Vals& q, T beta) const {
     if constexpr (SRC == SRC_P) return T(q.v[k]) + beta * q.w[k];
     else if constexpr (src_seed(SRC)) return zero_guess_sweep<T, TB>(a.omega, q.w[k], q.v[k]);
     else return q.v[k];
   }
-  __device__ __forceinline__ void store(const SymArgs<T>& a, T* lds, const T* ring, T beta,
+  __device__ __forceinline__ void store(const SymArgs<T, A>& a, T* lds, const T* ring, T beta,
                                         const Vals& q) const {
 #pragma unroll
     for (int k = 0; k < NR; ++k)
@@ -316,20 +328,20 @@ struct Stage {
 // The thread's entries of the coarse 10x10 tiles (clamped to the grid).  Fine
 // plane z interpolates from coarse planes z/2 and (z+1)/2; `next` holds the
 // latter of the plane prepared last.
-template <int NDPN, typename T>
+template <int NDPN, typename T, typename A>
 struct CoarseStage {
   static constexpr int N = TC * TC * NDPN, NR = (N + BS - 1) / BS;
   uint32_t off[NR];
   T cur[NR], next[NR];
   __device__ __forceinline__ bool has(int k) const { return int(threadIdx.x) + k * BS < N; }
-  __device__ __forceinline__ void load(const SymArgs<T>& a, int c, T (&v)[NR]) const {
+  __device__ __forceinline__ void load(const SymArgs<T, A>& a, int c, T (&v)[NR]) const {
     const T* p = a.xc + int64_t(min(c, a.cnz - 1)) * a.cnx * a.cny * NDPN;
 #pragma unroll
     for (int k = 0; k < NR; ++k)
       if (has(k)) v[k] = p[off[k]];
   }
   // Tiles of planes z0 - 1 (if any) to z0 + 2.
-  __device__ __forceinline__ void begin(const SymArgs<T>& a, int x0, int y0, int z0, T* ring) {
+  __device__ __forceinline__ void begin(const SymArgs<T, A>& a, int x0, int y0, int z0, T* ring) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
       const int e = int(threadIdx.x) + k * BS;
@@ -360,7 +372,7 @@ struct CoarseStage {
       if (has(k)) ring[(z % CR) * N + threadIdx.x + k * BS] = T(0.5) * (lo[k] + hi[k]);
   }
   // Start of the step that prepares plane z, and its end.
-  __device__ __forceinline__ void advance(const SymArgs<T>& a, int z) {
+  __device__ __forceinline__ void advance(const SymArgs<T, A>& a, int z) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) cur[k] = next[k];
     if (z & 1) load(a, (z + 1) >> 1, next);
@@ -370,26 +382,26 @@ struct CoarseStage {
 
 // In-plane modes of the thread's element from the staged plane, and the value
 // of its own output node (the element's corner (1, 1)).
-template <int NDPN, typename T>
-__device__ __forceinline__ void plane_modes(const T* lds, int tx, int ty, T (&f)[4 * NDPN],
+template <int NDPN, typename T, typename A>
+__device__ __forceinline__ void plane_modes(const T* lds, int tx, int ty, A (&f)[4 * NDPN],
                                             T (&uc)[NDPN]) {
   const T* p = lds + (tx * TS + ty) * NDPN;
 #pragma unroll
   for (int c = 0; c < NDPN; ++c) {
-    const T v00 = p[c], v01 = p[NDPN + c], v10 = p[TS * NDPN + c], v11 = p[(TS + 1) * NDPN + c];
-    const T a = v00 + v01, b = v00 - v01, d = v10 + v11, e = v10 - v11;
+    const A v00 = p[c], v01 = p[NDPN + c], v10 = p[TS * NDPN + c], v11 = p[(TS + 1) * NDPN + c];
+    const A a = v00 + v01, b = v00 - v01, d = v10 + v11, e = v10 - v11;
     f[c] = a + d;
     f[NDPN + c] = a - d;
     f[2 * NDPN + c] = b + e;
     f[3 * NDPN + c] = b - e;
-    uc[c] = v11;
+    uc[c] = T(v11);
   }
 }
 
 // Node planes z0 .. z1-1 of tile column col.
-template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
-__device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS * TS * NDPN],
-                                            T (*xch)[NDPN * BS], T* ring, unsigned col, int z0,
+template <int NDPN, typename T, typename A, int MODE, typename TB, typename TO, int SRC, bool CG>
+__device__ __forceinline__ void sym_segment(const SymArgs<T, A>& a, T (*plane)[TS * TS * NDPN],
+                                            A (*xch)[NDPN * BS], T* ring, unsigned col, int z0,
                                             int z1, T beta, double& dot) {
   constexpr bool CORR = src_corr(SRC), kTrans = MODE == KU_STORE || MODE == KU_STORE_DOT;
   const int tid = int(threadIdx.x), tx = tid >> 4, ty = tid & 15;
@@ -398,13 +410,14 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
   const bool active = tx < TN && ty < TN && ix < a.nx && iy < a.ny;
   const int64_t node0 = active ? int64_t(ix) * a.ny + iy : 0;
   const int64_t nplane = int64_t(a.nx) * a.ny;
-  Stage<NDPN, T, TB, SRC> st;
-  CoarseStage<NDPN, T> cs;
-  Scales<T, CG> S, Sn;
-  T flo[4 * NDPN], uc[NDPN], carry[4 * NDPN];
+  Stage<NDPN, T, A, TB, SRC> st;
+  CoarseStage<NDPN, T, A> cs;
+  Scales<A, CG> S, Sn;
+  A flo[4 * NDPN], carry[4 * NDPN];
+  T uc[NDPN];
   // (planes z0 - 1, z0 and z0 + 1 requested together: product and residual 3 us
   // slower at 192x96x96)
-  typename Stage<NDPN, T, TB, SRC>::Vals in;
+  typename Stage<NDPN, T, A, TB, SRC>::Vals in;
   st.init(a, x0, y0);
   st.load(a, z0, in);
   S.load(a, ix, iy, z0);
@@ -415,25 +428,26 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
   }
   st.store(a, plane[z0 & 1], ring, beta, in);
 #pragma unroll
-  for (int i = 0; i < 4 * NDPN; ++i) carry[i] = T(0);
+  for (int i = 0; i < 4 * NDPN; ++i) carry[i] = A(0);
   if (z0 > 0) {  // the layer below gives plane z0's lower part
-    Scales<T, CG> Sb;
+    Scales<A, CG> Sb;
     st.load(a, z0 - 1, in);
     Sb.load(a, ix, iy, z0 - 1);
     st.store(a, plane[(z0 + 1) & 1], ring, beta, in);
     st.load(a, z0 + 1, in);
     __syncthreads();
-    T fb[4 * NDPN], unused[4 * NDPN], ub[NDPN];
-    plane_modes<NDPN, T>(plane[(z0 + 1) & 1], tx, ty, fb, ub);
-    plane_modes<NDPN, T>(plane[z0 & 1], tx, ty, flo, uc);
+    A fb[4 * NDPN], unused[4 * NDPN];
+    T ub[NDPN];
+    plane_modes<NDPN, T, A>(plane[(z0 + 1) & 1], tx, ty, fb, ub);
+    plane_modes<NDPN, T, A>(plane[z0 & 1], tx, ty, flo, uc);
 #pragma unroll
-    for (int i = 0; i < 4 * NDPN; ++i) unused[i] = T(0);
+    for (int i = 0; i < 4 * NDPN; ++i) unused[i] = A(0);
     Sb.modes();
-    sym_layer<NDPN, T, CG, kTrans>(a, Sb, fb, flo, unused, carry);
+    sym_layer<NDPN, T, A, CG, kTrans>(a, Sb, fb, flo, unused, carry);
   } else {
     st.load(a, z0 + 1, in);
     __syncthreads();
-    plane_modes<NDPN, T>(plane[z0 & 1], tx, ty, flo, uc);
+    plane_modes<NDPN, T, A>(plane[z0 & 1], tx, ty, flo, uc);
   }
   if (z0 > 0) __syncthreads();  // plane z0 - 1 has been read
   st.store(a, plane[(z0 + 1) & 1], ring, beta, in);
@@ -456,18 +470,19 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
         bv[c] = static_cast<const TB*>(a.b)[node * NDPN + c];
       if constexpr (MODE == KU_JACOBI || MODE == KU_JACOBI_DOT) dv[c] = a.dinv[node * NDPN + c];
     }
-    T fhi[4 * NDPN], un[NDPN], up[4 * NDPN];
-    plane_modes<NDPN, T>(plane[(z + 1) & 1], tx, ty, fhi, un);
+    A fhi[4 * NDPN], up[4 * NDPN];
+    T un[NDPN];
+    plane_modes<NDPN, T, A>(plane[(z + 1) & 1], tx, ty, fhi, un);
     S.modes();
-    sym_layer<NDPN, T, CG, kTrans>(a, S, flo, fhi, carry, up);
+    sym_layer<NDPN, T, A, CG, kTrans>(a, S, flo, fhi, carry, up);
     // carry now holds plane z's in-plane modes from both layers: corner values,
     // summed over the element columns in y (DPP) and x (LDS)
-    T acc[NDPN];
-    T* xo = xch[z & 1];
+    A acc[NDPN];
+    A* xo = xch[z & 1];
 #pragma unroll
     for (int c = 0; c < NDPN; ++c) {
-      const T p = carry[c] + carry[2 * NDPN + c], q = carry[c] - carry[2 * NDPN + c];
-      const T r = carry[NDPN + c] + carry[3 * NDPN + c], s = carry[NDPN + c] - carry[3 * NDPN + c];
+      const A p = carry[c] + carry[2 * NDPN + c], q = carry[c] - carry[2 * NDPN + c];
+      const A r = carry[NDPN + c] + carry[3 * NDPN + c], s = carry[NDPN + c] - carry[3 * NDPN + c];
       xo[c * BS + tid] = (q + s) + next_lane(p + r);
       acc[c] = (q - s) + next_lane(p - r);
     }
@@ -485,14 +500,14 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
         TO* y = static_cast<TO*>(a.y);
         if constexpr (SRC == SRC_P) a.pout[g] = uc[c];
         if constexpr (MODE == KU_STORE || MODE == KU_STORE_DOT) {
-          const T v = fixed ? T(0) : acc[c];
+          const T v = fixed ? T(0) : T(acc[c]);
           y[g] = TO(v);
           if constexpr (MODE == KU_STORE_DOT) dot += double(uc[c]) * double(v);
         } else if constexpr (MODE == KU_RESID) {
-          y[g] = TO(fixed ? T(0) : T(bv[c]) - acc[c]);
+          y[g] = TO(fixed ? T(0) : T(A(T(bv[c])) - acc[c]));
         } else {
           const T bb = T(bv[c]);
-          const T v = fixed ? T(0) : uc[c] + a.omega * dv[c] * (bb - acc[c]);
+          const T v = fixed ? T(0) : uc[c] + a.omega * dv[c] * T(A(bb) - acc[c]);
           y[g] = TO(v);
           if constexpr (MODE == KU_JACOBI_DOT) dot += double(bb) * double(v);
         }
@@ -509,9 +524,9 @@ __device__ __forceinline__ void sym_segment(const SymArgs<T>& a, T (*plane)[TS *
   }
 }
 
-template <int NDPN, typename T, int SRC, bool CG>
+template <int NDPN, int SRC, bool CG>
 constexpr int sym_waves() {
-  return NDPN == 3 && sizeof(T) == 8 && CG && src_corr(SRC) ? 1 : 2;
+  return NDPN == 3 && CG && src_corr(SRC) ? 1 : 2;
 }
 
 // Split: every column into the same nseg z ranges, a workgroup each, numbered
@@ -539,11 +554,13 @@ constexpr int sym_waves() {
 // Measured and not kept: two layers per loop turn without the register moves
 // (the sweep spills, the rest is unchanged: the moves are not what bounds it).
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
-__global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kernel(SymArgs<T> a) {
+__global__ __launch_bounds__(BS, (sym_waves<NDPN, SRC, CG>())) void sym_kernel(
+    SymArgs<T, sym_arith<T, CG>> a) {
+  using A = sym_arith<T, CG>;
   __shared__ double sh[BS / 64 + 2];
   if (op_ended<SRC == SRC_SEED>(a.rr, a.done, blockIdx.x == 0 && threadIdx.x == 0, sh)) return;
   __shared__ T plane[2][TS * TS * NDPN];
-  __shared__ T xch[2][NDPN * BS];
+  __shared__ A xch[2][NDPN * BS];
   __shared__ T ring[src_corr(SRC) ? CR * TC * TC * NDPN : 1];
   // workgroups go round-robin over the 8 XCDs: give each a contiguous range
   const unsigned nb = gridDim.x, hw = blockIdx.x;
@@ -569,7 +586,7 @@ __global__ __launch_bounds__(BS, (sym_waves<NDPN, T, SRC, CG>())) void sym_kerne
     const unsigned col = u0 / unsigned(a.nz);
     const int z0 = int(u0 - col * unsigned(a.nz));
     const int z1 = min(a.nz, z0 + int(u1 - u0));
-    sym_segment<NDPN, T, MODE, TB, TO, SRC, CG>(a, plane, xch, ring, col, z0, z1, beta, dot);
+    sym_segment<NDPN, T, A, MODE, TB, TO, SRC, CG>(a, plane, xch, ring, col, z0, z1, beta, dot);
     u0 += unsigned(z1 - z0);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
@@ -612,7 +629,7 @@ unsigned sym_segments(int64_t ncol, int64_t nz, int64_t slots) {
 }
 
 template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, bool CG>
-int sym_launch(hipStream_t s, const Grid& g, SymArgs<T> a, unsigned* nblocks) {
+int sym_launch(hipStream_t s, const Grid& g, SymArgs<T, sym_arith<T, CG>> a, unsigned* nblocks) {
   auto* kern = sym_kernel<NDPN, T, MODE, TB, TO, SRC, CG>;
   a.nelx = g.nelx; a.nely = g.nely; a.nelz = g.nelz;
   a.nx = g.nx; a.ny = g.ny; a.nz = g.nz;
@@ -720,7 +737,7 @@ bool sym_fits(const Grid& g, int ndpn) {
 }
 
 template <int NDPN, typename T>
-static int fine_mode(tl_problem* P, const SymArgs<T>& a, int mode, bool b64, int src, unsigned* nb) {
+static int fine_mode(tl_problem* P, const SymArgs<T, T>& a, int mode, bool b64, int src, unsigned* nb) {
   hipStream_t s = P->stream;
   const Grid& g = P->g;
   switch (mode) {
@@ -754,7 +771,7 @@ static int fine_call(tl_problem* P, const void* u, void* y, int mode, const void
                      const void* dinv, double omega, const void* pin, void* pout,
                      const double* beta, const FoldIn& rho, const FoldIn& rr, double* partials,
                      const int* done, unsigned* nb) {
-  SymArgs<T> a{};
+  SymArgs<T, T> a{};
   a.u = static_cast<const T*>(u);
   a.pin = static_cast<const T*>(pin);
   a.pout = static_cast<T*>(pout);
@@ -805,11 +822,10 @@ template <int NDPN, typename T>
 static int coarse_call(tl_problem* P, int mode, const T* x, const T* xc, const T* b, T* y,
                        const int* done) {
   const Level& L = P->mg.lv[1];
-  SymArgs<T> a{};
+  SymArgs<T, double> a{};
   a.u = x;
   a.xc = xc;
-  a.sp = sizeof(T) == 8 ? reinterpret_cast<const T*>(P->op.sp64.ptr)
-                        : reinterpret_cast<const T*>(P->op.sp32.ptr);
+  a.sp = P->op.sp64.as<double>();
   a.mask = L.mask.as<uint8_t>();
   a.b = b;
   a.dinv = reinterpret_cast<const T*>(sizeof(T) == 8 ? L.dinv64.ptr : L.dinv32.ptr);
@@ -818,7 +834,7 @@ static int coarse_call(tl_problem* P, int mode, const T* x, const T* xc, const T
   a.done = done;
   a.fnelx = P->g.nelx;
   a.fnely = P->g.nely;
-  for (int g = 0; g < 16; ++g) a.kv[g] = T(P->mg.symkv[g]);
+  for (int g = 0; g < 16; ++g) a.kv[g] = P->mg.symkv[g];
   hipStream_t s = P->stream;
   if (mode == 0) return sym_launch<NDPN, T, KU_RESID, T, T, SRC_U, true>(s, L.g, a, nullptr);
   if (!xc) return sym_launch<NDPN, T, KU_JACOBI, T, T, SRC_U, true>(s, L.g, a, nullptr);
