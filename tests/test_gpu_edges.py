@@ -391,3 +391,38 @@ def test_solve_ends_alike_within_a_chunk(gpu, dims, ndpn, nlevels):
         again, i3 = op.solve(f, u0=want, rtol=1e-2, check_every=8)
         assert i3["iterations"] == 0 and torch.equal(again, want)
     op.close()
+
+
+def _no_pattern(KE):
+    s = np.random.default_rng(4).uniform(0.9, 1.1, len(KE))
+    return s[:, None] * KE * s
+
+
+# node lines: 1,090 of them, more than a consumer folds partials of; with the
+# unit-cell matrix and with one that matches no pattern
+@pytest.mark.parametrize("dims,ndpn", [((16400, 16, None), 1), ((16400, 16, None), 2),
+                                       ((833, 320, None), 2), ((40, 7, None), 2)])
+@pytest.mark.parametrize("pattern", [True, False])
+def test_node_lines(gpu, dims, ndpn, pattern):
+    """K u (FP64 1e-13, FP32 1e-5) and three diagonal-preconditioned PCG iterates
+    (1e-11), whose product carries the search-direction update and the dot
+    product, against the assembled matrix."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    say("node lines", dims, ndpn, pattern)
+    KE, edof, ndof, fixed, free, x = _problem(dims, ndpn)
+    KE = KE if pattern else _no_pattern(KE)
+    K = fem.apply_bc(fem.assemble_K(KE, edof, fem.simp(x), ndof), free).tocsr()
+    u = np.random.default_rng(1).standard_normal(len(free))
+    op = StiffnessOperator(*dims, KE=KE, fixed=fixed, device=gpu)
+    op.set_density(x)
+    y = K @ u
+    uf = op.full(torch.as_tensor(u, device=gpu))
+    assert rel(op.matvec_full(uf)[op._free_t].cpu().numpy(), y) < 1e-13
+    assert rel(op.matvec_full(uf, "fp32")[op._free_t].cpu().numpy(), y) < 1e-5
+    d = K.diagonal()
+    ref, _, _ = mg.pcg(K, y, lambda r: r / d, rtol=0.0, maxiter=3)
+    got, _ = op.solve(op.full(torch.as_tensor(y, device=gpu)), rtol=0.0, maxiter=3,
+                      preconditioner="jacobi", raise_on_fail=False)
+    assert rel(got[op._free_t].cpu().numpy(), ref) < 1e-11
+    op.close()

@@ -137,7 +137,7 @@ struct KuArgs {
   const int* done;
   int nelx, nely, nelz, nx, ny, nz, plane, ncol;  // ncol: 3D tile columns
   int ty;  // 2D workgroup shape the launch uses (0: node line), for the multi-instance form
-  unsigned nblk;  // 2D: workgroups (each takes tiles bid, bid + nblk, ...)
+  unsigned nblk;  // 2D node tiles: workgroups (each takes tiles bid, bid + nblk, ...)
   // group values of a pattern-matched element matrix (see ke_pattern.hpp)
   double kv64[8];
   float kv32[8];
@@ -192,12 +192,13 @@ __device__ inline void ku_epilogue(const KuArgs& a, int64_t node, const T (&uc)[
   }
 }
 
-// Entry c of 2D node (ix, iy) as the operator's input (SRC_*).  The trilinear
-// correction averages the four coarse nodes around: in a direction with an
-// even coordinate both are the coinciding one.
+// Entry c of a 2D node as the operator's input (SRC_*); its coordinates (ix,
+// iy) are read by the correction only.  The bilinear correction averages the
+// four coarse nodes around: in a direction with an even coordinate both are the
+// coinciding one.
 template <int NDPN, typename T, typename TB, int SRC>
-__device__ inline T stage_val(const KuArgs& a, int ix, int iy, int c, T beta) {
-  const int64_t node = int64_t(ix) * a.ny + iy, g = node * NDPN + c;
+__device__ inline T stage_val(const KuArgs& a, int64_t node, int ix, int iy, int c, T beta) {
+  const int64_t g = node * NDPN + c;
   if constexpr (SRC == SRC_U) return ldval<T>(a.u, g);
   else if constexpr (SRC == SRC_P) return ldval<T>(a.u, g) + beta * ldval<T>(a.pin, g);
   else {
@@ -272,7 +273,10 @@ __device__ inline void node_sum(const KuArgs& a, const T (&U)[3][9][NDPN],
   }
 }
 
-// Nodes j0 - ny - 1 .. j0 + BS + ny of a 2D grid (0 outside it).
+// Nodes j0 - ny - 1 .. j0 + BS + ny of a 2D grid (0 outside it).  A division
+// per entry for the coordinates only where the correction needs them: with one
+// for every source the FP64 product of a 20000x20 elasticity grid took 13.6
+// instead of 12.6 us, of 100000x8 20.6 instead of 19.3.
 template <int NDPN, typename T, typename TB, int SRC>
 __device__ inline void stage_line(const KuArgs& a, T* lds, int64_t j0, T beta) {
   const int L = BS + 2 * a.ny + 2;
@@ -282,8 +286,8 @@ __device__ inline void stage_line(const KuArgs& a, T* lds, int64_t j0, T beta) {
     T v = T(0);
     if (jj >= 0 && jj < a.plane) {
       // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
-      const int ix = int(uint32_t(jj) / uint32_t(a.ny));
-      v = stage_val<NDPN, T, TB, SRC>(a, ix, int(jj) - ix * a.ny, t % NDPN, beta);
+      const int ix = src_corr(SRC) ? int(uint32_t(jj) / uint32_t(a.ny)) : 0;
+      v = stage_val<NDPN, T, TB, SRC>(a, jj, ix, int(jj) - ix * a.ny, t % NDPN, beta);
     }
     lds[t] = v;
   }
@@ -629,42 +633,38 @@ __device__ __forceinline__ void ku2d_body(const KuArgs& a, unsigned bid, T* lds)
   if (op_ended<SRC == SRC_SEED>(a.rr, a.done, bid == 0 && threadIdx.x == 0, sh)) return;
   T beta = T(0);
   if constexpr (SRC == SRC_P) beta = T(fold_in_beta(a.rho, a.beta, bid == 0 && threadIdx.x == 0, sh));
+  const int64_t j0 = int64_t(bid) * BS;
+  const int64_t j = j0 + threadIdx.x;
+  const bool active = j < a.plane;
+  const int64_t jc = active ? j : a.plane - 1;
+  // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
+  const int ix = int(uint32_t(jc) / uint32_t(a.ny)), iy = int(jc) - ix * a.ny;
+  T U[3][9][NDPN];
+  T S[3][4];
+  stage_line<NDPN, T, TB, SRC>(a, lds, j0, beta);
+  // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
+  {
+    const T* sp = static_cast<const T*>(a.sp);
+#pragma unroll
+    for (int ox = -1; ox <= 0; ++ox)
+#pragma unroll
+      for (int oy = -1; oy <= 0; ++oy)
+        S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(ix + ox + 1) * (a.nely + 2) + iy + oy + 1];
+  }
+  __syncthreads();
+  read_nbrs<NDPN, T, 1>(a, lds, U);
+  T acc[NDPN];
+  node_sum<NDPN, T, 0, 1, 2, false, FAST>(a, U, S, 0, 1, acc);
   double dot = 0.0;
-  const unsigned nline = unsigned((int64_t(a.plane) + BS - 1) / BS);
-  for (unsigned tile = bid; tile < nline; tile += a.nblk) {
-    if (tile != bid) __syncthreads();  // the previous tile has been read
-    const int64_t j0 = int64_t(tile) * BS;
-    const int64_t j = j0 + threadIdx.x;
-    const bool active = j < a.plane;
-    const int64_t jc = active ? j : a.plane - 1;
-    // 32-bit division (planes hold fewer than 2^31 nodes, tl_create)
-    const int ix = int(uint32_t(jc) / uint32_t(a.ny)), iy = int(jc) - ix * a.ny;
-    T U[3][9][NDPN];
-    T S[3][4];
-    stage_line<NDPN, T, TB, SRC>(a, lds, j0, beta);
-    // 2D padded array: rows of (nely+2), one layer -> use ez = -1 addressing
-    {
-      const T* sp = static_cast<const T*>(a.sp);
+  if (active) {
+    T uc[NDPN];
 #pragma unroll
-      for (int ox = -1; ox <= 0; ++ox)
+    for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
+    if constexpr (SRC == SRC_P) {
 #pragma unroll
-        for (int oy = -1; oy <= 0; ++oy)
-          S[1][(ox + 1) * 2 + (oy + 1)] = sp[int64_t(ix + ox + 1) * (a.nely + 2) + iy + oy + 1];
+      for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
     }
-    __syncthreads();
-    read_nbrs<NDPN, T, 1>(a, lds, U);
-    T acc[NDPN];
-    node_sum<NDPN, T, 0, 1, 2, false, FAST>(a, U, S, 0, 1, acc);
-    if (active) {
-      T uc[NDPN];
-#pragma unroll
-      for (int d = 0; d < NDPN; ++d) uc[d] = U[1][4][d];
-      if constexpr (SRC == SRC_P) {
-#pragma unroll
-        for (int d = 0; d < NDPN; ++d) static_cast<T*>(a.pout)[j * NDPN + d] = uc[d];
-      }
-      ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
-    }
+    ku_epilogue<NDPN, T, MODE, TB, TO>(a, j, uc, acc, dot);
   }
   if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
     double v[1] = {dot};
@@ -714,7 +714,7 @@ __device__ __forceinline__ void ku2t_body(const KuArgs& a, unsigned bid, T* lds)
       const int hx = x0 - 1 + h / HY, hy = y0 - 1 + h % HY;
       T v = T(0);
       if (hx >= 0 && hx < a.nx && hy >= 0 && hy < a.ny)
-        v = stage_val<NDPN, T, TB, SRC>(a, hx, hy, c, beta);
+        v = stage_val<NDPN, T, TB, SRC>(a, int64_t(hx) * a.ny + hy, hx, hy, c, beta);
       lds[t] = v;
     }
     T U[3][9][NDPN];
@@ -828,10 +828,13 @@ static int resident_slots(const void* kernel, size_t lds, int64_t& slots) {
 // and 8.7 us (tile), 448x224 3.8 and 3.2, 300x100 3.4 and 2.9, 150x50 both 2.8.
 static int default_tile2d(const Grid& g) { return g.ny >= 64 ? 32 : 0; }
 
-// Workgroups of a 2D operator call over `tiles` tiles.  Where a scalar is
+// Workgroups of a 2D operator call over `tiles` node tiles.  Where a scalar is
 // folded before or after it (dot products, the seeded residual) a workgroup
 // takes several tiles, evenly, so that the partials stay within what a
-// consumer folds itself; otherwise one each.
+// consumer folds itself; otherwise one each.  Node lines go one to a workgroup
+// always: a loop over them costs the line kernel 20 registers and three of its
+// eight waves per SIMD (product inside PCG of a 20000x20 elasticity grid 10.9
+// us, with the loop 12.3-12.9; heat conduction 7.1 and 9.1).
 template <int MODE, int SRC>
 static int64_t ku2_groups(int64_t tiles) {
   if (MODE != KU_STORE_DOT && MODE != KU_JACOBI_DOT && SRC != SRC_SEED) return tiles;
@@ -930,21 +933,19 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
       set_error("fine operator grid exceeds the reduction slot count");
       return TL_EINVAL;
     }
-    const unsigned nb = unsigned(ku2_groups<MODE, SRC>(nbx));
-    a.nblk = nb;
     if (P->rec) {
       KuArgs ar = a;
       ar.ty = 0;
       P->rec->add(P->rec_phase, P->rec_level,
-                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, FAST>, ar, nb,
+                  &ku2_multi_launch<NDPN, T, MODE, TB, TO, SRC, FAST>, ar, nbx,
                   size_t(L) * NDPN * sizeof(T));
     } else {
-      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nb), dim3(BS),
+      hipLaunchKernelGGL((ku2d_kernel<NDPN, T, MODE, TB, TO, SRC, FAST>), dim3(nbx), dim3(BS),
                          size_t(L) * NDPN * sizeof(T), P->stream, a);
     }
     if constexpr (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) {
       TL_CHECK_LAUNCH();
-      return launch_fold(const_cast<tl_problem*>(P), nb, a.fin, a.dot_out, a.done);
+      return launch_fold(const_cast<tl_problem*>(P), nbx, a.fin, a.dot_out, a.done);
     }
   }
   TL_CHECK_LAUNCH();
