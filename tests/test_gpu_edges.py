@@ -426,3 +426,38 @@ def test_node_lines(gpu, dims, ndpn, pattern):
                       preconditioner="jacobi", raise_on_fail=False)
     assert rel(got[op._free_t].cpu().numpy(), ref) < 1e-11
     op.close()
+
+
+# cycles on node lines with a matrix of no pattern: 1,045 lines, more than fold
+# r.r themselves
+@pytest.mark.parametrize("dims,ndpn,nlevels", [((832, 320, None), 1, 6)])
+def test_node_line_cycles(gpu, dims, ndpn, nlevels):
+    """PCG iterates 1 and 3 of the FP64 cycle against the oracle's (bounds of
+    test_seeded_cycle_iterates); a solve stops at the same iteration with the
+    same bits whatever the chunk length, and in a lockstep batch."""
+    import torch
+    from topoptlab_amd.batch import batch_solve
+    from topoptlab_amd.fem import StiffnessOperator
+    say("node line cycles", dims, ndpn)
+    KE, edof, ndof, fixed, free, x = _problem(dims, ndpn)
+    KE = _no_pattern(KE)
+    K = fem.apply_bc(fem.assemble_K(KE, edof, fem.simp(x), ndof), free).tocsr()
+    b = np.random.default_rng(3).standard_normal(len(free))
+    h = mg.Hierarchy(K, *dims, ndpn, fixed, nlevels)
+    op = StiffnessOperator(*dims, KE=KE, fixed=fixed, device=gpu)
+    op.set_density(x)
+    f = op.full(torch.as_tensor(b, device=gpu))
+    op.setup_mg(nlevels=nlevels, precision="fp64")
+    for k, tol in ((1, 1e-8), (3, 1e-7)):
+        ref, _, _ = mg.pcg(K, b, h.vcycle, rtol=1e-10, maxiter=k)
+        got, _ = op.solve(f, rtol=1e-10, maxiter=k, raise_on_fail=False)
+        assert rel(got[op._free_t].cpu().numpy(), ref) < tol, k
+    for prec in ("fp64", "fp32"):
+        op.setup_mg(nlevels=nlevels, precision=prec)
+        want, inf = op.solve(f, rtol=1e-6, check_every=1)
+        for every in (3, 64):
+            got, i2 = op.solve(f, rtol=1e-6, check_every=every)
+            assert i2["iterations"] == inf["iterations"] and torch.equal(got, want), (prec, every)
+        got, _ = batch_solve([op], [f], rtol=1e-6)
+        assert torch.equal(got[0], want), prec
+    op.close()

@@ -828,6 +828,18 @@ static int resident_slots(const void* kernel, size_t lds, int64_t& slots) {
 // and 8.7 us (tile), 448x224 3.8 and 3.2, 300x100 3.4 and 2.9, 150x50 both 2.8.
 static int default_tile2d(const Grid& g) { return g.ny >= 64 ? 32 : 0; }
 
+static unsigned node_lines(const Grid& g) { return unsigned((int64_t(g.nx) * g.ny + BS - 1) / BS); }
+
+// Tile height that a 2D operator call takes (0: node lines).  Dot products of
+// more lines than reduction slots are refused by the line form's check.
+static int tile2d_of(const tl_problem* P, bool f64, bool dot) {
+  if (P->ndpn > 2 || !P->op.fast_ke) return 0;
+  const int ty = P->op.tile2d[f64 ? 0 : 1];
+  if (ty >= 0) return ty;
+  return dot && node_lines(P->g) > unsigned(kMaxRedBlocks) ? 0 : default_tile2d(P->g);
+}
+bool ku2d_on_tiles(const tl_problem* P, bool f64) { return tile2d_of(P, f64, true) != 0; }
+
 // Workgroups of a 2D operator call over `tiles` node tiles.  Where a scalar is
 // folded before or after it (dot products, the seeded residual) a workgroup
 // takes several tiles, evenly, so that the partials stay within what a
@@ -875,7 +887,7 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
   a.nelx = g.nelx; a.nely = g.nely; a.nelz = g.nelz;
   a.nx = g.nx; a.ny = g.ny; a.nz = g.nz; a.plane = g.nx * g.ny;
   const int L = BS + 2 * g.ny + 2;
-  const unsigned nbx = unsigned((int64_t(a.plane) + BS - 1) / BS);
+  const unsigned nbx = node_lines(g);
   if (g.dim == 3 && P->rec) {  // no multi-instance form of the 3D operator
     P->rec->unsupported = true;
     return TL_OK;
@@ -917,12 +929,7 @@ static int launch_ku_impl(const tl_problem* P, KuArgs a) {
   } else {
     a.ncol = 0;
     if constexpr (NDPN <= 2 && FAST) {
-      int ty = P->op.tile2d[sizeof(T) == 8 ? 0 : 1];
-      if (ty < 0) {
-        ty = default_tile2d(g);
-        if ((MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT) && nbx > unsigned(kMaxRedBlocks)) ty = 0;
-      }
-      switch (ty) {
+      switch (tile2d_of(P, sizeof(T) == 8, MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT)) {
         case 16: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 16>(P, a);
         case 32: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 32>(P, a);
         case 64: return launch_ku2t<NDPN, T, MODE, TB, TO, SRC, 64>(P, a);
@@ -1420,7 +1427,8 @@ static int launch_fold(tl_problem* P, unsigned nb, int fin, double* out, const i
     // operators fill the chip: every workgroup reading the partials first cost
     // more than that launch (136 systems, 13.9M DOF: 594 ms per batch solve,
     // 537 with the launch).
-    const bool in = nb <= kFoldInBlocks && !P->rec && !(fin == FIN_RHO && P->op.mfma64);
+    const bool in = nb <= kFoldInBlocks && (fin == FIN_RHO ? P->rho_wg : P->pq_wg) <= kFoldInBlocks &&
+                    !P->rec && !(fin == FIN_RHO && P->op.mfma64);
     (fin == FIN_RHO ? P->rho_nb : P->pq_nb) = in ? nb : 0u;
     if (in) return TL_OK;
   }
@@ -1769,6 +1777,20 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
   hipStream_t s = P->stream;
   // z = M r ; rho = r.z ; beta
   const bool fx0 = pcg_fuses_x0(P, precond);
+  // Workgroups of the product (or the update before it) and of the cycle's
+  // residual, 0 where there are few: node tiles are grouped, the 3D operators
+  // fill the chip once.
+  const bool general3d = P->g.dim == 3 && !P->op.sym && !(P->op.mfma64 && P->ndpn == 3);
+  auto lines = [&](bool f64) {
+    return P->g.dim == 2 && !ku2d_on_tiles(P, f64) ? node_lines(P->g) : 0u;
+  };
+  P->rho_wg = general3d ? c.nb : lines(true);
+  // seeded cycles: the next residual folds r.r and ends the solve (a lockstep
+  // batch folds all of its systems in one launch instead)
+  const bool lazy = fx0 && mg_seeds_x0(P) && !P->rec &&
+                    lines(P->mg.prec == TL_PREC_FP64) <= kFoldInBlocks;
+  const unsigned ub = lazy ? std::min(c.rb, kFoldInBlocks) : c.rb;
+  P->pq_wg = ub;
   if (precond == TL_PRECOND_GMG) {
     TL_TRY(mg_vcycle(P, c.r, c.z, c.done, fx0));
   } else {
@@ -1794,7 +1816,7 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
     P->rec->unsupported = true;
     return TL_OK;
   }
-  if (P->g.dim == 3 && !P->op.sym && !(P->op.mfma64 && P->ndpn == 3)) {
+  if (general3d) {
     FoldIn rho;
     if (P->rho_nb) rho = {fin_partials(P, FIN_RHO), P->rho_nb, c.st};
     hipLaunchKernelGGL(pupdate_kernel, dim3(c.nb), dim3(BS), 0, s, c.z, pin, pout, &c.st->beta,
@@ -1810,10 +1832,6 @@ int pcg_iteration(tl_problem* P, const PcgCtx& c, double* x, int precond, int64_
   FoldIn pq;
   if (P->pq_nb) pq = {fin_partials(P, FIN_PQ), P->pq_nb, c.st};
   double* rrp = fin_partials(P, FIN_RR);
-  // seeded cycles: the next residual folds r.r and ends the solve (a lockstep
-  // batch folds all of its systems in one launch instead)
-  const bool lazy = fx0 && mg_seeds_x0(P) && !P->rec;
-  const unsigned ub = lazy ? std::min(c.rb, kFoldInBlocks) : c.rb;
   auto upd = [&](auto ua) -> int {
     using TS = std::remove_pointer_t<decltype(ua.xs)>;
     if (P->rec) {

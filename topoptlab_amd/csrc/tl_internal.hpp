@@ -173,9 +173,11 @@ struct PcgState {
 // A PCG scalar whose block partials the consuming kernel folds itself (every
 // workgroup in the same fixed order as fold_kernel) instead of a one-block
 // kernel in between: a launch of 2-6 us and a gap less per scalar.  Beyond
-// kFoldInBlocks partials the reads of all workgroups together cost more than
-// the launch.  partials == nullptr: the scalar is in the state.  No workgroup
-// reads a state field that one of the same kernel writes.
+// kFoldInBlocks partials, or workgroups that read them, the reads together cost
+// more than the launch (20000x20 elasticity: x/r update of 3,282 workgroups
+// 11.0 us, 14.2 with the fold of 821 partials).  partials == nullptr: the scalar
+// is in the state.  No workgroup reads a state field that one of the same
+// kernel writes, but `done` (see fold_in_done).
 constexpr unsigned kFoldInBlocks = 1024;
 struct FoldIn {
   const double* partials = nullptr;
@@ -348,6 +350,8 @@ struct tl_problem {
   tl::DevBuf partials, state;
   // rho, p.q and r.r partials left for their consumer to fold (0: in the state)
   unsigned rho_nb = 0, pq_nb = 0, rr_nb = 0;
+  // workgroups of the kernels that would fold rho and p.q (0: at most kFoldInBlocks)
+  unsigned rho_wg = 0, pq_wg = 0;
   // launch timing of the fine operator (tl_profile)
   bool prof_on = false;
   std::vector<tl::ProfEvent> prof_used, prof_free;
@@ -361,6 +365,8 @@ int fine_apply_ex(tl_problem* P, const void* u, void* y, int prec, int mode, con
                   void* pout, const double* beta, double* dot_out, int fin, const int* done,
                   bool out64);
 int fine_diag(tl_problem* P);
+// whether a 2D grid's operator of that precision runs on node tiles (else node lines)
+bool ku2d_on_tiles(const tl_problem* P, bool f64);
 // launch timing (tl_profile): no-ops while profiling is off
 int prof_begin(tl_problem* P, int kind, ProfEvent& ev);
 int prof_end(tl_problem* P, ProfEvent& ev);
