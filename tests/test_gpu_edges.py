@@ -429,8 +429,10 @@ def test_node_lines(gpu, dims, ndpn, pattern):
 
 
 # cycles on node lines with a matrix of no pattern: 1,045 lines, more than fold
-# r.r themselves
-@pytest.mark.parametrize("dims,ndpn,nlevels", [((832, 320, None), 1, 6)])
+# r.r themselves; up to 320 nodes in y the first sweep is formed inside the
+# operators, beyond it is stored
+@pytest.mark.parametrize("dims,ndpn,nlevels", [((832, 320, None), 1, 6), ((40, 316, None), 2, 3),
+                                               ((40, 324, None), 2, 3), ((40, 324, None), 1, 3)])
 def test_node_line_cycles(gpu, dims, ndpn, nlevels):
     """PCG iterates 1 and 3 of the FP64 cycle against the oracle's (bounds of
     test_seeded_cycle_iterates); a solve stops at the same iteration with the
@@ -461,3 +463,28 @@ def test_node_line_cycles(gpu, dims, ndpn, nlevels):
         got, _ = batch_solve([op], [f], rtol=1e-6)
         assert torch.equal(got[0], want), prec
     op.close()
+
+
+def test_stored_and_formed_sweeps_in_one_batch(gpu):
+    """A lockstep batch of systems whose first sweep is stored (node lines of 325
+    nodes) and formed inside (tiles, short lines): each the single solve's bits."""
+    import torch
+    from topoptlab_amd.batch import batch_solve
+    from topoptlab_amd.fem import StiffnessOperator
+    say("mixed sweeps")
+    ops, fs, want = [], [], []
+    for dims, pattern in (((40, 324, None), False), ((64, 72, None), True), ((64, 40, None), False),
+                          ((36, 324, None), False)):
+        KE, _, ndof, fixed, free, x = _problem(dims, 2)
+        op = StiffnessOperator(*dims, KE=KE if pattern else _no_pattern(KE), fixed=fixed, device=gpu)
+        op.set_density(x)
+        op.setup_mg(nlevels=3, precision="fp32")
+        ops.append(op)
+        fs.append(op.full(torch.as_tensor(np.random.default_rng(3).standard_normal(len(free)),
+                                          device=gpu)))
+        want.append(op.solve(fs[-1], rtol=1e-6)[0])
+    for graphs in (True, False):
+        got, _ = batch_solve(ops, fs, rtol=1e-6, use_graphs=graphs)
+        assert all(torch.equal(a, b) for a, b in zip(got, want)), graphs
+    for op in ops:
+        op.close()

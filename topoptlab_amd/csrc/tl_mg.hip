@@ -1795,8 +1795,9 @@ int vcycle_fine(tl_problem* P, const double* r, double* z, const int* done, bool
 
 bool mg_seeds_x0(const tl_problem* P) {
   const MgState& M = P->mg;
-  return (P->g.dim == 2 || (P->op.sym && !P->op.mfma64)) && M.nu1 == 1 && M.nu2 == 1 &&
-         (M.prec == TL_PREC_FP64 || M.prec == TL_PREC_FP32);
+  if (M.nu1 != 1 || M.nu2 != 1 || (M.prec != TL_PREC_FP64 && M.prec != TL_PREC_FP32)) return false;
+  if (P->g.dim == 2) return P->g.ny <= 320 || ku2d_on_tiles(P, M.prec == TL_PREC_FP64);
+  return P->op.sym && !P->op.mfma64;
 }
 
 int mg_vcycle(tl_problem* P, const double* r, double* z, const int* done, bool x0_ready) {
