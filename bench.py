@@ -41,16 +41,18 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
-def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4):
+def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4, seeded=True):
     """Algorithmic HBM bytes of one solve (each array touched once per kernel).
 
     Fine level per PCG iteration: p = z + beta p inside the product q = K p
     32 B/DOF + 8 B/el, x/r update 48 B/DOF; V-cycle fine level: residual from
     the first sweep formed on the fly (r, dinv -> r0), final smoothing from the
     same and the coarse correction, writing z in FP64 (r, dinv, xc -> z).
-    Level 1 is applied from the fine densities (residual and smoothing), deeper
-    levels read their stencils twice, plus the levels' vectors; coarsest dense
-    inverse once.
+    Not seeded (a matrix-core fine operator): the update writes the first sweep
+    (dinv -> x), which the residual (x, r -> r0), a prolongation-add (x) and the
+    final smoothing (x, r, dinv -> z) read.  Level 1 is applied from the fine
+    FP64 densities (residual and smoothing), deeper levels read their stencils
+    twice, plus the levels' vectors; coarsest dense inverse once.
     """
     nelx, nely, nelz = dims
     ndpn = 3
@@ -59,6 +61,9 @@ def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4):
     w = vprec_bytes
     fine_pcg = 32 * ndof + 8 * nel + 48 * ndof
     fine_v = (8 + 2 * w) * ndof + w * nel + (16 + w) * ndof + w * nel
+    if not seeded:
+        fine_pcg += 2 * w * ndof
+        fine_v += 3 * w * ndof
     coarse = 0
     d = [nelx, nely, nelz]
     for lvl in range(1, nlevels):
@@ -69,7 +74,7 @@ def solve_traffic_bytes(dims, nlevels, iters, vprec_bytes=4):
             coarse += 8 * nd * nd + 2 * w * nd
         else:
             # fine densities, or the forward half of the block stencil
-            st = nel * w if lvl == 1 else 14 * ndpn * ndpn * nn * w
+            st = 8 * nel if lvl == 1 else 14 * ndpn * ndpn * nn * w
             coarse += 2 * st + 12 * w * nd
     return iters * (fine_pcg + fine_v + coarse)
 
@@ -268,9 +273,9 @@ def kernel_kinds(dims, vcycle, nlevels, fp64_mfma=False):
         2: (f"{vk} V-cycle damped-Jacobi sweep (z in FP64, r.z)",
             sweep * ndof + corr + vb * nel + ndof // 3, flops_ku, vbound, vpeak),
         3: (f"sym_kernel {l1} level-1 residual (Galerkin operator from the fine densities)",
-            vb * nel + 3 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
+            8 * nel + 3 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
         4: (f"sym_kernel {l1} level-1 damped-Jacobi sweep with the level-2 correction",
-            vb * nel + 4 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
+            8 * nel + 4 * vb * nd1 + nn1, 2.0 * 243 * nn1, "hbm", HBM_PEAK_GBS),
     }
 
 
@@ -706,7 +711,8 @@ def main():
     dom = max(prof, key=lambda k: prof[k][0])
     avg_ms = prof[dom][0] / max(prof[dom][1], 1)
     vb = 8 if args.vcycle == "fp64" else 4
-    traffic = solve_traffic_bytes(dims, args.levels, iters, vb)
+    traffic = solve_traffic_bytes(dims, args.levels, iters, vb,
+                                  args.vcycle in ("fp64", "fp32") and args.fp64_operator != "mfma")
     solve_tbps = traffic / (ms * 1e-3) / 1e12
     hbm = None
     tfile = ROOT / "profiles" / "traffic.json"

@@ -41,3 +41,15 @@ def test_cpu_full_mode_small_grid():
     b = f[free, 0]
     c = float(b @ spsolve(K, b))
     assert abs(out["compliance"] - c) / abs(c) < 1e-7
+
+
+def test_traffic_of_stored_and_formed_sweeps():
+    """The cycles of a matrix-core fine operator store their first sweep: the
+    update writes x (dinv, x), the residual reads x for dinv, the prolongation
+    reads and writes x, the last sweep reads x besides (5 vectors more)."""
+    import bench
+    dims, ndof = (16, 8, 8), 3 * 17 * 9 * 9
+    for w in (4, 8):
+        a = bench.solve_traffic_bytes(dims, 3, 10, w, True)
+        b = bench.solve_traffic_bytes(dims, 3, 10, w, False)
+        assert b - a == 10 * 5 * w * ndof
