@@ -192,7 +192,7 @@ int tl_oc_update(int64_t n, const double* x, const double* dc,
  * arguments, kernels and results as tl_oc_update; the reduction partials and
  * the bisection state live in a statically allocated device array of
  * 41,216 bytes per device (held until the process ends), whose size does not
- * depend on n (the grid is capped at 1024 blocks), so no n is too large for
+ * depend on n (the grid is capped at 256 blocks), so no n is too large for
  * it.  Its address is looked up once per device on the first call.  Every
  * call on a device shares that device's array: calls that overlap on one
  * device (several host threads or streams) race and must be serialised by

@@ -843,7 +843,9 @@ bool ku2d_on_tiles(const tl_problem* P, bool f64) { return tile2d_of(P, f64, tru
 // Workgroups of a 2D operator call over `tiles` node tiles.  Where a scalar is
 // folded before or after it (dot products, the seeded residual) a workgroup
 // takes several tiles, evenly, so that the partials stay within what a
-// consumer folds itself; otherwise one each.  Node lines go one to a workgroup
+// consumer folds itself; otherwise one each.  (A lockstep batch folds nothing
+// there and is faster with the groups all the same: 136 systems of 40 grids 530
+// ms, one tile each 547.)  Node lines go one to a workgroup
 // always: a loop over them costs the line kernel 20 registers and three of its
 // eight waves per SIMD (product inside PCG of a 20000x20 elasticity grid 10.9
 // us, with the loop 12.3-12.9; heat conduction 7.1 and 9.1).
@@ -858,6 +860,8 @@ template <int NDPN, typename T, int MODE, typename TB, typename TO, int SRC, int
 static int launch_ku2t(const tl_problem* P, KuArgs a) {
   constexpr int TX = BS / TY;
   const int64_t tiles = int64_t((a.nx + TX - 1) / TX) * ((a.ny + TY - 1) / TY);
+  // (The groups would fit: the limit is on tiles so that a set shape serves the
+  // sizes that it served with a workgroup per tile.)
   if (tiles > kMaxRedBlocks && P->op.tile2d[sizeof(T) == 8 ? 0 : 1] == TY &&
       (MODE == KU_STORE_DOT || MODE == KU_JACOBI_DOT)) {
     set_error("fine operator grid exceeds the reduction slot count");
@@ -1113,6 +1117,11 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
         return launch_fold(P, nb, a.fin, a.dot_out, a.done);
       return TL_OK;
     }
+    // Tiles wherever the matrix has their pattern, also where a grid ends just
+    // past one: of 24 grids from 8^3 to 144^3, 16 and 17 nodes per side and 3 to
+    // 1025 long among them, none is slower than with the general form (48 FP64
+    // cycles of 16^3 elasticity 3.62 -> 2.15 ms, 16x16x1024 8.43 -> 7.52; heat
+    // conduction 2.18 -> 1.60 and 4.69 -> 4.17).
     if (P->op.sym && (mode == KU_STORE || mode == KU_STORE_DOT || b64)) return sym();
     a.sp = P->op.sp64.ptr; a.KE = P->op.KE64.ptr;
     switch (P->ndpn) {
@@ -1121,8 +1130,8 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
       case 3: return dispatch_mode<3, double>(P, a, mode, fusep, b64, out64);
     }
   } else {
-    // the V-cycle's FP32 modes; FP32 products (tl_apply_K) keep the general form
-    // and its order of sums, which is what their callers compare runs by
+    // the V-cycle's FP32 modes; FP32 products (tl_apply_K alone, no part of a
+    // solve) run on the general form, the tiles have no FP32 product
     if (P->op.sym && b64) return sym();
     a.sp = P->op.sp32.ptr; a.KE = P->op.KE32.ptr;
     switch (P->ndpn) {
