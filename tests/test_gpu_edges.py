@@ -488,3 +488,30 @@ def test_stored_and_formed_sweeps_in_one_batch(gpu):
         assert all(torch.equal(a, b) for a, b in zip(got, want)), graphs
     for op in ops:
         op.close()
+
+
+@pytest.mark.parametrize("decades,bound", [(0, 1.8e-16), (9, 2.5e-16)])
+def test_tiled_product_error(gpu, decades, bound):
+    """FP64 K u on white noise against the caller's matrix in extended precision.
+    The product's group values are the means of its entries: 1.4e-16 and 2.1e-16
+    in a host model of the kernel's sums, 2.2e-16 and 2.9e-16 with single ones."""
+    import torch
+    from topoptlab_amd.fem import StiffnessOperator
+    say("tiled product error", decades)
+    dims = (31, 22, 17)
+    KE, edof, ndof, _, _, _ = _problem(dims, 3)
+    rng = np.random.default_rng(5)
+    x = 10.0 ** (-decades / 3.0 * rng.random(edof.shape[0]))
+    u = rng.standard_normal(ndof)
+    op = StiffnessOperator(*dims, KE=KE, fixed=[], device=gpu)
+    op.set_density(x)
+    got = op.matvec_full(torch.as_tensor(u, device=gpu)).cpu().numpy()
+    ld = np.longdouble
+    s = ld(1e-9) + (ld(1) - ld(1e-9)) * x.astype(ld) ** 3
+    f = s[:, None] * np.stack([(u[edof].astype(ld) * k).sum(axis=1) for k in KE.astype(ld)], axis=1)
+    ref = np.zeros(ndof, dtype=ld)
+    np.add.at(ref, edof.ravel(), f.ravel())
+    err = float(np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()))
+    print(f"  {err:.2e}", flush=True)
+    assert err < bound
+    op.close()

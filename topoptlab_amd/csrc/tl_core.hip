@@ -137,6 +137,7 @@ struct KuArgs {
   const int* done;
   int nelx, nely, nelz, nx, ny, nz, plane, ncol;  // ncol: 3D tile columns
   int ty;  // 2D workgroup shape the launch uses (0: node line), for the multi-instance form
+  bool caller;  // a product for the caller (KU_APPLY)
   unsigned nblk;  // 2D node tiles: workgroups (each takes tiles bid, bid + nblk, ...)
   // group values of a pattern-matched element matrix (see ke_pattern.hpp)
   double kv64[8];
@@ -1023,6 +1024,8 @@ int fine_apply_ex(tl_problem* P, const void* u, void* y, int prec, int mode, con
                   void* pout, const double* beta, double* dot_out, int fin, const int* done,
                   bool out64) {
   KuArgs a{};
+  a.caller = mode == KU_APPLY;
+  if (a.caller) mode = KU_STORE;
   a.u = u; a.y = y; a.b = b; a.dinv = dinv; a.omega = omega;
   a.pin = zfuse_pin; a.pout = pout; a.beta = beta;
   a.mask = P->op.mask.as<uint8_t>();
@@ -1089,7 +1092,7 @@ static int fine_apply_dispatch(tl_problem* P, KuArgs& a, int prec, int mode, boo
       return TL_OK;
     }
     unsigned nb = 0;
-    TL_TRY(sym_fine_apply(P, a.u, a.y, prec, mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
+    TL_TRY(sym_fine_apply(P, a.u, a.y, prec, a.caller ? KU_APPLY : mode, a.b, b64, a.dinv, a.omega, a.pin, a.pout, a.beta,
                           a.rho, a.rr, a.partials, a.done, &nb));
     if (mode == KU_STORE_DOT || mode == KU_JACOBI_DOT)
       return launch_fold(P, nb, a.fin, a.dot_out, a.done);
@@ -1547,7 +1550,7 @@ int tl_create(const tl_grid_desc* d, tl_problem** out) {
       ks[i] = p > 0 ? P->op.kv[p - 1] : -P->op.kv[-p - 1];
     }
   P->op.sym = sym_fits(P->g, P->ndpn) && ku3d_serves(P->g, P->ndpn) &&
-              sym_detect(P->ndpn, ks.data(), P->op.symkv, P->op.symkt);
+              sym_detect(P->ndpn, ks.data(), P->KEh.data(), P->op.symkv, P->op.symkvp, P->op.symkt);
   P->op.mfma64 = false;  // the vector kernel is faster (tl_set_fp64_operator selects)
   std::vector<float> ke32(nd * nd);
   for (int i = 0; i < nd * nd; ++i) ke32[i] = float(P->KEh[i]);
@@ -1622,7 +1625,7 @@ int tl_apply_K(tl_problem* P, const double* u, double* y, int32_t prec) {
                      P->op.mask.as<uint8_t>(), P->ndpn, P->ndof);
   TL_CHECK_LAUNCH();
   if (prec == TL_PREC_FP64)
-    return fine_apply_ex(P, P->t.ptr, y, TL_PREC_FP64, KU_STORE, nullptr, false, nullptr, 0.0,
+    return fine_apply_ex(P, P->t.ptr, y, TL_PREC_FP64, KU_APPLY, nullptr, false, nullptr, 0.0,
                          nullptr, nullptr, nullptr, nullptr, FIN_STORE, nullptr, true);
   // fp32: cast input, apply, widen output
   TL_TRY(P->z.alloc(sizeof(double) * P->ndof));

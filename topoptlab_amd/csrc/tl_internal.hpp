@@ -268,6 +268,7 @@ struct FineOp {
   double kv[8] = {};           // group values of the pattern
   bool sym = false;            // 3D: the tiled reflection-symmetric operator applies (tl_sym.hip)
   double symkv[16] = {};       // its group values
+  double symkvp[16] = {};      // and those of a product for the caller (mean_values)
   double symkt = 0.0;          // and its stiffness against a translation
   // 2D operator workgroup shape per precision [fp64, fp32]: 0 = node line
   // (BS consecutive nodes), TY = 16/32/64: (BS/TY) x TY node tile; -1: by rule
@@ -392,7 +393,8 @@ int fine_apply_mfma64(tl_problem* P, const double* u, double* y, int mode, const
                       const double* beta, double* partials, const int* done,
                       unsigned* nblocks_out);
 // tiled 3D operators in the reflection-symmetric form (tl_sym.hip)
-bool sym_detect(int ndpn, const double* KE, double (&kv)[16], double& kt);
+bool sym_detect(int ndpn, const double* KE, const double* given, double (&kv)[16],
+                double (&kv_product)[16], double& kt);
 bool sym_detect_coarse(int ndpn, const double* G, double (&kv)[16]);
 bool sym_fits(const Grid& g, int ndpn);
 int sym_fine_apply(tl_problem* P, const void* u, void* y, int prec, int mode, const void* b,
@@ -429,4 +431,5 @@ enum {
   KU_RESID = 2,       // y = b - K u
   KU_JACOBI = 3,      // y = u + omega*dinv*(b - K u)
   KU_JACOBI_DOT = 4,  // as KU_JACOBI, y written fp64, dot += b.y
+  KU_APPLY = 5,       // KU_STORE for the caller (tl_apply_K): see mean_values in tl_sym.hip
 };
